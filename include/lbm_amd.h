@@ -71,7 +71,7 @@ typedef enum lbm_storage {
 typedef enum lbm_step_flags {
     LBM_STEP_MACRO = 1u,    /* the last step of the call also stores rho/u (reference global_rho/global_u) */
     LBM_STEP_CHECK = 2u,    /* synchronise after the call and report LBM_ERR_NAN (or LBM_ERR_RANGE) */
-    LBM_STEP_NO_GRAPH = 4u  /* launch every step eagerly instead of replaying a captured HIP graph */
+    LBM_STEP_NO_GRAPH = 4u  /* launch every step by itself, eagerly, instead of replaying a captured HIP graph */
 } lbm_step_flags;
 
 typedef struct lbm_desc {
@@ -300,8 +300,10 @@ int lbm_get_scale(lbm_ctx *ctx, double *scale);
  * idles on a solid node, or LBM_LAUNCH_RUN_TABLE: the same runs with every
  * lane's neighbour addressing read from a table built on first use (4 bytes
  * per wet node and step more traffic, far fewer instructions per wave).
- * Results are the same bits for every shape.  No counterpart in the
- * reference (a tuning knob of this engine). */
+ * Results are the same bits for every shape.  With 0 (the default), steps
+ * without new prescribed values may run several to a launch (FP64 and FP32
+ * storage, blocked layout); a shape set here is a launch of one step.  No
+ * counterpart in the reference (a tuning knob of this engine). */
 enum { LBM_LAUNCH_WET_RUNS = 64, LBM_LAUNCH_RUN_TABLE = 65 };
 int lbm_set_launch(lbm_ctx *ctx, int32_t segments);
 int lbm_get_launch(lbm_ctx *ctx, int32_t *segments);
@@ -317,11 +319,12 @@ int lbm_set_occupancy(lbm_ctx *ctx, int32_t groups_per_cu);
 int lbm_get_occupancy(lbm_ctx *ctx, int32_t *groups_per_cu);
 
 /* Times each launch shape (1, 2, 4, 8 segments, wet runs, tabled wet runs)
- * at each occupancy (no limit, 7 down to 3 work-groups per compute unit)
- * over `steps` launches (every launch rewrites the spare buffer from the
+ * at each occupancy (no limit, 7 down to 3 work-groups per compute unit),
+ * and launches of several steps where the lattice takes them, over `steps` launches (every launch rewrites the spare buffer from the
  * current state, so the state does not change) and keeps the fastest
- * pair.  Reports the shape and its time per step (outputs may be NULL);
- * lbm_get_occupancy reports the occupancy.  LBM_ERR_STATE for a context
+ * pair for single steps, and several steps per launch if they are faster
+ * still.  Reports the shape of the single steps and the time per step
+ * (outputs may be NULL); lbm_get_occupancy reports the occupancy.  LBM_ERR_STATE for a context
  * that belongs to an ensemble (the ensemble has its own,
  * lbm_batch_autotune) and for a lattice with partially saturated
  * bounce-back (every launch advances its carried obstacle values).  No

@@ -86,6 +86,9 @@ StepArgs make_args(const lbm_ctx *c)
     a.nruns = c->nruns;
     a.perim = c->d_perim;
     a.nperim = c->nperim;
+    a.wet_top = c->wet_top;
+    a.wet_bottom = c->wet_bottom;
+    a.cus = c->cus;
     a.trun = c->d_trun;
     a.tlane = c->d_tlane;
     a.psbb = c->psbb ? 1 : 0;
@@ -100,9 +103,19 @@ StepArgs make_args(const lbm_ctx *c)
 
 namespace {
 
-// Steps per captured graph: even, so a replay leaves the buffer holding
-// the state unchanged.
-constexpr int64_t kGraphSteps = 32;
+// Launches per captured graph: an even number, so a replay leaves the
+// buffer holding the state unchanged.
+constexpr int64_t kGraphLaunches = 8, kGraphSteps = 32;
+
+// Steps per launch of a steady run (1: the step kernels).
+int32_t steps_per_launch(const lbm_ctx *c)
+{
+    const int32_t k = c->march ? march_steps(c->storage, make_args(c)) : 0;
+    return std::max(k, 1);
+}
+
+// Steps per captured graph.
+int64_t graph_steps(int32_t per_launch) { return per_launch > 1 ? kGraphLaunches * per_launch : kGraphSteps; }
 
 void drop_graphs(lbm_ctx *c)
 {
@@ -113,21 +126,25 @@ void drop_graphs(lbm_ctx *c)
         }
 }
 
-// Captures kGraphSteps gathering steps from the context's current buffer
-// and prescribed values (both steps of a run after its first).
-int capture_steps(lbm_ctx *c)
+// Launch of k steady steps (k = 1: the step kernels) from buffer `in`.
+hipError_t launch_steady(const lbm_ctx *c, int in, int32_t k)
+{
+    StepArgs a = make_args(c);
+    a.fin = c->d_F[in];
+    a.fout = c->d_F[1 - in];
+    a.macro = nullptr;
+    return k > 1 ? launch_march(c->storage, k, a, c->stream) : launch_step(c->storage, true, a, c->stream, c->segments);
+}
+
+// Captures a graph's steady steps, per_launch each, from the context's
+// current buffer and prescribed values.
+int capture_steps(lbm_ctx *c, int32_t per_launch)
 {
     hipGraph_t g = nullptr;
     HIP_TRY(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
     hipError_t err = hipSuccess;
-    for (int64_t k = 0; k < kGraphSteps && err == hipSuccess; ++k) {
-        StepArgs a = make_args(c);
-        const int in = c->cur ^ (int)(k & 1);
-        a.fin = c->d_F[in];
-        a.fout = c->d_F[1 - in];
-        a.macro = nullptr;
-        err = launch_step(c->storage, true, a, c->stream, c->segments);
-    }
+    const int64_t launches = graph_steps(per_launch) / per_launch;
+    for (int64_t k = 0; k < launches && err == hipSuccess; ++k) err = launch_steady(c, c->cur ^ (int)(k & 1), per_launch);
     hipError_t e2 = hipStreamEndCapture(c->stream, &g);
     if (err != hipSuccess) return fail(LBM_ERR_HIP, "step graph capture: %s", hipGetErrorString(err));
     if (e2 != hipSuccess) return fail(LBM_ERR_HIP, "hipStreamEndCapture: %s", hipGetErrorString(e2));
@@ -499,6 +516,9 @@ int lbm_create(const lbm_desc *desc, lbm_ctx **out)
     lbm_ctx *c = new lbm_ctx();
     c->desc = *desc;
     c->storage = desc->storage;
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, desc->device) == hipSuccess && cus > 0)
+        c->cus = cus;
     c->esize = desc->storage == kF64 ? 8 : desc->storage == kF32 ? 4 : 2;
     hipError_t e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
     if (e != hipSuccess) {
@@ -668,6 +688,7 @@ int lbm_set_geometry(lbm_ctx *c, const uint8_t *cls)
     std::vector<uint8_t> edge((size_t)c->E, kEdgePlain);
     for (int k = 0; k < 7; ++k) c->counts[k] = 0;
     c->n_wet = 0;
+    c->wet_top = c->wet_bottom = false;
     for (int w = 0; w < 2; ++w) { c->open_ij[w].clear(); c->open_e[w].clear(); }
     c->obst_ij.clear();
     c->obst_mask.clear();
@@ -678,6 +699,8 @@ int lbm_set_geometry(lbm_ctx *c, const uint8_t *cls)
             if (wet_cls(k)) {
                 wet[(size_t)((j + 1) * c->wl + 1 + i / 64)] |= 1ull << (i % 64);
                 c->n_wet++;
+                c->wet_top |= i == 0;
+                c->wet_bottom |= i == nr - 1;
             }
             if (k == LBM_INLET || k == LBM_OUTLET) edge[(size_t)edge_slot_host(i, j, nr, nc)] = k == LBM_INLET ? kEdgeInlet : kEdgeOutlet;
         }
@@ -715,6 +738,7 @@ int lbm_set_geometry(lbm_ctx *c, const uint8_t *cls)
                 prev = (m >> 63) & 1;
             }
             if (stretches == 1 && count >= kAlignRows) acc += ((r0 - acc) % 64 + 64) % 64;
+            sb[w0 - 1] = (int32_t)acc;  // the guard word above: the column's first index
             for (int64_t k = 0; k < nrw; ++k) {
                 sb[w0 + k] = (int32_t)acc;
                 acc += __builtin_popcountll(wet[w0 + k]);
@@ -1000,20 +1024,34 @@ int lbm_step(lbm_ctx *c, int64_t n, uint32_t flags)
     if (c->state == kNone) return fail(LBM_ERR_STATE, "no populations (call lbm_init_equilibrium)");
     HIP_TRY(hipSetDevice(c->desc.device));
     const bool macro = (flags & LBM_STEP_MACRO) != 0;
+    const int32_t per_launch = steps_per_launch(c);
     for (int64_t s = 0; s < n;) {
         // After the first step of a run (collide-only pass, new prescribed
-        // values) every step is the same launch on alternating buffers:
-        // replay a captured loop of kGraphSteps of them.
+        // values) every launch takes the same steps on alternating buffers:
+        // replay a captured loop of them, then launch the rest, as many
+        // steps at a time as are left.
         const bool steady = c->state == kFstar && c->bc_prev == c->bc_cur;
-        if (!(flags & LBM_STEP_NO_GRAPH) && steady && n - s - (macro ? 1 : 0) >= kGraphSteps) {
-            if (!c->graph[c->cur][c->bc_cur]) {
-                int r = capture_steps(c);
-                if (r) return r;
+        const int64_t left = n - s - (macro ? 1 : 0);
+        if (!(flags & LBM_STEP_NO_GRAPH) && steady && left >= std::min<int64_t>(per_launch, 2)) {
+            if (left >= graph_steps(per_launch)) {
+                if (!c->graph[c->cur][c->bc_cur]) {
+                    int r = capture_steps(c, per_launch);
+                    if (r) return r;
+                }
+                HIP_TRY(hipGraphLaunch(c->graph[c->cur][c->bc_cur], c->stream));
+                c->t += graph_steps(per_launch);
+                s += graph_steps(per_launch);
+                continue;
             }
-            HIP_TRY(hipGraphLaunch(c->graph[c->cur][c->bc_cur], c->stream));
-            c->t += kGraphSteps;
-            s += kGraphSteps;
-            continue;
+            if (per_launch > 1) {
+                // no single step is left over where two launches can share the rest
+                const int32_t k = (int32_t)(left == per_launch + 1 ? left - 2 : std::min<int64_t>(left, per_launch));
+                HIP_TRY(launch_steady(c, c->cur, k));
+                c->cur = 1 - c->cur;
+                c->t += k;
+                s += k;
+                continue;
+            }
         }
         StepArgs a = make_args(c);
         a.fin = c->d_F[c->cur];
@@ -1060,6 +1098,7 @@ int lbm_set_launch(lbm_ctx *c, int32_t segments)
         if (r) return r;
     }
     c->segments = segments;
+    c->march = segments == 0;
     drop_graphs(c);
     return LBM_OK;
 }
@@ -1145,11 +1184,28 @@ int lbm_autotune(lbm_ctx *c, int32_t steps, int32_t *segments, double *ms_per_st
             }
         }
     }
+    // several steps per launch against the best single step
+    bool march = false;
+    const int32_t k = march_steps(c->storage, a);
+    if (k > 1) {
+        if (err == hipSuccess) err = launch_march(c->storage, k, a, c->stream);
+        if (err == hipSuccess) err = hipEventRecord(t0, c->stream);
+        for (int32_t s = 0; s < steps && err == hipSuccess; ++s) err = launch_march(c->storage, k, a, c->stream);
+        if (err == hipSuccess) err = hipEventRecord(t1, c->stream);
+        if (err == hipSuccess) err = hipEventSynchronize(t1);
+        float ms = 0.f;
+        if (err == hipSuccess) err = hipEventElapsedTime(&ms, t0, t1);
+        if (err == hipSuccess && ms / (float)k < best) {
+            best = ms / (float)k;
+            march = true;
+        }
+    }
     (void)hipEventDestroy(t0);
     if (t1) (void)hipEventDestroy(t1);
     if (err != hipSuccess) return fail(LBM_ERR_HIP, "autotune: %s", hipGetErrorString(err));
     c->segments = best_R;
     c->occupancy = best_occ;
+    c->march = march;
     drop_graphs(c);
     if (segments) *segments = best_R;
     if (ms_per_step) *ms_per_step = best / steps;

@@ -53,6 +53,7 @@ struct lbm_ctx {
     uint32_t *d_tlane = nullptr;
     int32_t *d_perim = nullptr;  // perimeter items (column, segment) of the perimeter kernel
     int64_t nperim = 0;
+    bool wet_top = false, wet_bottom = false;  // row 0 / row NR-1 holds a wet node
     uint8_t *d_edge_kind = nullptr;
     void *d_frozen = nullptr;
     void *d_F[2] = {nullptr, nullptr};
@@ -111,6 +112,10 @@ struct lbm_ctx {
     struct lbm_batch *batch = nullptr;
     // 64-row segments per wave of the step kernel (0 = default_segments)
     int32_t segments = 0;
+    // several steps per launch where nothing asks for single ones: off while
+    // a shape is set by hand, or where the autotuner measured it slower
+    bool march = true;
+    int32_t cus = 256;  // compute units of the device
     // partially saturated bounce-back of the wet obstacles (lbm_set_partial_bounce_back)
     bool psbb = false;
     double ps_tau = 0.0;

@@ -72,6 +72,8 @@ struct StepArgs {
     int32_t esize;          // bytes per stored population
     int32_t wpc;            // step kernel: waves per column
     int64_t nblocks;
+    int32_t wet_top, wet_bottom;  // row 0 / row NR-1 holds a wet node
+    int32_t cus;            // host side: compute units of the device
     double bgk_t, bgk_omt;              // 1/tau, 1 - 1/tau
     double trt_inv_te, trt_a, trt_b;    // 1/tau+, 0.5/tau+, 0.5/tau-
     float sh_a, sh_b;                   // shifted paths: 0.5/tau+, 0.5/tau- (BGK: both 0.5/tau)
@@ -132,6 +134,18 @@ constexpr uint32_t occupancy_lds(int32_t groups_per_cu)
     return groups_per_cu >= 2 && groups_per_cu <= 7 ? 163840u / (uint32_t)(groups_per_cu + 1) + 64u : 0u;
 }
 
+// How a launch of the marching kernel deals its waves (march_kernel).
+struct MarchPlan {
+    int32_t stripes;         // stripes of rows
+    int32_t top, bottom;     // of these, the first / last ones, whose windows hold wet nodes of row 0 / NR-1
+    int32_t cols;            // columns per wave
+    int32_t edge_cols;       // columns per wave of the edge stripes
+    int32_t edge_chunks;     // waves per edge stripe
+    int32_t edge_row_waves;  // waves of the edge stripes
+    int32_t edge_waves;      // and with the first and last columns of the others, rounded up to whole work-groups
+    int32_t xcd_chunk;       // work-groups per XCD chunk (xcd_remap)
+};
+
 // A batch step: per sample two complete argument sets, args[2 s + p] for
 // buffer parity p (p = 0: input in the sample's current buffer).
 struct BatchArgs {
@@ -185,6 +199,11 @@ hipError_t launch_lift_drag(int32_t storage, const StepArgs &a, const void *fsta
                             int64_t *nblocks_out, hipStream_t s);
 hipError_t launch_reduce_partials(const double *partials, int64_t nblocks, int32_t ncomp, double *out,
                                   hipStream_t s);
+// Steps per launch of the marching kernel for this lattice (0: not for it),
+// and such a launch: `steps` steps (2 .. march_steps) without new prescribed
+// values from fin (F*) to fout, blocked layout.
+int32_t march_steps(int32_t storage, const StepArgs &a);
+hipError_t launch_march(int32_t storage, int32_t steps, const StepArgs &a, hipStream_t s);
 int64_t readout_blocks(const StepArgs &a);
 // rho = 1, u = 0 over a field of n nodes ([3][n] doubles).
 hipError_t launch_fill_macro(double *macro, int64_t n, hipStream_t s);

@@ -30,6 +30,9 @@
 // g = f - w (FP32) or (f - w) * scale (FP16) and compute in FP32.
 #include "lbm_internal.h"
 
+#include <algorithm>
+#include <type_traits>
+
 namespace lbm {
 
 namespace {
@@ -634,27 +637,44 @@ __device__ __forceinline__ int load_p64(const StepArgs &a, int i, int j, const I
     return policy;
 }
 
+// The velocity prescribed at a velocity or no-op node at this step (unused
+// elsewhere).
+struct Prescribed {
+    double ux, uy;
+};
+
+__device__ __forceinline__ Prescribed prescribed(const StepArgs &a, int policy, int64_t e)
+{
+    if (policy == kVelocity || policy == kNoop) return {a.bc_cur[e], a.bc_cur[a.g.E + e]};
+    return {0.0, 0.0};
+}
+
 // Moments, equilibrium, collision and store of one wet node in FP64, in
 // the reference's expression order (update_macro, calc_equilibrium,
 // collide: Lattice.hpp:351-382).  Fluid and pressure nodes take their
 // moments; velocity-prescribed and no-op nodes keep rho = 1
 // (Lattice.hpp:295; the Zou-He density write is lost on a by-value copy,
-// ZouHePolicy.hpp:58,71) and the prescribed u.
-__device__ __forceinline__ void collide_f64(const StepArgs &a, const double *p, int policy, int64_t e, int i, int j,
+// ZouHePolicy.hpp:58,71) and the prescribed u.  Returns whether the node's
+// density is a NaN; REPORT: sets the device flag for it and writes the
+// macro fields.
+template <bool REPORT = true>
+__device__ __forceinline__ bool collide_f64(const StepArgs &a, const double *p, int policy, Prescribed v, int i, int j,
                                             double *o, double *eq_out = nullptr)
 {
     double rho, ux, uy;
+    bool nan;
     if (policy == kVelocity || policy == kNoop) {
         rho = 1.0;
-        ux = a.bc_cur[e];
-        uy = a.bc_cur[a.g.E + e];
+        ux = v.ux;
+        uy = v.uy;
         double s = p[0] + p[1] + p[2] + p[3] + p[4] + p[5] + p[6] + p[7] + p[8];
-        if (s != s) atomicOr(a.flag, 1);
+        nan = s != s;
     } else {
         moments64(p, rho, ux, uy);
-        if (rho != rho) atomicOr(a.flag, 1);
+        nan = rho != rho;
     }
-    if (a.macro) {
+    if (REPORT && nan) atomicOr(a.flag, 1);
+    if (REPORT && a.macro) {
         int64_t q = (int64_t)j * a.g.nr + i, N = (int64_t)a.g.nr * a.g.nc;
         LBM_GLOBAL double *mq = (LBM_GLOBAL double *)a.macro + q;
         mq[0] = rho;
@@ -681,13 +701,14 @@ __device__ __forceinline__ void collide_f64(const StepArgs &a, const double *p, 
             o[d] = p[d] - ca * (p[d] + p[q] - eq[d] - eq[q]) - cb * (p[d] - p[q] - eq[d] + eq[q]);
         }
     }
+    return nan;
 }
 
 __device__ __forceinline__ void collide_store_f64(const StepArgs &a, const double *p, int policy, int64_t e, int i,
                                                   int j, int64_t n)
 {
     double o[9];
-    collide_f64(a, p, policy, e, i, j, o);
+    collide_f64(a, p, policy, prescribed(a, policy, e), i, j, o);
     store9(a, n, o);
 }
 
@@ -704,7 +725,7 @@ __device__ __forceinline__ void node_general_f64(const StepArgs &a, int i, int j
     int policy = load_p64<GATHER>(a, i, j, x, m, edge, e, p);
     if (a.psbb) {
         double o[9], eq[9];
-        collide_f64(a, p, policy, e, i, j, o, eq);
+        collide_f64(a, p, policy, prescribed(a, policy, e), i, j, o, eq);
         psbb_update(a, x.src[0], p, eq, o);
         store9(a, x.src[0], o);
         return;
@@ -884,9 +905,9 @@ __device__ __forceinline__ void moments_shifted(const float *g, Moments &m)
 // (scaled form: 1 / (S rho) = 1 / (S + S drho)).
 // TRT on pairs of n = geq - g:  o_d = g_d + ca (n_d + n_q) + cb (n_d - n_q)
 // (BGK: ca = cb = omega / 2).
-template <bool F16>
-__device__ __forceinline__ void collide_shifted(const StepArgs &a, const float *g, int policy, int64_t e, int i, int j,
-                                                float *o)
+template <bool F16, bool REPORT = true>
+__device__ __forceinline__ bool collide_shifted(const StepArgs &a, const float *g, int policy, Prescribed v, int i,
+                                                int j, float *o)
 {
     float ps[4], pa[4];  // pair sums / differences, pairs (1,3) (2,4) (5,7) (6,8)
     float drho, jx, jy;
@@ -924,11 +945,12 @@ __device__ __forceinline__ void collide_shifted(const StepArgs &a, const float *
         jx = (float)mx;
         jy = (float)my;
     }
-    if (md != md) atomicOr(a.flag, 1);
+    const bool nan = md != md;
+    if (REPORT && nan) atomicOr(a.flag, 1);
     double rho_out, ux_out, uy_out;
     if (policy == kVelocity || policy == kNoop) {
         // rho = 1 and the prescribed velocity (see collide_store_f64)
-        const float ux = (float)a.bc_cur[e], uy = (float)a.bc_cur[a.g.E + e];
+        const float ux = (float)v.ux, uy = (float)v.uy;
         drho = 0.f;
         jx = F16 ? ux * a.scale : ux;
         jy = F16 ? uy * a.scale : uy;
@@ -940,7 +962,7 @@ __device__ __forceinline__ void collide_shifted(const StepArgs &a, const float *
         ux_out = mx / rho_out;
         uy_out = my / rho_out;
     }
-    if (a.macro) {
+    if (REPORT && a.macro) {
         int64_t q = (int64_t)j * a.g.nr + i, N = (int64_t)a.g.nr * a.g.nc;
         LBM_GLOBAL double *mq = (LBM_GLOBAL double *)a.macro + q;
         mq[0] = rho_out;
@@ -970,6 +992,7 @@ __device__ __forceinline__ void collide_shifted(const StepArgs &a, const float *
     }
     const float geq0 = drho - seq_sum;
     o[0] = __builtin_fmaf(2.f * ca, geq0 - g[0], g[0]);
+    return nan;
 }
 
 // Converts the post-collision shifted populations to the storage type and
@@ -1032,7 +1055,7 @@ __device__ __forceinline__ void collide_store_shifted(const StepArgs &a, const f
                                                       int j, int64_t n)
 {
     float o[9];
-    collide_shifted<sizeof(T) == 2>(a, g, policy, e, i, j, o);
+    collide_shifted<sizeof(T) == 2>(a, g, policy, prescribed(a, policy, e), i, j, o);
     encode_store<T>(a, n, o, false);
 }
 
@@ -1169,7 +1192,7 @@ __device__ __forceinline__ void step_wave(const StepArgs &a, int j, int64_t row0
         for (int r = 0; r < R; ++r) {
             if (!act[r]) continue;
             const int i = (int)row0 + 64 * r + lane;
-            collide_shifted<false>(a, raw[r], -1, 0, i, j, out[r]);
+            collide_shifted<false>(a, raw[r], -1, {}, i, j, out[r]);
         }
         uint32_t b0 = slot_bytes<T>(a, (uint32_t)own[0]), b1 = slot_bytes<T>(a, (uint32_t)own[1]);
         if ((lines & 3u) == 3u) {
@@ -1198,12 +1221,12 @@ __device__ __forceinline__ void step_wave(const StepArgs &a, int j, int64_t row0
             for (int d = 0; d < 9; ++d) p[d] = (V)raw[r][d];  // FP16: scaled, see collide_shifted
             if constexpr (sizeof(T) == 8) {
                 double out[9];
-                collide_f64(a, p, -1, 0, i, j, out);
+                collide_f64(a, p, -1, {}, i, j, out);
                 if ((lines >> r) & 1) store9_stream(a, own[r], out);
                 else store9(a, own[r], out);
             } else {
                 float out[9];
-                collide_shifted<sizeof(T) == 2>(a, p, -1, 0, i, j, out);
+                collide_shifted<sizeof(T) == 2>(a, p, -1, {}, i, j, out);
                 encode_store<T>(a, own[r], out, (lines >> r) & 1);
             }
         }
@@ -1334,12 +1357,12 @@ __device__ __forceinline__ void run_finish(const StepArgs &a, int i, int j, int 
     const bool lines = n == 64 && (s0 & 63) == 0;
     if constexpr (sizeof(T) == 8) {
         double out[9];
-        collide_f64(a, p, -1, 0, i, j, out);
+        collide_f64(a, p, -1, {}, i, j, out);
         if (lines) store9_stream(a, own, out);
         else store9(a, own, out);
     } else {
         float out[9];
-        collide_shifted<sizeof(T) == 2>(a, p, -1, 0, i, j, out);
+        collide_shifted<sizeof(T) == 2>(a, p, -1, {}, i, j, out);
         encode_store<T>(a, own, out, lines);
     }
 }
@@ -1358,6 +1381,8 @@ __device__ __forceinline__ void run_lane(const StepArgs &a, int i, int j, int s0
                  "+v"(raw[6]), "+v"(raw[7]), "+v"(raw[8]));
     run_finish<T>(a, i, j, s0, n, lane, act, raw);
 }
+
+#include "lbm_march.h"
 
 // The time-step kernel of one lattice: wave w of the (XCD-remapped) grid
 // owns segments [w mod wpc] * R .. of column w / wpc.
@@ -1926,6 +1951,69 @@ hipError_t launch_step_t(bool gather, StepArgs a, hipStream_t s)
     return launch_perimeter<T>(a, s);
 }
 
+// Waves per SIMD the marching kernels' registers allow.
+template <typename T>
+constexpr int64_t kMarchWaves = sizeof(T) == 8 ? 2 : 3;
+
+// Deals the columns to waves.  A wave computes cols + 2 K columns' levels
+// for cols columns of results, so long chunks waste less, but the waves
+// should fill the chip a whole number of times (every wave takes about the
+// same time): the longest chunk of at most kMarchCols columns that does.
+// Small lattices: as many chunks as fit on the chip at once, of at least
+// kMarchMinCols columns.  Measured at K = 4, us a step by cols: FP64
+// 4096^2 open 141.8 (40), 143.6 (56, 2.6 fills), 136.0 (78, 2 fills), 169
+// (146, 1 fill); porous 8192^2 FP32 278 (32), 271 (64), 273 (128); FP64
+// 512 x 2048 16.0 (8), 14.3 (12), 17.2 (16).
+constexpr int64_t kMarchCols = 80, kMarchMinCols = 6;
+
+template <typename T, int K>
+MarchPlan march_plan(const StepArgs &a)
+{
+    constexpr int32_t kRows = 64 - 2 * K;
+    const int32_t nr = a.g.nr, nc = a.g.nc;
+    MarchPlan m{};
+    m.stripes = (nr + kRows - 1) / kRows;
+    if (nc < 2 * (K + 1) + 1) {  // no column is free of the first and last columns' influence
+        m.top = m.stripes;
+    } else {
+        m.top = a.wet_top ? 1 : 0;
+        if (a.wet_bottom)
+            for (int32_t q = m.stripes - 1; q >= m.top && q * kRows - K + 64 >= nr; --q) ++m.bottom;
+    }
+    const int64_t inner = m.stripes - m.top - m.bottom, free_cols = nc - 2 * (K + 1);
+    // edge waves are slower and start first: short ones, shorter still
+    // where the whole launch is short
+    m.edge_cols = (int64_t)nr * nc < (int64_t)1 << 21 ? 2 : 8;
+    m.edge_chunks = (nc + m.edge_cols - 1) / m.edge_cols;
+    m.edge_row_waves = (m.top + m.bottom) * m.edge_chunks;
+    m.edge_waves = (int32_t)((m.edge_row_waves + 2 * inner + 3) & ~(int64_t)3);
+    m.xcd_chunk = std::max(1, m.stripes / 4);  // about one chunk of columns per XCD
+    m.cols = kMarchMinCols;
+    if (inner > 0) {
+        const int64_t chip = a.cus * 4 * kMarchWaves<T>;
+        for (int64_t fills = 1;; ++fills) {
+            const int64_t chunks = (fills * chip - m.edge_waves) / inner;
+            if (chunks < 1) continue;
+            const int64_t cols = (free_cols + chunks - 1) / chunks;
+            if (cols > kMarchCols) continue;
+            m.cols = (int32_t)std::max(cols, kMarchMinCols);
+            break;
+        }
+    }
+    return m;
+}
+
+template <typename T, int K>
+hipError_t launch_march_t(StepArgs a, hipStream_t s)
+{
+    const MarchPlan m = march_plan<T, K>(a);
+    const int64_t inner = m.stripes - m.top - m.bottom;
+    const int64_t chunks = inner > 0 ? (a.g.nc - 2 * (K + 1) + m.cols - 1) / m.cols : 0;
+    a.nblocks = (m.edge_waves + inner * chunks + kBlockRows / 64 - 1) / (kBlockRows / 64);
+    hipLaunchKernelGGL((march_kernel<T, K>), dim3((unsigned)a.nblocks), dim3(kBlockRows), 0, s, a, m);
+    return hipGetLastError();
+}
+
 template <typename T>
 hipError_t launch_step_tab(StepArgs a, hipStream_t s)
 {
@@ -2085,6 +2173,33 @@ hipError_t launch_batch_step(int32_t storage, bool gather, int32_t R, const Batc
     case kF64: return launch_batch_r<double>(gather, R, b, blocks, s);
     case kF32: return launch_batch_r<float>(gather, R, b, blocks, s);
     default: return launch_batch_r<_Float16>(gather, R, b, blocks, s);
+    }
+}
+
+// A launch of marching waves takes at least the time one wave needs for its
+// columns (30 us at K = 4 in FP64, half of it in FP32; more where the top
+// or bottom row is wet), so lattices below 2^17 nodes keep single steps
+// there.  Measured, us a step, single -> marching: cavity 300^2 FP64 9.0 ->
+// 8.9, FP32 8.0 -> 7.3; 400^2 11.7 -> 8.7, 9.0 -> 7.4; 200^2 8.2 -> 9.1;
+// channel 200 x 1000 12.0 -> 7.6, 9.4 -> 5.3.  FP64 at K = 5 is 5-7 % faster
+// than K = 4 on 4096^2 (BGK; the same in TRT) and slower on small lattices.
+int32_t march_steps(int32_t storage, const StepArgs &a)
+{
+    const int64_t nodes = (int64_t)a.g.nr * a.g.nc;
+    if (storage == kF16 || a.psbb || !a.block_mask || nodes < (int64_t)1 << 17) return 0;
+    return storage == kF64 && nodes >= (int64_t)1 << 22 ? 5 : 4;
+}
+
+hipError_t launch_march(int32_t storage, int32_t steps, const StepArgs &a, hipStream_t s)
+{
+    if (storage == kF16 || a.psbb || !a.block_mask) return hipErrorInvalidValue;
+    const bool f64 = storage == kF64;
+    switch (steps) {
+    case 2: return f64 ? launch_march_t<double, 2>(a, s) : launch_march_t<float, 2>(a, s);
+    case 3: return f64 ? launch_march_t<double, 3>(a, s) : launch_march_t<float, 3>(a, s);
+    case 4: return f64 ? launch_march_t<double, 4>(a, s) : launch_march_t<float, 4>(a, s);
+    case 5: return f64 ? launch_march_t<double, 5>(a, s) : hipErrorInvalidValue;
+    default: return hipErrorInvalidValue;
     }
 }
 
