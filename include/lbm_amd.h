@@ -338,7 +338,9 @@ int lbm_autotune(lbm_ctx *ctx, int32_t steps, int32_t *segments, double *ms_per_
  * process (Lattice.hpp:287-425).  An ensemble groups lattices that were
  * set up as usual (lbm_create, lbm_set_geometry, lbm_set_open_values,
  * lbm_init_equilibrium or lbm_upload_populations) and advances all of them
- * with one step-kernel launch per time step over a table of tiles
+ * with one step-kernel launch per time step (several time steps per launch
+ * where all samples are blocked FP64 or FP32 and no launch shape was set by
+ * hand) over a table of tiles
  * (sample, column, 64*R rows) -- one wave per tile by default, or a
  * persistent grid that walks the table -- plus one small launch for the
  * samples' perimeter segments.  Each sample's results are those of
@@ -370,8 +372,9 @@ int lbm_batch_get_launch(lbm_batch *batch, int32_t *segments, int64_t *blocks);
  * or 2, 4, 8, 16 persistent work-groups per compute unit; and wet-run
  * waves) over `steps`
  * launches each (a launch rewrites the spare buffer from the current
- * state, so the state does not change) and keeps the fastest.  Reports
- * the choice and its time per step (any output may be NULL). */
+ * state, so the state does not change) and keeps the fastest, and several
+ * steps per launch if they are faster still.  Reports the shape of the
+ * single steps and the time per step (any output may be NULL). */
 int lbm_batch_autotune(lbm_batch *batch, int32_t steps, int32_t *segments, int64_t *blocks,
                        double *ms_per_step);
 

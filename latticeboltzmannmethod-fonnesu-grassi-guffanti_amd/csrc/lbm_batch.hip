@@ -5,8 +5,10 @@
 // row of R 64-row segments) covering every tile that holds a wet node.
 // One time step of the whole ensemble is one launch of batch_kernel, a
 // persistent grid that walks the table.  Runs of steps replay a captured
-// HIP graph of kGraphSteps launches (an even number, so a replay leaves
-// the buffer parity unchanged).
+// HIP graph of an even number of launches, so a replay leaves the buffer
+// parity unchanged.  Steps without new prescribed values run kBatchMarchSteps
+// to a launch (batch_march_kernel) where every sample is blocked FP64 or
+// FP32, unless a launch shape was set by hand.
 //
 // Parity bookkeeping: sample s's state is in buffer base_cur[s] ^ phase,
 // where phase counts the ensemble's steps mod 2 since the sample's
@@ -25,7 +27,9 @@ using namespace lbm;
 
 namespace {
 
-constexpr int64_t kGraphSteps = 32;
+// Launches of a captured graph, an even number (see below): 32 of one step,
+// or 8 of kBatchMarchSteps steps.
+constexpr int64_t kGraphLaunches = 32, kMarchGraphLaunches = 8;
 
 // Device copy of an argument array, uploaded from pinned staging memory on
 // the batch stream (ordered after the launches that read the old copy).
@@ -61,6 +65,10 @@ struct lbm_batch {
     // wet-run table (launch shape kRunLaunch): every sample's runs
     int32_t *d_runs = nullptr;
     int64_t nruns = 0;
+    // marching waves (several steps per launch); march: they are in use
+    int32_t *d_marches = nullptr;
+    int64_t nmarches = 0;
+    bool march = false;
     // "first" = each sample's arguments as lbm_step would build them for its
     // next step; "steady" = the same with the previous prescribed values set
     // to the current ones (every step after the first of a run)
@@ -213,6 +221,32 @@ int build_runs(lbm_batch *b)
     return LBM_OK;
 }
 
+// Table of the marching waves.  Chunks of columns: the longest of these
+// that still fill the chip twice over (each wave recomputes the 2 K columns
+// at its ends), and the shortest for ensembles that never do.
+int build_marches(lbm_batch *b)
+{
+    int64_t nodes = 0;
+    std::vector<StepArgs> args;
+    for (const lbm_ctx *c : b->samples) {
+        if (c->storage == kF16 || !c->blocked) return LBM_OK;
+        nodes += c->nr * c->nc;
+        args.push_back(make_args(c));
+    }
+    if (nodes < kMarchMinNodes) return LBM_OK;
+    std::vector<int32_t> table;
+    const int64_t chip = (int64_t)b->cus * 4 * (b->storage == kF64 ? 2 : 3);
+    for (int32_t cols : {48, 32, 24, 16, 12, 8, 6}) {
+        march_table(args.data(), (int64_t)args.size(), cols, table);
+        if ((int64_t)table.size() / 4 >= 2 * chip) break;
+    }
+    b->nmarches = (int64_t)table.size() / 4;
+    HIP_TRY(hipMalloc(&b->d_marches, table.size() * sizeof(int32_t)));
+    HIP_TRY(hipMemcpy(b->d_marches, table.data(), table.size() * sizeof(int32_t), hipMemcpyHostToDevice));
+    b->march = true;
+    return LBM_OK;
+}
+
 int64_t round8(int64_t v) { return std::max<int64_t>(8, (v + 7) / 8 * 8); }
 
 // Brings the device arguments up to date with the samples: a sample whose
@@ -260,7 +294,17 @@ BatchArgs batch_args(const lbm_batch *b, const ArgBuffer &ab, int parity)
     a.direct = 0;
     a.runs = b->d_runs;
     a.nruns = b->nruns;
+    a.marches = b->d_marches;
+    a.nmarches = b->nmarches;
     return a;
+}
+
+// One launch of steady steps (b->march: kBatchMarchSteps of them).
+hipError_t launch_steady(const lbm_batch *b, int phase)
+{
+    const BatchArgs a = batch_args(b, b->steady, phase);
+    return b->march ? launch_batch_march(b->storage, a, b->stream)
+                    : launch_batch_step(b->storage, true, b->R, a, b->blocks, b->stream);
 }
 
 int capture_graph(lbm_batch *b, int phase)
@@ -268,9 +312,8 @@ int capture_graph(lbm_batch *b, int phase)
     hipGraph_t g = nullptr;
     HIP_TRY(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
     hipError_t err = hipSuccess;
-    for (int64_t k = 0; k < kGraphSteps && err == hipSuccess; ++k)
-        err = launch_batch_step(b->storage, true, b->R, batch_args(b, b->steady, phase ^ (int)(k & 1)), b->blocks,
-                                b->stream);
+    const int64_t launches = b->march ? kMarchGraphLaunches : kGraphLaunches;
+    for (int64_t k = 0; k < launches && err == hipSuccess; ++k) err = launch_steady(b, phase ^ (int)(k & 1));
     hipError_t e2 = hipStreamEndCapture(b->stream, &g);
     if (err != hipSuccess) return fail(LBM_ERR_HIP, "batch graph capture: %s", hipGetErrorString(err));
     if (e2 != hipSuccess) return fail(LBM_ERR_HIP, "hipStreamEndCapture: %s", hipGetErrorString(e2));
@@ -342,6 +385,7 @@ int lbm_batch_create(lbm_ctx *const *samples, int64_t n, lbm_batch **out)
     if (!r) r = build_tiles(b, b->R);
     if (!r) r = build_perimeter_tiles(b);
     if (!r) r = build_runs(b);
+    if (!r) r = build_marches(b);
     if (r) return bail(r);
     for (lbm_ctx *c : b->samples) c->batch = b;
     *out = b;
@@ -361,6 +405,7 @@ int lbm_batch_destroy(lbm_batch *b)
     (void)hipFree(b->d_tiles);
     (void)hipFree(b->d_ptiles);
     (void)hipFree(b->d_runs);
+    (void)hipFree(b->d_marches);
     (void)hipFree(b->d_tile_begin);
     (void)hipFree(b->d_flags);
     (void)hipFree(b->d_partials);
@@ -389,9 +434,10 @@ int lbm_batch_set_launch(lbm_batch *b, int32_t segments, int64_t blocks)
         int r = build_tiles(b, tiles_R);
         if (r) return r;
     }
-    if (nb != b->blocks || segments != b->R) drop_graphs(b);
+    if (nb != b->blocks || segments != b->R || b->march) drop_graphs(b);
     b->R = segments;
     b->blocks = nb;
+    b->march = false;
     return LBM_OK;
 }
 
@@ -444,6 +490,21 @@ int lbm_batch_autotune(lbm_batch *b, int32_t steps, int32_t *segments, int64_t *
     if (r) return r;
     b->R = best_R;
     b->blocks = best_nb;
+    b->march = false;
+    if (b->nmarches > 0) {  // several steps per launch against the best single step
+        const BatchArgs ba = batch_args(b, b->steady, b->phase);
+        HIP_TRY(launch_batch_march(b->storage, ba, b->stream));
+        HIP_TRY(hipEventRecord(b->t0, b->stream));
+        for (int32_t s = 0; s < steps; ++s) HIP_TRY(launch_batch_march(b->storage, ba, b->stream));
+        HIP_TRY(hipEventRecord(b->t1, b->stream));
+        HIP_TRY(hipEventSynchronize(b->t1));
+        float ms = 0.f;
+        HIP_TRY(hipEventElapsedTime(&ms, b->t0, b->t1));
+        if (ms / kBatchMarchSteps < best) {
+            best = ms / kBatchMarchSteps;
+            b->march = true;
+        }
+    }
     drop_graphs(b);
     if (segments) *segments = best_R;
     if (blocks) *blocks = best_nb;
@@ -483,12 +544,17 @@ int lbm_batch_step(lbm_batch *b, int64_t n, uint32_t flags)
             r = upload_args(b, b->first, false);
             if (r) return r;
         }
-        if (!(flags & LBM_STEP_NO_GRAPH) && left >= kGraphSteps) {
-            if (!b->graph[b->phase]) {
+        if (!(flags & LBM_STEP_NO_GRAPH)) {
+            const int64_t per_graph = b->march ? kMarchGraphLaunches * kBatchMarchSteps : kGraphLaunches;
+            if (left >= per_graph && !b->graph[b->phase]) {
                 r = capture_graph(b, b->phase);
                 if (r) return r;
             }
-            for (; left >= kGraphSteps; left -= kGraphSteps) HIP_TRY(hipGraphLaunch(b->graph[b->phase], b->stream));
+            for (; left >= per_graph; left -= per_graph) HIP_TRY(hipGraphLaunch(b->graph[b->phase], b->stream));
+            for (; b->march && left >= kBatchMarchSteps; left -= kBatchMarchSteps) {
+                HIP_TRY(launch_steady(b, b->phase));
+                b->phase ^= 1;
+            }
         }
         for (; left > 0; --left) {
             HIP_TRY(launch_batch_step(b->storage, true, b->R, batch_args(b, b->steady, b->phase), b->blocks, b->stream));

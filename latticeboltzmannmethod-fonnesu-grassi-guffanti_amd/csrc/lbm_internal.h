@@ -5,6 +5,7 @@
 
 #include <hip/hip_runtime.h>
 #include <cstdint>
+#include <vector>
 
 #include "../../include/lbm_amd.h"
 
@@ -161,7 +162,18 @@ struct BatchArgs {
     // wet rows (each sample's own run table, as run_kernel reads it)
     const int32_t *runs;
     int64_t nruns;
+    // marching waves of the ensemble: per wave, 4 int32 -- sample, first
+    // row of the window, columns [j0, j1) (sign bit of j1: perimeter window)
+    const int32_t *marches;
+    int64_t nmarches;
 };
+
+// Steps per launch of an ensemble's marching waves, their table over chunks
+// of `cols` columns (a[s]: any of sample s's arguments), and a launch: the
+// samples blocked and without new prescribed values.
+constexpr int32_t kBatchMarchSteps = 4;
+void march_table(const StepArgs *a, int64_t samples, int32_t cols, std::vector<int32_t> &table);
+hipError_t launch_batch_march(int32_t storage, const BatchArgs &b, hipStream_t s);
 
 // Per-sample FP64 sums (readout's five) of a batch's current state:
 // out[5 s + k].  partials needs 5 * ntiles doubles; tile_begin has
@@ -199,6 +211,8 @@ hipError_t launch_lift_drag(int32_t storage, const StepArgs &a, const void *fsta
                             int64_t *nblocks_out, hipStream_t s);
 hipError_t launch_reduce_partials(const double *partials, int64_t nblocks, int32_t ncomp, double *out,
                                   hipStream_t s);
+// Lattices (or ensembles) of fewer nodes keep one step per launch.
+constexpr int64_t kMarchMinNodes = (int64_t)1 << 17;
 // Steps per launch of the marching kernel for this lattice (0: not for it),
 // and such a launch: `steps` steps (2 .. march_steps) without new prescribed
 // values from fin (F*) to fout, blocked layout.

@@ -118,3 +118,29 @@ def test_nan_is_reported(storage):
         lat.step(8, L.STEP_CHECK)
     assert e.value.code == L.ERR_NAN
     lat.close()
+
+
+@pytest.mark.parametrize("storage", [L.F64, L.F32_SHIFTED])
+def test_ensemble_same_bits_as_single_steps(storage):
+    """Samples of every small size beside larger ones, all kinds of
+    perimeter: the ensemble's marching launches against its single steps."""
+    shapes = [(3, 3), (5, 9), (57, 10), (56, 11), (64, 12), (113, 40), (300, 200), (129, 700)]
+    rng = np.random.default_rng(17)
+    classes = [random_class(rng, nr, nc, 0.15) for nr, nc in shapes]
+    states = [state(rng, nc, nr) for nr, nc in shapes]
+    out = []
+    for flags in (0, L.STEP_NO_GRAPH):
+        lats = [make(c, np.random.default_rng(k), storage, L.TRT, POLICIES[:2]) for k, c in enumerate(classes)]
+        for lat, p in zip(lats, states):
+            lat.upload_populations(p)
+        with L.Batch(lats) as b:
+            for n in (1, 4, 5, 43):
+                b.step(n, flags)
+            lats[6].set_open_values(0, ux=np.full(len(lats[6].open_nodes(0)), 0.005))
+            b.step(13, flags)
+        assert all(lat.time == 66 for lat in lats)
+        out.append([lat.populations() for lat in lats])
+        for lat in lats:
+            lat.close()
+    for shape, x, y in zip(shapes, *out):
+        assert np.array_equal(x, y), shape
