@@ -107,11 +107,21 @@ namespace {
 // buffer holding the state unchanged.
 constexpr int64_t kGraphLaunches = 8, kGraphSteps = 32;
 
-// Steps per launch of a steady run (1: the step kernels).
-int32_t steps_per_launch(const lbm_ctx *c)
+// How a run's steps are launched: kind kTile / kMarch with `steps` steps a
+// launch, or one step a launch through the step kernels.
+struct Launching {
+    enum Kind { kSingle, kMarch, kTile } kind;
+    int32_t steps;
+};
+
+Launching launching(const lbm_ctx *c)
 {
-    const int32_t k = c->march ? march_steps(c->storage, make_args(c)) : 0;
-    return std::max(k, 1);
+    if (c->multi) {
+        const StepArgs a = make_args(c);
+        if (const int32_t k = tile_steps(c->storage, a)) return {Launching::kTile, k};
+        if (const int32_t k = march_steps(c->storage, a)) return {Launching::kMarch, k};
+    }
+    return {Launching::kSingle, 1};
 }
 
 // Steps per captured graph.
@@ -126,25 +136,30 @@ void drop_graphs(lbm_ctx *c)
         }
 }
 
-// Launch of k steady steps (k = 1: the step kernels) from buffer `in`.
-hipError_t launch_steady(const lbm_ctx *c, int in, int32_t k)
+// Launch of k steps from buffer `in`; steady ones unless the kind is kTile.
+hipError_t launch_steps(const lbm_ctx *c, Launching::Kind kind, int in, int32_t k, double *macro = nullptr)
 {
     StepArgs a = make_args(c);
     a.fin = c->d_F[in];
     a.fout = c->d_F[1 - in];
-    a.macro = nullptr;
-    return k > 1 ? launch_march(c->storage, k, a, c->stream) : launch_step(c->storage, true, a, c->stream, c->segments);
+    a.macro = macro;
+    switch (kind) {
+    case Launching::kTile: return launch_tile(c->storage, k, a, c->stream);
+    case Launching::kMarch: return launch_march(c->storage, k, a, c->stream);
+    default: return launch_step(c->storage, true, a, c->stream, c->segments);
+    }
 }
 
-// Captures a graph's steady steps, per_launch each, from the context's
-// current buffer and prescribed values.
-int capture_steps(lbm_ctx *c, int32_t per_launch)
+// Captures a graph's steady steps from the context's current buffer and
+// prescribed values.
+int capture_steps(lbm_ctx *c, Launching how)
 {
     hipGraph_t g = nullptr;
     HIP_TRY(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
     hipError_t err = hipSuccess;
-    const int64_t launches = graph_steps(per_launch) / per_launch;
-    for (int64_t k = 0; k < launches && err == hipSuccess; ++k) err = launch_steady(c, c->cur ^ (int)(k & 1), per_launch);
+    const int64_t launches = graph_steps(how.steps) / how.steps;
+    for (int64_t k = 0; k < launches && err == hipSuccess; ++k)
+        err = launch_steps(c, how.kind, c->cur ^ (int)(k & 1), how.steps);
     hipError_t e2 = hipStreamEndCapture(c->stream, &g);
     if (err != hipSuccess) return fail(LBM_ERR_HIP, "step graph capture: %s", hipGetErrorString(err));
     if (e2 != hipSuccess) return fail(LBM_ERR_HIP, "hipStreamEndCapture: %s", hipGetErrorString(e2));
@@ -1024,30 +1039,42 @@ int lbm_step(lbm_ctx *c, int64_t n, uint32_t flags)
     if (c->state == kNone) return fail(LBM_ERR_STATE, "no populations (call lbm_init_equilibrium)");
     HIP_TRY(hipSetDevice(c->desc.device));
     const bool macro = (flags & LBM_STEP_MACRO) != 0;
-    const int32_t per_launch = steps_per_launch(c);
+    const Launching how = launching(c);
     for (int64_t s = 0; s < n;) {
         // After the first step of a run (collide-only pass, new prescribed
         // values) every launch takes the same steps on alternating buffers:
         // replay a captured loop of them, then launch the rest, as many
-        // steps at a time as are left.
+        // steps at a time as are left.  Tiles also take the steps with new
+        // values and the one that writes the fields.
         const bool steady = c->state == kFstar && c->bc_prev == c->bc_cur;
-        const int64_t left = n - s - (macro ? 1 : 0);
-        if (!(flags & LBM_STEP_NO_GRAPH) && steady && left >= std::min<int64_t>(per_launch, 2)) {
-            if (left >= graph_steps(per_launch)) {
+        const int64_t left = n - s, plain = left - (macro ? 1 : 0);
+        if (!(flags & LBM_STEP_NO_GRAPH)) {
+            if (steady && plain >= graph_steps(how.steps)) {
                 if (!c->graph[c->cur][c->bc_cur]) {
-                    int r = capture_steps(c, per_launch);
+                    int r = capture_steps(c, how);
                     if (r) return r;
                 }
                 HIP_TRY(hipGraphLaunch(c->graph[c->cur][c->bc_cur], c->stream));
-                c->t += graph_steps(per_launch);
-                s += graph_steps(per_launch);
+                c->t += graph_steps(how.steps);
+                s += graph_steps(how.steps);
                 continue;
             }
-            if (per_launch > 1) {
+            int32_t k = 0;
+            double *fields = nullptr;
+            if (how.kind == Launching::kMarch && steady && plain >= 2) {
                 // no single step is left over where two launches can share the rest
-                const int32_t k = (int32_t)(left == per_launch + 1 ? left - 2 : std::min<int64_t>(left, per_launch));
-                HIP_TRY(launch_steady(c, c->cur, k));
+                k = (int32_t)(plain == how.steps + 1 ? plain - 2 : std::min<int64_t>(plain, how.steps));
+            } else if (how.kind == Launching::kTile && c->state == kFstar) {
+                k = (int32_t)std::min<int64_t>(left, how.steps);
+                if (macro && k == left) {
+                    int r = claim_macro(c, &fields);
+                    if (r) return r;
+                }
+            }
+            if (k > 0) {
+                HIP_TRY(launch_steps(c, how.kind, c->cur, k, fields));
                 c->cur = 1 - c->cur;
+                c->bc_prev = c->bc_cur;
                 c->t += k;
                 s += k;
                 continue;
@@ -1098,7 +1125,7 @@ int lbm_set_launch(lbm_ctx *c, int32_t segments)
         if (r) return r;
     }
     c->segments = segments;
-    c->march = segments == 0;
+    c->multi = segments == 0;
     drop_graphs(c);
     return LBM_OK;
 }
@@ -1185,19 +1212,26 @@ int lbm_autotune(lbm_ctx *c, int32_t steps, int32_t *segments, double *ms_per_st
         }
     }
     // several steps per launch against the best single step
-    bool march = false;
-    const int32_t k = march_steps(c->storage, a);
-    if (k > 1) {
-        if (err == hipSuccess) err = launch_march(c->storage, k, a, c->stream);
+    const bool was_multi = c->multi;
+    c->multi = true;
+    const Launching how = launching(c);
+    c->multi = was_multi;
+    bool multi = false;
+    if (how.kind != Launching::kSingle) {
+        auto launch = [&] {
+            return how.kind == Launching::kTile ? launch_tile(c->storage, how.steps, a, c->stream)
+                                                : launch_march(c->storage, how.steps, a, c->stream);
+        };
+        if (err == hipSuccess) err = launch();
         if (err == hipSuccess) err = hipEventRecord(t0, c->stream);
-        for (int32_t s = 0; s < steps && err == hipSuccess; ++s) err = launch_march(c->storage, k, a, c->stream);
+        for (int32_t s = 0; s < steps && err == hipSuccess; ++s) err = launch();
         if (err == hipSuccess) err = hipEventRecord(t1, c->stream);
         if (err == hipSuccess) err = hipEventSynchronize(t1);
         float ms = 0.f;
         if (err == hipSuccess) err = hipEventElapsedTime(&ms, t0, t1);
-        if (err == hipSuccess && ms / (float)k < best) {
-            best = ms / (float)k;
-            march = true;
+        if (err == hipSuccess && ms / (float)how.steps < best) {
+            best = ms / (float)how.steps;
+            multi = true;
         }
     }
     (void)hipEventDestroy(t0);
@@ -1205,7 +1239,7 @@ int lbm_autotune(lbm_ctx *c, int32_t steps, int32_t *segments, double *ms_per_st
     if (err != hipSuccess) return fail(LBM_ERR_HIP, "autotune: %s", hipGetErrorString(err));
     c->segments = best_R;
     c->occupancy = best_occ;
-    c->march = march;
+    c->multi = multi;
     drop_graphs(c);
     if (segments) *segments = best_R;
     if (ms_per_step) *ms_per_step = best / steps;

@@ -114,7 +114,7 @@ struct lbm_ctx {
     int32_t segments = 0;
     // several steps per launch where nothing asks for single ones: off while
     // a shape is set by hand, or where the autotuner measured it slower
-    bool march = true;
+    bool multi = true;
     int32_t cus = 256;  // compute units of the device
     // partially saturated bounce-back of the wet obstacles (lbm_set_partial_bounce_back)
     bool psbb = false;

@@ -211,13 +211,22 @@ hipError_t launch_lift_drag(int32_t storage, const StepArgs &a, const void *fsta
                             int64_t *nblocks_out, hipStream_t s);
 hipError_t launch_reduce_partials(const double *partials, int64_t nblocks, int32_t ncomp, double *out,
                                   hipStream_t s);
-// Lattices (or ensembles) of fewer nodes keep one step per launch.
+// Lattices below these node counts take tiles (tile_steps), FP64 and FP32
+// lattices from there on marching waves; ensembles take marching waves from
+// kMarchMinNodes nodes in all.
+constexpr int64_t kTileMaxNodes = 300000, kTileMaxNodesF16 = (int64_t)1 << 19;
 constexpr int64_t kMarchMinNodes = (int64_t)1 << 17;
 // Steps per launch of the marching kernel for this lattice (0: not for it),
 // and such a launch: `steps` steps (2 .. march_steps) without new prescribed
 // values from fin (F*) to fout, blocked layout.
 int32_t march_steps(int32_t storage, const StepArgs &a);
 hipError_t launch_march(int32_t storage, int32_t steps, const StepArgs &a, hipStream_t s);
+// Steps per launch of the tile kernel for this lattice (0: not for it), and
+// such a launch of 1 .. tile_steps steps from fin (F*) to fout.  The first
+// gather is closed with bc_prev, everything after takes bc_cur; a.macro is
+// written by the last step.
+int32_t tile_steps(int32_t storage, const StepArgs &a);
+hipError_t launch_tile(int32_t storage, int32_t steps, const StepArgs &a, hipStream_t s);
 int64_t readout_blocks(const StepArgs &a);
 // rho = 1, u = 0 over a field of n nodes ([3][n] doubles).
 hipError_t launch_fill_macro(double *macro, int64_t n, hipStream_t s);

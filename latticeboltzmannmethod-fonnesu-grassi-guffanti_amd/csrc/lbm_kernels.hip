@@ -995,50 +995,76 @@ __device__ __forceinline__ bool collide_shifted(const StepArgs &a, const float *
     return nan;
 }
 
-// Converts the post-collision shifted populations to the storage type and
-// stores them (whole_lines: non-temporal, see store9_stream).  FP16 values
-// arrive scaled (collide_shifted<true>).  FP16 rounds stochastically unless
-// the context asked for round-to-nearest: 13 random bits are added below
-// the FP16 cut of the FP32 value, which is then converted toward zero
-// (sign-magnitude, so the same for both signs; two values per packed
-// conversion).  The bits come from one hash per node of its index and its
-// new rest population, a different window per direction.  Each rounding
-// mode stores in its own branch so the uniform flag stays a branch instead
-// of both conversions being computed and selected.
+// Range guard of FP16 storage: a scaled value at or beyond the largest FP16
+// number (65504) would be clamped by the conversion toward zero or become
+// infinite to nearest; bit 1 of the flag reports it (the storage scale is
+// too large for the flow).  NaNs pass fmaxf unnoticed: the density check
+// reports them.
+__device__ __forceinline__ void range_guard(const StepArgs &a, const float *o)
+{
+    const float mx = fmaxf(fmaxf(fmaxf(fabsf(o[0]), fabsf(o[1])), fmaxf(fabsf(o[2]), fabsf(o[3]))),
+                           fmaxf(fmaxf(fabsf(o[4]), fabsf(o[5])),
+                                 fmaxf(fmaxf(fabsf(o[6]), fabsf(o[7])), fabsf(o[8]))));
+    if (mx >= 65504.f) atomicOr(a.flag, 2);
+}
+
+// Stochastic rounding of a node's nine scaled values to FP16: 13 random
+// bits are added below the FP16 cut of the FP32 value, which is then
+// converted toward zero (sign-magnitude, so the same for both signs; two
+// values per packed conversion).  The bits come from one hash per node of
+// its index and its new rest population, a different window per direction.
+template <typename T>
+__device__ __forceinline__ void round_stochastic(int64_t n, const float *o, T *raw)
+{
+    uint32_t h = (uint32_t)n * 0x9E3779B9u ^ __float_as_uint(o[0]);
+    h ^= h >> 16;
+    h *= 0x85EBCA6Bu;
+    h ^= h >> 13;
+    h *= 0xC2B2AE35u;
+    h ^= h >> 16;
+    float u[10];
+#pragma unroll
+    for (int d = 0; d < 9; ++d) {
+        const uint32_t r = __builtin_amdgcn_alignbit(h, h, 3 * d) & 0x1FFFu;
+        u[d] = __uint_as_float(__float_as_uint(o[d]) + r);
+    }
+    u[9] = 0.f;
+#pragma unroll
+    for (int d = 0; d < 9; d += 2) {
+        const auto p = __builtin_amdgcn_cvt_pkrtz(u[d], u[d + 1]);
+        raw[d] = (T)p[0];
+        if (d + 1 < 9) raw[d + 1] = (T)p[1];
+    }
+}
+
+// Converts the post-collision shifted populations to the storage type (FP16
+// values arrive scaled, collide_shifted<true>, and round stochastically
+// unless the context asked for round-to-nearest).
+template <typename T>
+__device__ __forceinline__ void encode(const StepArgs &a, int64_t n, const float *o, T *raw)
+{
+    if constexpr (sizeof(T) == 2) {
+        range_guard(a, o);
+        if (a.f16_sr) {
+            round_stochastic(n, o, raw);
+            return;
+        }
+    }
+#pragma unroll
+    for (int d = 0; d < 9; ++d) raw[d] = (T)o[d];
+}
+
+// Encodes and stores (whole_lines: non-temporal, see store9_stream).  Each
+// rounding mode stores in its own branch so the uniform flag stays a branch
+// instead of both conversions being computed and selected.
 template <typename T>
 __device__ __forceinline__ void encode_store(const StepArgs &a, int64_t n, const float *o, bool whole_lines)
 {
     T raw[9];
     if constexpr (sizeof(T) == 2) {
-        // Range guard: a scaled value at or beyond the largest FP16 number
-        // (65504) would be clamped by the conversion toward zero or become
-        // infinite to nearest; bit 1 of the flag reports it (the storage
-        // scale is too large for the flow).  NaNs pass fmaxf unnoticed:
-        // the density check above reports them.
-        const float mx = fmaxf(fmaxf(fmaxf(fabsf(o[0]), fabsf(o[1])), fmaxf(fabsf(o[2]), fabsf(o[3]))),
-                               fmaxf(fmaxf(fabsf(o[4]), fabsf(o[5])),
-                                     fmaxf(fmaxf(fabsf(o[6]), fabsf(o[7])), fabsf(o[8]))));
-        if (mx >= 65504.f) atomicOr(a.flag, 2);
+        range_guard(a, o);
         if (a.f16_sr) {
-            uint32_t h = (uint32_t)n * 0x9E3779B9u ^ __float_as_uint(o[0]);
-            h ^= h >> 16;
-            h *= 0x85EBCA6Bu;
-            h ^= h >> 13;
-            h *= 0xC2B2AE35u;
-            h ^= h >> 16;
-            float u[10];
-#pragma unroll
-            for (int d = 0; d < 9; ++d) {
-                const uint32_t r = __builtin_amdgcn_alignbit(h, h, 3 * d) & 0x1FFFu;
-                u[d] = __uint_as_float(__float_as_uint(o[d]) + r);
-            }
-            u[9] = 0.f;
-#pragma unroll
-            for (int d = 0; d < 9; d += 2) {
-                const auto p = __builtin_amdgcn_cvt_pkrtz(u[d], u[d + 1]);
-                raw[d] = (T)p[0];
-                if (d + 1 < 9) raw[d + 1] = (T)p[1];
-            }
+            round_stochastic(n, o, raw);
             if (whole_lines) store9_stream(a, n, raw);
             else store9(a, n, raw);
             return;
@@ -1383,6 +1409,7 @@ __device__ __forceinline__ void run_lane(const StepArgs &a, int i, int j, int s0
 }
 
 #include "lbm_march.h"
+#include "lbm_tile.h"
 
 // The time-step kernel of one lattice: wave w of the (XCD-remapped) grid
 // owns segments [w mod wpc] * R .. of column w / wpc.
@@ -2218,15 +2245,13 @@ hipError_t launch_batch_step(int32_t storage, bool gather, int32_t R, const Batc
 
 // A launch of marching waves takes at least the time one wave needs for its
 // columns (30 us at K = 4 in FP64, half of it in FP32; more where the top
-// or bottom row is wet), so lattices below 2^17 nodes keep single steps
-// there.  Measured, us a step, single -> marching: cavity 300^2 FP64 9.0 ->
-// 8.9, FP32 8.0 -> 7.3; 400^2 11.7 -> 8.7, 9.0 -> 7.4; 200^2 8.2 -> 9.1;
-// channel 200 x 1000 12.0 -> 7.6, 9.4 -> 5.3.  FP64 at K = 5 is 5-7 % faster
-// than K = 4 on 4096^2 (BGK; the same in TRT) and slower on small lattices.
+// or bottom row is wet): small lattices take tiles (tile_shape).  FP64 at
+// K = 5 is 5-7 % faster than K = 4 on 4096^2 (BGK; the same in TRT) and
+// slower on small lattices.
 int32_t march_steps(int32_t storage, const StepArgs &a)
 {
     const int64_t nodes = (int64_t)a.g.nr * a.g.nc;
-    if (storage == kF16 || a.psbb || !a.block_mask || nodes < kMarchMinNodes) return 0;
+    if (storage == kF16 || a.psbb || !a.block_mask || nodes < kTileMaxNodes) return 0;
     return storage == kF64 && nodes >= (int64_t)1 << 22 ? 5 : 4;
 }
 
@@ -2240,6 +2265,68 @@ hipError_t launch_march(int32_t storage, int32_t steps, const StepArgs &a, hipSt
     case 4: return f64 ? launch_march_t<double, 4>(a, s) : launch_march_t<float, 4>(a, s);
     case 5: return f64 ? launch_march_t<double, 5>(a, s) : hipErrorInvalidValue;
     default: return hipErrorInvalidValue;
+    }
+}
+
+namespace {
+
+struct TileShape {
+    int32_t side, halo;  // halo 0: no tiles for this lattice
+};
+
+int64_t tiles_of(const StepArgs &a, TileShape t)
+{
+    const int64_t n = t.side - 2 * t.halo;
+    return ((a.g.nr + n - 1) / n) * ((a.g.nc + n - 1) / n);
+}
+
+// As many steps a launch as leave one tile per CU: more steps share a
+// launch's fixed cost, and a second tile on a CU costs what it saves.  The
+// 24 x 24 region steps faster (1.3 us against 1.55 in FP64) and holds 6
+// steps where the lattice is small enough; then 32 x 32.  Beyond one tile
+// per CU, two; then 4 steps.  Measured, us a step in FP64: 129^2 24 x 24 at
+// 4 / 6 / 8 steps 2.52 / 2.12 / 2.54, 32 x 32 at 10 2.15; 200^2 24 x 24 at
+// 5 2.76, 32 x 32 at 8 2.67; 400^2 32 x 32 at 4 / 6 / 8 5.5 / 5.0 / 5.8;
+// 251 x 1003 7.1 / 7.9 / 8.3.  From about 300000 nodes the marching waves
+// are as fast (FP64 / FP32: 1400 x 200 march 7.8 / 5.6, porous 500 x 700 7.6
+// / 5.7; 500^2 tiles 7.0 / 4.9); FP16, which has none, stays until single
+// steps are (700^2 8.5 against 12.4, 1000^2 16.4).
+TileShape tile_shape(int32_t storage, const StepArgs &a)
+{
+    const int64_t nodes = (int64_t)a.g.nr * a.g.nc;
+    if (a.psbb || nodes >= (storage == kF16 ? kTileMaxNodesF16 : kTileMaxNodes)) return {0, 0};
+    for (int32_t halo = 8; halo >= 6; --halo)
+        if (tiles_of(a, {24, halo}) <= a.cus) return {24, halo};
+    for (int32_t per_cu : {1, 2})
+        for (int32_t halo = 10; halo >= 4; --halo)
+            if (tiles_of(a, {32, halo}) <= (int64_t)per_cu * a.cus) return {32, halo};
+    return {32, 4};
+}
+
+template <typename T>
+hipError_t launch_tile_t(const StepArgs &a, TileShape t, int32_t steps, hipStream_t s)
+{
+    const int32_t n = t.side - 2 * t.halo, ti = (a.g.nr + n - 1) / n;
+    const dim3 grid((unsigned)tiles_of(a, t)), block((unsigned)(t.side * t.side));
+    if (t.side == 24) hipLaunchKernelGGL((tile_kernel<T, 24>), grid, block, 0, s, a, steps, t.halo, ti);
+    else hipLaunchKernelGGL((tile_kernel<T, 32>), grid, block, 0, s, a, steps, t.halo, ti);
+    return hipGetLastError();
+}
+
+}  // namespace
+
+int32_t tile_steps(int32_t storage, const StepArgs &a) { return tile_shape(storage, a).halo; }
+
+hipError_t launch_tile(int32_t storage, int32_t steps, const StepArgs &a0, hipStream_t s)
+{
+    StepArgs a = a0;
+    set_planes(a);
+    const TileShape t = tile_shape(storage, a);
+    if (steps < 1 || steps > t.halo) return hipErrorInvalidValue;
+    switch (storage) {
+    case kF64: return launch_tile_t<double>(a, t, steps, s);
+    case kF32: return launch_tile_t<float>(a, t, steps, s);
+    default: return launch_tile_t<_Float16>(a, t, steps, s);
     }
 }
 

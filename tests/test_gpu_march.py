@@ -44,9 +44,9 @@ def state(rng, nc, nr):
 
 # windows end at these row counts (wide lattices), chunks at these column
 # counts (tall ones); all of the sizes that take several steps a launch
-SIZES = [(3, 43700), (53, 2480), (54, 2440), (55, 2400), (56, 2350), (57, 2301), (58, 2270), (60, 2200), (64, 2048),
-         (65, 2021), (112, 1180), (113, 1170), (14600, 9), (13200, 10), (12000, 11), (11000, 12), (10100, 13),
-         (9400, 14), (260, 521)]
+SIZES = [(3, 100100), (53, 5700), (54, 5560), (55, 5460), (56, 5370), (57, 5301), (58, 5190), (60, 5003), (64, 4700),
+         (65, 4630), (112, 2680), (113, 2670), (33400, 9), (30100, 10), (27300, 11), (25100, 12), (23100, 13),
+         (21500, 14), (560, 541)]
 
 
 @pytest.mark.parametrize("storage", [L.F64, L.F32_SHIFTED])
