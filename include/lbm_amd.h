@@ -327,8 +327,8 @@ int lbm_get_occupancy(lbm_ctx *ctx, int32_t *groups_per_cu);
  * (outputs may be NULL); lbm_get_occupancy reports the occupancy.  LBM_ERR_STATE for a context
  * that belongs to an ensemble (the ensemble has its own,
  * lbm_batch_autotune) and for a lattice with partially saturated
- * bounce-back (every launch advances its carried obstacle values).  No
- * counterpart in the reference. */
+ * bounce-back (it has one launch shape).  No counterpart in the
+ * reference. */
 int lbm_autotune(lbm_ctx *ctx, int32_t steps, int32_t *segments, double *ms_per_step);
 
 /* ------------------------------------------------------------------ */

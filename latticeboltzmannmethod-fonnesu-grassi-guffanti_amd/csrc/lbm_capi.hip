@@ -41,6 +41,15 @@ int fail(int code, const char *fmt, ...)
     return code;
 }
 
+// Buffer `in` as a step's input (the other one is its output).
+static void set_input(const lbm_ctx *c, StepArgs &a, int in)
+{
+    a.fin = c->d_F[in];
+    a.fout = c->d_F[1 - in];
+    a.ps_val = c->d_ps_val[in];
+    a.ps_next = c->d_ps_val[1 - in];
+}
+
 StepArgs make_args(const lbm_ctx *c)
 {
     StepArgs a{};
@@ -95,7 +104,7 @@ StepArgs make_args(const lbm_ctx *c)
     a.ps_t = c->psbb ? 1.0 / c->ps_tau : 0.0;
     a.ps_mask = c->d_ps_mask;
     a.ps_b = c->d_ps_b;
-    a.ps_val = c->d_ps_val;
+    set_input(c, a, c->cur);
     return a;
 }
 
@@ -140,8 +149,7 @@ void drop_graphs(lbm_ctx *c)
 hipError_t launch_steps(const lbm_ctx *c, Launching::Kind kind, int in, int32_t k, double *macro = nullptr)
 {
     StepArgs a = make_args(c);
-    a.fin = c->d_F[in];
-    a.fout = c->d_F[1 - in];
+    set_input(c, a, in);
     a.macro = macro;
     switch (kind) {
     case Launching::kTile: return launch_tile(c->storage, k, a, c->stream);
@@ -173,7 +181,10 @@ void free_psbb(lbm_ctx *c)
 {
     (void)hipFree(c->d_ps_mask); c->d_ps_mask = nullptr;
     (void)hipFree(c->d_ps_b); c->d_ps_b = nullptr;
-    (void)hipFree(c->d_ps_val); c->d_ps_val = nullptr;
+    for (double *&v : c->d_ps_val) {
+        (void)hipFree(v);
+        v = nullptr;
+    }
     c->psbb = false;
     c->ps_tau = 0.0;
 }
@@ -645,8 +656,10 @@ int lbm_set_partial_bounce_back(lbm_ctx *c, double tau, const double *b)
     HIP_TRY(hipMemcpy(c->d_ps_mask, mask.data(), plane * sizeof(uint16_t), hipMemcpyHostToDevice));
     HIP_TRY(hipMalloc(&c->d_ps_b, 9 * plane * sizeof(double)));
     HIP_TRY(hipMemcpy(c->d_ps_b, wb.data(), 9 * plane * sizeof(double), hipMemcpyHostToDevice));
-    HIP_TRY(hipMalloc(&c->d_ps_val, 9 * plane * sizeof(double)));
-    HIP_TRY(hipMemset(c->d_ps_val, 0, 9 * plane * sizeof(double)));
+    for (double *&v : c->d_ps_val) {
+        HIP_TRY(hipMalloc(&v, 9 * plane * sizeof(double)));
+        HIP_TRY(hipMemset(v, 0, 9 * plane * sizeof(double)));
+    }
     c->psbb = true;
     c->ps_tau = tau;
     return LBM_OK;
@@ -1081,9 +1094,6 @@ int lbm_step(lbm_ctx *c, int64_t n, uint32_t flags)
             }
         }
         StepArgs a = make_args(c);
-        a.fin = c->d_F[c->cur];
-        a.fout = c->d_F[1 - c->cur];
-        a.macro = nullptr;
         if (macro && s == n - 1) {
             int r = claim_macro(c, &a.macro);
             if (r) return r;
@@ -1168,12 +1178,11 @@ int lbm_autotune(lbm_ctx *c, int32_t steps, int32_t *segments, double *ms_per_st
     if (steps < 1) return fail(LBM_ERR_INVALID, "steps must be >= 1");
     if (c->batch) return fail(LBM_ERR_STATE, "context belongs to an ensemble: tune it with lbm_batch_autotune");
     if (c->state == kNone) return fail(LBM_ERR_STATE, "no populations (call lbm_init_equilibrium)");
-    // Every launch of a partially saturated bounce-back lattice rewrites the
-    // carried obstacle values (ps_val) in place, so a timing launch would
-    // change the state.
+    // A partially saturated bounce-back lattice runs its tiles or one general
+    // kernel: there are no shapes to choose from.
     if (c->psbb)
-        return fail(LBM_ERR_STATE, "autotune: a lattice with partially saturated bounce-back runs one general "
-                                   "kernel and would change its carried obstacle values; set the occupancy by hand");
+        return fail(LBM_ERR_STATE, "autotune: a lattice with partially saturated bounce-back has one launch shape; "
+                                   "set the occupancy by hand");
     HIP_TRY(hipSetDevice(c->desc.device));
     {
         // the tabled-run candidate's tables, before the arguments that point

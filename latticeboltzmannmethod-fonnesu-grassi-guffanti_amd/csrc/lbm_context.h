@@ -121,7 +121,7 @@ struct lbm_ctx {
     double ps_tau = 0.0;
     uint16_t *d_ps_mask = nullptr;
     double *d_ps_b = nullptr;
-    double *d_ps_val = nullptr;
+    double *d_ps_val[2] = {nullptr, nullptr};  // by the buffer holding the state they belong to
     // captured step loops, by [buffer holding the state][prescribed-value copy]
     hipGraphExec_t graph[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};
 };

@@ -114,7 +114,8 @@ struct StepArgs {
     double ps_t;             // 1 / tau of the policy
     const uint16_t *ps_mask; // per wet node (compact index): bit d set when n - c_d is a wet obstacle
     const double *ps_b;      // [9][plane]: weight b of that obstacle
-    double *ps_val;          // [9][plane]: populations entering n through those slots (read, then rewritten)
+    const double *ps_val;    // [9][plane]: populations entering n through those slots
+    double *ps_next;         // the same, written for the next step
 };
 
 // Launch shape value selecting the run kernel: one wave per run of up to 64

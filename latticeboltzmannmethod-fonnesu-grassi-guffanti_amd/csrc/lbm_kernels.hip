@@ -581,24 +581,28 @@ __device__ __forceinline__ void psbb_gather(const StepArgs &a, int64_t n, double
 //   P'_d = p_q - (1 - b) (p_q - e_q) t + b ((P_d - e_d) - (p_q - 2 w_d rho_o))
 // with t = 1 / tau of the policy and 2 w_d written 2 * (1/18) on the axes
 // and 1/36 on the diagonals, in the reference's operation order.
+__device__ __forceinline__ double psbb_value(const StepArgs &a, int d, double b, const double *p, const double *eq,
+                                             const double *o)
+{
+    constexpr double one18 = (1.0 / 18.0);
+    constexpr double one36 = (1.0 / 36.0);
+    const double rho_o = 1.0;
+    const int q = kOpp[d];
+    const double wr = d < 5 ? 2 * one18 * rho_o : one36 * rho_o;
+    const double pq = o[q];
+    return pq - (1.0 - b) * (pq - eq[q]) * a.ps_t + b * ((p[d] - eq[d]) - (pq - wr));
+}
+
 __device__ __forceinline__ void psbb_update(const StepArgs &a, int64_t n, const double *p, const double *eq,
                                             const double *o)
 {
     const uint32_t mask = a.ps_mask[n];
     if (!mask) return;
-    constexpr double one18 = (1.0 / 18.0);
-    constexpr double one36 = (1.0 / 36.0);
-    const double rho_o = 1.0;
-    const double t = a.ps_t;
 #pragma unroll
     for (int d = 1; d < 9; ++d) {
         if (!((mask >> d) & 1u)) continue;
-        const int q = kOpp[d];
         const int64_t k = (int64_t)d * a.g.plane + n;
-        const double b = a.ps_b[k];
-        const double wr = d < 5 ? 2 * one18 * rho_o : one36 * rho_o;
-        const double pq = o[q];
-        a.ps_val[k] = pq - (1.0 - b) * (pq - eq[q]) * t + b * ((p[d] - eq[d]) - (pq - wr));
+        a.ps_next[k] = psbb_value(a, d, a.ps_b[k], p, eq, o);
     }
 }
 
@@ -2294,7 +2298,7 @@ int64_t tiles_of(const StepArgs &a, TileShape t)
 TileShape tile_shape(int32_t storage, const StepArgs &a)
 {
     const int64_t nodes = (int64_t)a.g.nr * a.g.nc;
-    if (a.psbb || nodes >= (storage == kF16 ? kTileMaxNodesF16 : kTileMaxNodes)) return {0, 0};
+    if (nodes >= (storage == kF16 ? kTileMaxNodesF16 : kTileMaxNodes)) return {0, 0};
     for (int32_t halo = 8; halo >= 6; --halo)
         if (tiles_of(a, {24, halo}) <= a.cus) return {24, halo};
     for (int32_t per_cu : {1, 2})
@@ -2308,6 +2312,13 @@ hipError_t launch_tile_t(const StepArgs &a, TileShape t, int32_t steps, hipStrea
 {
     const int32_t n = t.side - 2 * t.halo, ti = (a.g.nr + n - 1) / n;
     const dim3 grid((unsigned)tiles_of(a, t)), block((unsigned)(t.side * t.side));
+    if constexpr (sizeof(T) == 8) {
+        if (a.psbb) {
+            if (t.side == 24) hipLaunchKernelGGL((tile_kernel<T, 24, true>), grid, block, 0, s, a, steps, t.halo, ti);
+            else hipLaunchKernelGGL((tile_kernel<T, 32, true>), grid, block, 0, s, a, steps, t.halo, ti);
+            return hipGetLastError();
+        }
+    }
     if (t.side == 24) hipLaunchKernelGGL((tile_kernel<T, 24>), grid, block, 0, s, a, steps, t.halo, ti);
     else hipLaunchKernelGGL((tile_kernel<T, 32>), grid, block, 0, s, a, steps, t.halo, ti);
     return hipGetLastError();

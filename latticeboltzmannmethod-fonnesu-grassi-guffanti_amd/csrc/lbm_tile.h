@@ -22,7 +22,11 @@
 // FP64 7.0 -> 1.7; 300^2 FP64 9.1 -> 3.3; 251 x 1003 FP32 9.6 -> 5.1.
 //
 // Same arithmetic per node as the step kernels, same bits.
-template <typename T, int kTileSide>
+// PS: partially saturated obstacles (FP64).  A node keeps the populations
+// that enter it through its obstacle slots, and their weights, in registers
+// (psbb_gather, psbb_update); its carried values alternate between two
+// buffers like the state, since the tiles around it read the old ones.
+template <typename T, int kTileSide, bool PS = false>
 __global__ __launch_bounds__(kTileSide * kTileSide) void tile_kernel(StepArgs a, int32_t steps, int32_t halo, int32_t tiles_i)
 {
     constexpr int kTileNodes = kTileSide * kTileSide;
@@ -60,6 +64,20 @@ __global__ __launch_bounds__(kTileSide * kTileSide) void tile_kernel(StepArgs a,
             const int32_t xi = i + kOffI[d], xj = j + kOffJ[d];  // the node this slot streams into
             if ((uint32_t)xi < (uint32_t)nr && (uint32_t)xj < (uint32_t)nc)
                 F[d * kTileNodes + pos] = ((const LBM_GLOBAL T *)a.frozen)[d * a.g.E + edge_slot(xi, xj, nr, nc)];
+        }
+    }
+    uint32_t ps_mask = 0;
+    double ps_val[9], ps_b[9];
+    if constexpr (PS) {
+        if (wet) ps_mask = ((const LBM_GLOBAL uint16_t *)a.ps_mask)[own];
+#pragma unroll
+        for (int d = 1; d < 9; ++d) {
+            ps_val[d] = ps_b[d] = 0.0;
+            if ((ps_mask >> d) & 1u) {
+                const int64_t k = (int64_t)d * a.g.plane + own;
+                ps_val[d] = ((const LBM_GLOBAL double *)a.ps_val)[k];
+                ps_b[d] = ((const LBM_GLOBAL double *)a.ps_b)[k];
+            }
         }
     }
     // perimeter node: its policy and prescribed values (prev: those of the
@@ -103,12 +121,22 @@ __global__ __launch_bounds__(kTileSide * kTileSide) void tile_kernel(StepArgs a,
         }
         if (!last) __syncthreads();
         if (act) {
+            if constexpr (PS) {
+#pragma unroll
+                for (int d = 1; d < 9; ++d)
+                    if ((ps_mask >> d) & 1u) raw[d] = ps_val[d];
+            }
             if constexpr (sizeof(T) == 8) {
                 if (policy == kVelocity) zouhe_velocity64(bt, raw, prev.ux, prev.uy);
                 else if (policy == kPressure) zouhe_pressure64(bt, raw, rho_prev);
-                T o[9];
-                if (last) collide_f64<true>(a, raw, policy, v, i, j, o);
-                else collide_f64<false>(a, raw, policy, v, i, j, o);
+                T o[9], eq[9];
+                if (last) collide_f64<true>(a, raw, policy, v, i, j, o, eq);
+                else collide_f64<false>(a, raw, policy, v, i, j, o, eq);
+                if constexpr (PS) {
+#pragma unroll
+                    for (int d = 1; d < 9; ++d)
+                        if ((ps_mask >> d) & 1u) ps_val[d] = psbb_value(a, d, ps_b[d], raw, eq, o);
+                }
 #pragma unroll
                 for (int d = 0; d < 9; ++d) raw[d] = o[d];
             } else {
@@ -132,6 +160,11 @@ __global__ __launch_bounds__(kTileSide * kTileSide) void tile_kernel(StepArgs a,
             }
             if (last) {
                 store9(a, own, raw);
+                if constexpr (PS) {
+#pragma unroll
+                    for (int d = 1; d < 9; ++d)
+                        if ((ps_mask >> d) & 1u) a.ps_next[(int64_t)d * a.g.plane + own] = ps_val[d];
+                }
             } else {
 #pragma unroll
                 for (int d = 0; d < 9; ++d) F[d * kTileNodes + pos] = raw[d];

@@ -107,3 +107,27 @@ def test_range_is_reported_from_tiles():
         lat.step(1, L.STEP_CHECK)
     assert e.value.code == L.ERR_RANGE
     lat.close()
+
+
+@pytest.mark.parametrize("nr,nc", [(24, 24), (57, 61), (129, 129), (230, 290), (400, 410)])
+def test_partially_saturated_obstacles(nr, nc):
+    """Obstacles of every weight through the tiles against single steps,
+    across calls and captured graphs."""
+    rng = np.random.default_rng(nr)
+    cls = random_class(rng, nr, nc, 0.1)
+    p0 = state(rng, nc, nr)
+    lats = [make(cls, np.random.default_rng(1), L.F64, (L.BGK, L.TRT)[nr % 2], POLICIES[:2]) for _ in range(2)]
+    nob = int(lats[0].node_counts()[6])
+    b = rng.random(nob)
+    for lat, flags in zip(lats, (0, L.STEP_NO_GRAPH)):
+        lat.set_partial_bounce_back(0.9, b)
+        lat.upload_populations(p0)
+        for n in (1, 2, 13, 97):
+            lat.step(n, flags | L.STEP_MACRO)
+    x, y = lats
+    assert np.array_equal(x.populations(), y.populations())
+    for u, v in zip(x.macro(), y.macro()):
+        assert np.array_equal(u, v)
+    assert x.lift_drag() == y.lift_drag()
+    for lat in lats:
+        lat.close()
