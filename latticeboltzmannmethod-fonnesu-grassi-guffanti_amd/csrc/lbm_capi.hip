@@ -23,6 +23,7 @@
 #include "../../include/lbm_amd.h"
 #include "lbm_context.h"
 #include "lbm_internal.h"
+#include "lbm_transfer.h"
 
 using namespace lbm;
 
@@ -540,6 +541,7 @@ int lbm_create(const lbm_desc *desc, lbm_ctx **out)
         if (r) return r;
     }
     lbm_ctx *c = new lbm_ctx();
+    transfer_retain();
     c->desc = *desc;
     c->storage = desc->storage;
     int cus = 0;
@@ -548,6 +550,7 @@ int lbm_create(const lbm_desc *desc, lbm_ctx **out)
     c->esize = desc->storage == kF64 ? 8 : desc->storage == kF32 ? 4 : 2;
     hipError_t e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
     if (e != hipSuccess) {
+        transfer_release();
         delete c;
         return fail(LBM_ERR_HIP, "hipStreamCreate: %s", hipGetErrorString(e));
     }
@@ -593,6 +596,7 @@ int lbm_destroy(lbm_ctx *c)
     if (c->copy_go) (void)hipEventDestroy(c->copy_go);
     if (c->copy_stream) (void)hipStreamDestroy(c->copy_stream);
     if (c->stream) (void)hipStreamDestroy(c->stream);
+    transfer_release();
     delete c;
     return LBM_OK;
 }
@@ -1001,8 +1005,7 @@ int lbm_upload_populations(lbm_ctx *c, const double *P)
     if (r) return r;
     if (c->state == kNone) c->scale = choose_scale(c);
     drop_graphs(c);
-    HIP_TRY(hipMemcpyAsync(c->d_staging, P, (size_t)(9 * c->nr * c->nc) * sizeof(double), hipMemcpyHostToDevice,
-                           c->stream));
+    HIP_TRY(copy_to_device(c->desc.device, c->d_staging, P, (size_t)(9 * c->nr * c->nc) * sizeof(double), c->stream));
     StepArgs a = make_args(c);
     HIP_TRY(launch_upload(c->storage, a, c->d_staging, c->d_F[c->cur], c->d_frozen, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
@@ -1021,9 +1024,7 @@ int lbm_download_populations(lbm_ctx *c, double *P)
     StepArgs a = make_args(c);
     a.fin = c->d_F[c->cur];
     HIP_TRY(launch_readout(c->storage, c->state == kFstar, a, c->d_staging, nullptr, c->stream));
-    HIP_TRY(hipMemcpyAsync(P, c->d_staging, (size_t)(9 * c->nr * c->nc) * sizeof(double), hipMemcpyDeviceToHost,
-                           c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
+    HIP_TRY(copy_to_host(c->desc.device, P, c->d_staging, (size_t)(9 * c->nr * c->nc) * sizeof(double), c->stream));
     return LBM_OK;
 }
 
@@ -1037,9 +1038,7 @@ int lbm_download_after_collision(lbm_ctx *c, double *P)
     StepArgs a = make_args(c);
     a.fin = c->d_F[c->cur];
     HIP_TRY(launch_readout(c->storage, false, a, c->d_staging, nullptr, c->stream));
-    HIP_TRY(hipMemcpyAsync(P, c->d_staging, (size_t)(9 * c->nr * c->nc) * sizeof(double), hipMemcpyDeviceToHost,
-                           c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
+    HIP_TRY(copy_to_host(c->desc.device, P, c->d_staging, (size_t)(9 * c->nr * c->nc) * sizeof(double), c->stream));
     return LBM_OK;
 }
 
@@ -1269,8 +1268,8 @@ int lbm_download_macro(lbm_ctx *c, double *rho, double *u)
     HIP_TRY(hipSetDevice(c->desc.device));
     size_t N = (size_t)(c->nr * c->nc);
     const double *m = c->d_macro[c->macro_slot];
-    if (rho) HIP_TRY(hipMemcpyAsync(rho, m, N * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    if (u) HIP_TRY(hipMemcpyAsync(u, m + N, 2 * N * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    if (rho) HIP_TRY(copy_to_host(c->desc.device, rho, m, N * sizeof(double), c->stream));
+    if (u) HIP_TRY(copy_to_host(c->desc.device, u, m + N, 2 * N * sizeof(double), c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
     return LBM_OK;
 }

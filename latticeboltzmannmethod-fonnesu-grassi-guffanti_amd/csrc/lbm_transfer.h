@@ -1,0 +1,22 @@
+// Large copies between device memory and a caller's ordinary (pageable)
+// host memory.  Internal.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstddef>
+
+namespace lbm {
+
+// Copies `bytes` on stream s and waits for them: what hipMemcpyAsync and
+// hipStreamSynchronize do, and done by these for small copies and for
+// page-locked host memory.  `device` is the stream's.
+hipError_t copy_to_host(int device, void *dst, const void *src, size_t bytes, hipStream_t s);
+hipError_t copy_to_device(int device, void *dst, const void *src, size_t bytes, hipStream_t s);
+
+// Contexts alive: the page-locked chunks the copies go through are shared by
+// all of them and freed with the last one.
+void transfer_retain();
+void transfer_release();
+
+}  // namespace lbm
