@@ -387,6 +387,8 @@ int lbm_batch_create(lbm_ctx *const *samples, int64_t n, lbm_batch **out)
     if (!r) r = build_runs(b);
     if (!r) r = build_marches(b);
     if (r) return bail(r);
+    for (lbm_ctx *c : b->samples)
+        if ((r = flush_bc(c))) return bail(r);
     for (lbm_ctx *c : b->samples) c->batch = b;
     *out = b;
     return LBM_OK;

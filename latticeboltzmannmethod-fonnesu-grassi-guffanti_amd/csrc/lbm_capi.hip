@@ -109,6 +109,15 @@ StepArgs make_args(const lbm_ctx *c)
     return a;
 }
 
+int flush_bc(lbm_ctx *c)
+{
+    if (!c->bc_pending) return LBM_OK;
+    HIP_TRY(hipMemcpyAsync(c->d_bc[c->bc_cur], c->h_bc_pin + (size_t)c->bc_slot * c->h_bc.size(),
+                           c->h_bc.size() * sizeof(double), hipMemcpyHostToDevice, c->stream));
+    c->bc_pending = false;
+    return LBM_OK;
+}
+
 }  // namespace lbm
 
 namespace {
@@ -152,6 +161,10 @@ hipError_t launch_steps(const lbm_ctx *c, Launching::Kind kind, int in, int32_t 
     StepArgs a = make_args(c);
     set_input(c, a, in);
     a.macro = macro;
+    if (c->bc_pending) {  // the launch reads the waiting values and leaves them in the device copy
+        a.bc_cur = c->h_bc_pin + (size_t)c->bc_slot * c->h_bc.size();
+        a.bc_new = c->d_bc[c->bc_cur];
+    }
     switch (kind) {
     case Launching::kTile: return launch_tile(c->storage, k, a, c->stream);
     case Launching::kMarch: return launch_march(c->storage, k, a, c->stream);
@@ -204,9 +217,10 @@ void free_geometry(lbm_ctx *c)
     for (int k = 0; k < 2; ++k) {
         (void)hipFree(c->d_F[k]); c->d_F[k] = nullptr;
         (void)hipFree(c->d_bc[k]); c->d_bc[k] = nullptr;
-        if (c->h_bc_pin[k]) (void)hipHostFree(c->h_bc_pin[k]);
-        c->h_bc_pin[k] = nullptr;
     }
+    if (c->h_bc_pin) (void)hipHostFree(c->h_bc_pin);
+    c->h_bc_pin = nullptr;
+    c->bc_pending = false;
     for (int k = 0; k < 2; ++k) {
         (void)hipFree(c->d_macro[k]);
         c->d_macro[k] = nullptr;
@@ -241,20 +255,31 @@ int ensure_staging(lbm_ctx *c)
     return LBM_OK;
 }
 
-// Pushes the host values h_bc into the device copy the next step reads as
-// "current".  The copy that the last step read as "current" becomes
-// "previous" and stays untouched.
+// Slots of at most this many bytes are left for the step to read: a copy
+// into device memory between two kernels costs 10 us, the step's own reads
+// over the link 2 us.  Larger ones are copied at once.
+constexpr size_t kPendingBytes = 65536;
+constexpr int kPendingSlots = 8;
+
+// Makes the host values h_bc the ones the next step reads as "current".
+// The copy that the last step read as "current" becomes "previous" and
+// stays untouched.
 int push_bc(lbm_ctx *c)
 {
     if (c->bc_cur == c->bc_prev) c->bc_cur = 1 - c->bc_prev;
-    int k = c->bc_cur;
-    // The pinned staging copy k may still be in flight from an earlier push.
-    HIP_TRY(hipEventSynchronize(c->bc_ev[k]));
-    std::memcpy(c->h_bc_pin[k], c->h_bc.data(), c->h_bc.size() * sizeof(double));
-    HIP_TRY(hipMemcpyAsync(c->d_bc[k], c->h_bc_pin[k], c->h_bc.size() * sizeof(double), hipMemcpyHostToDevice,
-                           c->stream));
-    HIP_TRY(hipEventRecord(c->bc_ev[k], c->stream));
-    return LBM_OK;
+    // The next slot's last reader may still be in flight: each half of the
+    // slots has an event behind everything queued while it was in use.
+    const int half = c->bc_slots / 2, slot = (c->bc_slot + 1) % c->bc_slots;
+    if (slot % half == 0) {
+        const int h = slot / half;
+        HIP_TRY(hipEventRecord(c->bc_ev[1 - h], c->stream));
+        HIP_TRY(hipEventSynchronize(c->bc_ev[h]));
+    }
+    c->bc_slot = slot;
+    std::memcpy(c->h_bc_pin + (size_t)slot * c->h_bc.size(), c->h_bc.data(), c->h_bc.size() * sizeof(double));
+    c->bc_pending = true;
+    // an ensemble's kernels and large lattices read the device copy
+    return c->batch || c->bc_slots == 2 ? flush_bc(c) : LBM_OK;
 }
 
 // Storage scale of the FP16 path: a power of two that puts the largest
@@ -909,9 +934,11 @@ int lbm_set_geometry(lbm_ctx *c, const uint8_t *cls)
         HIP_TRY(hipMalloc(&c->d_F[k], fbytes));
         HIP_TRY(hipMemset(c->d_F[k], 0, fbytes));
         HIP_TRY(hipMalloc(&c->d_bc[k], (size_t)(3 * c->E) * sizeof(double)));
-        HIP_TRY(hipHostMalloc((void **)&c->h_bc_pin[k], (size_t)(3 * c->E) * sizeof(double), hipHostMallocDefault));
         HIP_TRY(hipMemcpy(c->d_bc[k], c->h_bc.data(), (size_t)(3 * c->E) * sizeof(double), hipMemcpyHostToDevice));
     }
+    c->bc_slots = (size_t)(3 * c->E) * sizeof(double) <= kPendingBytes ? kPendingSlots : 2;
+    HIP_TRY(hipHostMalloc((void **)&c->h_bc_pin, (size_t)(c->bc_slots * 3 * c->E) * sizeof(double), hipHostMallocDefault));
+    c->bc_slot = 0;
     c->bc_cur = c->bc_prev = 0;
     // both copies of the fields start at rho = 1, u = 0 (Lattice.hpp:295-296):
     // the steps write the wet nodes only
@@ -1085,6 +1112,7 @@ int lbm_step(lbm_ctx *c, int64_t n, uint32_t flags)
             }
             if (k > 0) {
                 HIP_TRY(launch_steps(c, how.kind, c->cur, k, fields));
+                c->bc_pending = false;
                 c->cur = 1 - c->cur;
                 c->bc_prev = c->bc_cur;
                 c->t += k;
@@ -1092,6 +1120,7 @@ int lbm_step(lbm_ctx *c, int64_t n, uint32_t flags)
                 continue;
             }
         }
+        if (int r = flush_bc(c)) return r;
         StepArgs a = make_args(c);
         if (macro && s == n - 1) {
             int r = claim_macro(c, &a.macro);
@@ -1189,6 +1218,7 @@ int lbm_autotune(lbm_ctx *c, int32_t steps, int32_t *segments, double *ms_per_st
         const int r = ensure_run_tables(c);
         if (r) return r;
     }
+    if (const int r = flush_bc(c)) return r;
     hipEvent_t t0 = nullptr, t1 = nullptr;
     HIP_TRY(hipEventCreate(&t0));
     hipError_t err = hipEventCreate(&t1);

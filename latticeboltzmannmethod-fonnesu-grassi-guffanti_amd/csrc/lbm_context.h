@@ -59,10 +59,14 @@ struct lbm_ctx {
     void *d_F[2] = {nullptr, nullptr};
     int cur = 0;
     // prescribed values: two device copies [3][E]; `bc_prev` is the one the
-    // last step used as "current", `bc_cur` the one the next step uses.
+    // last step used as "current", `bc_cur` the one the next step uses.  New
+    // values wait in a page-locked slot (bc_pending) until the step that
+    // uses them reads them there, or a copy brings them to the device.
     double *d_bc[2] = {nullptr, nullptr};
-    double *h_bc_pin[2] = {nullptr, nullptr};
-    hipEvent_t bc_ev[2] = {nullptr, nullptr};
+    double *h_bc_pin = nullptr;  // bc_slots slots of [3][E], used in turn
+    int bc_slots = 0, bc_slot = 0;
+    bool bc_pending = false;
+    hipEvent_t bc_ev[2] = {nullptr, nullptr};  // last reader of each half of the slots
     int bc_cur = 0, bc_prev = 0;
     std::vector<double> h_bc;  // [3][E] latest values
     // rho/u fields of LBM_STEP_MACRO steps: two device copies, written in
@@ -131,5 +135,8 @@ namespace lbm {
 // Step arguments of a context (geometry, prescribed values, relaxation,
 // storage scale); the caller sets fin/fout/macro.
 StepArgs make_args(const lbm_ctx *c);
+
+// Queues the copy of prescribed values that are still waiting for their step.
+int flush_bc(lbm_ctx *c);
 
 }  // namespace lbm

@@ -67,6 +67,7 @@ struct StepArgs {
     const void *frozen;   // [9][E] populations with out-of-domain source, storage type
     const double *bc_prev;  // [3][E]: ux, uy, rho prescribed at the previous step
     const double *bc_cur;   // [3][E]: values prescribed at this step
+    double *bc_new;         // tiles: where bc_cur is page-locked host memory, the device copy to fill from it
     int32_t inlet_policy, outlet_policy;
     int32_t collision;      // 0 BGK, 1 TRT
     int32_t segs;           // row segments (of kBlockRows) per column
@@ -226,8 +227,8 @@ int32_t march_steps(int32_t storage, const StepArgs &a);
 hipError_t launch_march(int32_t storage, int32_t steps, const StepArgs &a, hipStream_t s);
 // Steps per launch of the tile kernel for this lattice (0: not for it), and
 // such a launch of 1 .. tile_steps steps from fin (F*) to fout.  The first
-// gather is closed with bc_prev, everything after takes bc_cur; a.macro is
-// written by the last step.
+// gather is closed with bc_prev, everything after takes bc_cur (in host
+// memory: copied to a.bc_new); a.macro is written by the last step.
 int32_t tile_steps(int32_t storage, const StepArgs &a);
 hipError_t launch_tile(int32_t storage, int32_t steps, const StepArgs &a, hipStream_t s);
 int64_t readout_blocks(const StepArgs &a);

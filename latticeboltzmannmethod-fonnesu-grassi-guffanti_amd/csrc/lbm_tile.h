@@ -8,7 +8,9 @@
 // ring of the region, so the work-group stores the (S - 2 halo)^2 nodes in
 // the middle.  Perimeter nodes (frozen slots, Zou-He, prescribed
 // velocities), new prescribed values and the macro fields are handled here
-// too, so one launch does all a lattice needs.
+// too, so one launch does all a lattice needs.  New prescribed values are
+// read from the page-locked memory they wait in, and kept in the device copy
+// for the steps after (bc_new).
 //
 // Slots whose source lies outside the domain keep their value (the
 // reference never writes them): the region's positions just outside the
@@ -95,6 +97,12 @@ __global__ __launch_bounds__(kTileSide * kTileSide) void tile_kernel(StepArgs a,
         rho = bc[2 * a.g.E];
         prev = {bp[0], bp[a.g.E]};
         rho_prev = bp[2 * a.g.E];
+        if (a.bc_new && depth >= halo) {  // this tile stores the node: it also keeps its new values
+            LBM_GLOBAL double *bn = (LBM_GLOBAL double *)a.bc_new + e;
+            bn[0] = v.ux;
+            bn[a.g.E] = v.uy;
+            bn[2 * a.g.E] = rho;
+        }
         if (k != kEdgePlain) policy = k == kEdgeInlet ? a.inlet_policy : a.outlet_policy;
         bt = edge_btype(i, j, nr, nc);
     }

@@ -131,3 +131,33 @@ def test_partially_saturated_obstacles(nr, nc):
     assert x.lift_drag() == y.lift_drag()
     for lat in lats:
         lat.close()
+
+
+@pytest.mark.parametrize("storage", [L.F64, L.F16_SHIFTED])
+@pytest.mark.parametrize("nr,nc", [(40, 96), (300, 700)])
+def test_new_values_every_step(nr, nc, storage):
+    """More new values in flight than the waiting slots hold, values that are
+    replaced before any step reads them, and steps that take them together
+    with older ones; against single steps that wait for every value."""
+    rng = np.random.default_rng(nc)
+    cls = random_class(rng, nr, nc, 0.1)
+    p0 = state(rng, nc, nr)
+    lats = [make(cls, np.random.default_rng(4), storage, L.BGK, (L.ZOUHE_VELOCITY, L.ZOUHE_PRESSURE))
+            for _ in range(2)]
+    n0, n1 = (len(lats[0].open_nodes(k)) for k in (0, 1))
+    values = rng.uniform(-0.02, 0.02, (60, 3))
+    for lat in lats:
+        lat.upload_populations(p0)
+    for k, (x, y, r) in enumerate(values):
+        for lat, flags in zip(lats, (0, L.STEP_NO_GRAPH)):
+            if k % 7 == 3:
+                lat.set_open_values(0, ux=np.full(n0, 9.0 * x))    # replaced below
+            lat.set_open_values(0, ux=np.full(n0, x), uy=np.full(n0, y))
+            if k % 3 == 0:
+                lat.set_open_values(1, rho=np.full(n1, 1.0 + r / 4))
+            lat.step(1 + (k % 5) * (k % 2), flags)
+            if flags:
+                lat.synchronize()
+    assert np.array_equal(lats[0].populations(), lats[1].populations())
+    for lat in lats:
+        lat.close()
