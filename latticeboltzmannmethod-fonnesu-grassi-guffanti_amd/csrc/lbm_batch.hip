@@ -69,6 +69,7 @@ struct lbm_batch {
     int32_t *d_marches = nullptr;
     int64_t nmarches = 0;
     bool march = false;
+    bool fused = false;
     // "first" = each sample's arguments as lbm_step would build them for its
     // next step; "steady" = the same with the previous prescribed values set
     // to the current ones (every step after the first of a run)
@@ -244,6 +245,7 @@ int build_marches(lbm_batch *b)
     HIP_TRY(hipMalloc(&b->d_marches, table.size() * sizeof(int32_t)));
     HIP_TRY(hipMemcpy(b->d_marches, table.data(), table.size() * sizeof(int32_t), hipMemcpyHostToDevice));
     b->march = true;
+    b->fused = nodes >= kBatchFusedNodes;
     return LBM_OK;
 }
 
@@ -296,6 +298,7 @@ BatchArgs batch_args(const lbm_batch *b, const ArgBuffer &ab, int parity)
     a.nruns = b->nruns;
     a.marches = b->d_marches;
     a.nmarches = b->nmarches;
+    a.fused = b->fused;
     return a;
 }
 

@@ -168,6 +168,7 @@ struct BatchArgs {
     // row of the window, columns [j0, j1) (sign bit of j1: perimeter window)
     const int32_t *marches;
     int64_t nmarches;
+    int32_t fused;  // enough nodes to keep the SIMDs full (march_kernel)
 };
 
 // Steps per launch of an ensemble's marching waves, their table over chunks
@@ -219,7 +220,7 @@ hipError_t launch_reduce_partials(double *partials, int64_t nblocks, int32_t nco
 // lattices from there on marching waves; ensembles take marching waves from
 // kMarchMinNodes nodes in all.
 constexpr int64_t kTileMaxNodes = 300000, kTileMaxNodesF16 = (int64_t)1 << 19;
-constexpr int64_t kMarchMinNodes = (int64_t)1 << 17;
+constexpr int64_t kMarchMinNodes = (int64_t)1 << 17, kBatchFusedNodes = (int64_t)1 << 20;
 // Steps per launch of the marching kernel for this lattice (0: not for it),
 // and such a launch: `steps` steps (2 .. march_steps) without new prescribed
 // values from fin (F*) to fout, blocked layout.

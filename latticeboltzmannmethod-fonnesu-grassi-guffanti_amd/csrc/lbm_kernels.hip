@@ -1618,7 +1618,7 @@ __global__ __launch_bounds__(kBlockRows) void batch_perimeter_kernel(BatchArgs b
 // step a launch (R = 1 tiles) -> several: 32 porous lattices of up to
 // 1024^2 FP32 107.9 -> 49.6, FP64 193 -> 82; 150 of them FP32 488 -> 225;
 // 8 of up to 256^2 FP32 15.2 -> 6.5.
-template <typename T, int K>
+template <typename T, int K, bool FUSED>
 __global__ __launch_bounds__(kBlockRows) void batch_march_kernel(BatchArgs bt)
 {
     asm volatile("" ::"s"(bt.nmarches), "s"(bt.marches), "s"(bt.args), "s"(bt.parity));  // one round trip
@@ -1633,8 +1633,8 @@ __global__ __launch_bounds__(kBlockRows) void batch_march_kernel(BatchArgs bt)
     const int j0 = __builtin_amdgcn_readfirstlane(e[2]);
     const int j1 = __builtin_amdgcn_readfirstlane(e[3]);
     const StepArgs a = args_at(bt, s);
-    if (j1 < 0) march_wave<T, K, true>(a, i0, j0, j1 & 0x7fffffff, lane);
-    else march_wave<T, K, false>(a, i0, j0, j1, lane);
+    if (j1 < 0) march_wave<T, K, FUSED, true>(a, i0, j0, j1 & 0x7fffffff, lane);
+    else march_wave<T, K, FUSED, false>(a, i0, j0, j1, lane);
 }
 
 // The time-step kernel of a batch of independent lattices: a persistent
@@ -2067,6 +2067,9 @@ MarchPlan march_plan(const StepArgs &a)
     return m;
 }
 
+// Lattices whose waves keep the SIMDs full.
+bool march_large(const StepArgs &a) { return (int64_t)a.g.nr * a.g.nc >= (int64_t)1 << 22; }
+
 template <typename T, int K>
 hipError_t launch_march_t(StepArgs a, hipStream_t s)
 {
@@ -2074,7 +2077,15 @@ hipError_t launch_march_t(StepArgs a, hipStream_t s)
     const int64_t inner = m.stripes - m.top - m.bottom;
     const int64_t chunks = inner > 0 ? (a.g.nc - 2 * (K + 1) + m.cols - 1) / m.cols : 0;
     a.nblocks = (m.edge_waves + inner * chunks + kBlockRows / 64 - 1) / (kBlockRows / 64);
-    hipLaunchKernelGGL((march_kernel<T, K>), dim3((unsigned)a.nblocks), dim3(kBlockRows), 0, s, a, m);
+    const dim3 grid((unsigned)a.nblocks), block(kBlockRows);
+    if constexpr (K == 5) {  // large lattices only
+        hipLaunchKernelGGL((march_kernel<T, K, true>), grid, block, 0, s, a, m);
+    } else if constexpr (K == 4) {
+        if (march_large(a)) hipLaunchKernelGGL((march_kernel<T, K, true>), grid, block, 0, s, a, m);
+        else hipLaunchKernelGGL((march_kernel<T, K, false>), grid, block, 0, s, a, m);
+    } else {
+        hipLaunchKernelGGL((march_kernel<T, K, false>), grid, block, 0, s, a, m);
+    }
     return hipGetLastError();
 }
 
@@ -2117,7 +2128,9 @@ template <typename T>
 hipError_t launch_batch_march_t(const BatchArgs &b, hipStream_t s)
 {
     const int64_t nb = (b.nmarches + kBlockRows / 64 - 1) / (kBlockRows / 64);
-    hipLaunchKernelGGL((batch_march_kernel<T, kBatchMarchSteps>), dim3((unsigned)nb), dim3(kBlockRows), 0, s, b);
+    const dim3 grid((unsigned)nb), block(kBlockRows);
+    if (b.fused) hipLaunchKernelGGL((batch_march_kernel<T, kBatchMarchSteps, true>), grid, block, 0, s, b);
+    else hipLaunchKernelGGL((batch_march_kernel<T, kBatchMarchSteps, false>), grid, block, 0, s, b);
     return hipGetLastError();
 }
 
@@ -2257,7 +2270,7 @@ int32_t march_steps(int32_t storage, const StepArgs &a)
 {
     const int64_t nodes = (int64_t)a.g.nr * a.g.nc;
     if (storage == kF16 || a.psbb || !a.block_mask || nodes < kTileMaxNodes) return 0;
-    return storage == kF64 && nodes >= (int64_t)1 << 22 ? 5 : 4;
+    return storage == kF64 && march_large(a) ? 5 : 4;
 }
 
 hipError_t launch_march(int32_t storage, int32_t steps, const StepArgs &a, hipStream_t s)

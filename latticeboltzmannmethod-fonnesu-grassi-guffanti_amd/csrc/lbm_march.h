@@ -22,14 +22,14 @@
 // perimeter nodes (EDGE); the prescribed values are those of the current
 // step throughout, so the launch is for steps without new values.
 //
-// What bounds it: in FP32 the VALU (138 instructions per level and lane of
-// 124 that the collision and the streaming need), in FP64 latency (two
-// waves per SIMD, VALU busy 0.65; nine values per level stay in
+// What bounds it: in FP32 the VALU (busy throughout; 122 instructions per
+// level and lane, of which the collision takes 110), in FP64 the VALU at 0.8
+// and latency (two waves per SIMD: nine values per level stay in
 // registers).  us a step, before (one step a launch, tuned) -> K = 4 (FP32),
-// 5 (FP64): porous 8192^2 FP32 561 -> 271, FP64 1159 -> 454; open 4096^2
-// FP64 419 -> 125; TRT cavity 4096^2 FP32 194 -> 80, FP64 416 -> 163.
-// K = 2 / 3 / 4 / 5 on the porous 4096^2: FP64 211 / 146 / 119 / 114, FP32
-// 121 / 78 / 71 / 74: the launch stays near 550 us (FP64) up to K = 4, where
+// 5 (FP64): porous 8192^2 FP32 561 -> 254; open 4096^2 FP64 419 -> 121; TRT
+// cavity 4096^2 FP32 194 -> 78, FP64 416 -> 157; porous 4096^2 FP64 303 -> 112.
+// K = 2 / 3 / 4 / 5 on the porous 4096^2 (before FUSED): FP64 211 / 146 / 119
+// / 114, FP32 121 / 78 / 71 / 74: the launch stays near 550 us (FP64) up to K = 4, where
 // memory binds it, and the lanes and columns lost to the window's ends
 // outweigh the traffic beyond.  FP16 keeps one step a launch: its rounding
 // takes another 50 instructions per node, and it was at the VALU limit with
@@ -99,10 +99,79 @@ __device__ __forceinline__ T lane_shift(T v)
     }
 }
 
-template <typename T>
-__device__ __forceinline__ T from_below(T v) { return lane_shift<0x130>(v); }  // wave_shl:1 -- lane l + 1
-template <typename T>
-__device__ __forceinline__ T from_above(T v) { return lane_shift<0x138>(v); }  // wave_shr:1 -- lane l - 1
+// A move from the neighbouring lane and the choice against y in one
+// instruction: lanes of m take the neighbour's x (the lane below's or
+// above's), the others y.  v_cndmask has a DPP form only with its condition
+// in VCC and picks its moved operand where the bit is clear, which the
+// compiler does not form from a mask in other scalar registers; keep: the
+// complement of m.  s_mov leaves SCC alone.  A DPP read must stay two wait
+// states behind the write of its register (s_mov, s_nop).
+#define LBM_BELOW "wave_shl:1 row_mask:0xf bank_mask:0xf bound_ctrl:0"
+#define LBM_ABOVE "wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:0"
+#define LBM_MOVED(DIR)                                                                                         \
+    asm("s_mov_b64 vcc, %6\n\ts_nop 0\n\tv_cndmask_b32_dpp %0, %2, %4, vcc " DIR                              \
+        "\n\tv_cndmask_b32_dpp %1, %3, %5, vcc " DIR                                                            \
+        : "=&v"(r0), "=&v"(r1)                                                                                 \
+        : "v"(x0), "v"(x1), "v"(y0), "v"(y1), "s"(keep)                                                        \
+        : "vcc")
+
+template <bool BELOW>
+__device__ __forceinline__ void moved2(uint64_t keep, uint32_t x0, uint32_t y0, uint32_t x1, uint32_t y1, uint32_t &r0,
+                                       uint32_t &r1)
+{
+    if constexpr (BELOW) LBM_MOVED(LBM_BELOW);
+    else LBM_MOVED(LBM_ABOVE);
+}
+
+template <bool BELOW>
+__device__ __forceinline__ uint32_t moved1(uint64_t keep, uint32_t x, uint32_t y)
+{
+    uint32_t r;
+    if constexpr (BELOW)
+        asm("s_mov_b64 vcc, %3\n\ts_nop 0\n\tv_cndmask_b32_dpp %0, %1, %2, vcc " LBM_BELOW
+            : "=v"(r)
+            : "v"(x), "v"(y), "s"(keep)
+            : "vcc");
+    else
+        asm("s_mov_b64 vcc, %3\n\ts_nop 0\n\tv_cndmask_b32_dpp %0, %1, %2, vcc " LBM_ABOVE
+            : "=v"(r)
+            : "v"(x), "v"(y), "s"(keep)
+            : "vcc");
+    return r;
+}
+
+// FUSED: the form above; otherwise a move and a choice.
+template <bool BELOW, bool FUSED, typename T>
+__device__ __forceinline__ T moved(uint64_t m, T x, T y)
+{
+    if constexpr (!FUSED) {
+        const T z = lane_shift<BELOW ? 0x130 : 0x138>(x);  // wave_shl:1 (lane l + 1), wave_shr:1 (lane l - 1)
+        return __builtin_amdgcn_inverse_ballot_w64(m) ? z : y;
+    } else if constexpr (sizeof(T) == 8) {
+        const uint2 a = __builtin_bit_cast(uint2, x), b = __builtin_bit_cast(uint2, y);
+        uint2 r;
+        moved2<BELOW>(~m, a.x, b.x, a.y, b.y, r.x, r.y);
+        return __builtin_bit_cast(T, r);
+    } else {
+        return __builtin_bit_cast(T, moved1<BELOW>(~m, __builtin_bit_cast(uint32_t, x), __builtin_bit_cast(uint32_t, y)));
+    }
+}
+
+// Two values under one mask (FP32: one asm for both).
+template <bool BELOW, bool FUSED, typename T>
+__device__ __forceinline__ void moved_pair(uint64_t m, T x0, T y0, T x1, T y1, T &r0, T &r1)
+{
+    if constexpr (FUSED && sizeof(T) == 4) {
+        uint32_t u0, u1;
+        moved2<BELOW>(~m, __builtin_bit_cast(uint32_t, x0), __builtin_bit_cast(uint32_t, y0),
+                      __builtin_bit_cast(uint32_t, x1), __builtin_bit_cast(uint32_t, y1), u0, u1);
+        r0 = __builtin_bit_cast(T, u0);
+        r1 = __builtin_bit_cast(T, u1);
+    } else {
+        r0 = moved<BELOW, FUSED>(m, x0, y0);
+        r1 = moved<BELOW, FUSED>(m, x1, y1);
+    }
+}
 
 // What one level of a marching wave keeps of the last column it was fed:
 // the six pre-collision populations that are complete, and the three
@@ -117,7 +186,7 @@ struct Level {
 // Streams column c's post-collision populations o into a level that holds
 // column c - 1: p receives the complete pre-collision populations of column
 // c - 1.  wc, wp: the windows of columns c and c - 1.
-template <typename T>
+template <bool FUSED, typename T>
 __device__ __forceinline__ void feed(Level<T> &s, const T *o, const Win &wc, const Win &wp, T *p)
 {
     auto sel = [](uint64_t m, T x, T y) { return __builtin_amdgcn_inverse_ballot_w64(m) ? x : y; };
@@ -128,14 +197,12 @@ __device__ __forceinline__ void feed(Level<T> &s, const T *o, const Win &wc, con
     p[5] = s.p5;
     p[8] = s.p8;
     p[3] = sel(wc.mid, o[3], s.e1);
-    p[6] = sel(wc.dn, from_below(o[6]), s.e8);
-    p[7] = sel(wc.up, from_above(o[7]), s.e5);
     s.p0 = o[0];
     s.p1 = sel(wp.mid, s.e1, o[3]);
-    s.p5 = sel(wp.dn, from_below(s.e5), o[7]);
-    s.p8 = sel(wp.up, from_above(s.e8), o[6]);
-    s.p2 = sel(wc.dn, from_below(o[2]), o[4]);
-    s.p4 = sel(wc.up, from_above(o[4]), o[2]);
+    s.p5 = moved<true, FUSED>(wp.dn, s.e5, o[7]);
+    s.p8 = moved<false, FUSED>(wp.up, s.e8, o[6]);
+    moved_pair<true, FUSED>(wc.dn, o[6], s.e8, o[2], o[4], p[6], s.p2);
+    moved_pair<false, FUSED>(wc.up, o[7], s.e5, o[4], o[2], p[7], s.p4);
     s.e1 = o[1];
     s.e5 = o[5];
     s.e8 = o[8];
@@ -247,7 +314,7 @@ __device__ __forceinline__ bool march_collide(const StepArgs &a, T *p, const Win
     else return collide_shifted<false, false>(a, p, policy, v, 0, j, o);
 }
 
-template <typename T, int K, bool EDGE>
+template <typename T, int K, bool FUSED, bool EDGE>
 __device__ __forceinline__ void march_wave(const StepArgs &a, int32_t i0, int32_t j0, int32_t j1, int lane)
 {
     constexpr uint64_t kOut = ((1ull << (64 - 2 * K)) - 1ull) << K;  // lanes whose rows this wave owns
@@ -272,7 +339,7 @@ __device__ __forceinline__ void march_wave(const StepArgs &a, int32_t i0, int32_
         for (int q = K + 1; q > 0; --q) w[q] = w[q - 1];
         w[0] = window(nw, i0);
         nw = load_words(a.g, EDGE ? min(c + 2, nc) : c + 2, i0);
-        feed(lv[0], raw, w[1], w[2], p);
+        feed<FUSED>(lv[0], raw, w[1], w[2], p);
         win_load(a, w[0], raw);
 #pragma unroll
         for (int q = 1; q <= K; ++q) {
@@ -282,7 +349,7 @@ __device__ __forceinline__ void march_wave(const StepArgs &a, int32_t i0, int32_
             bool nan = false;
             if (!EDGE || j < nc) nan = march_collide<T, EDGE>(a, p, w[q + 1], i0, j, lane, o);
             if (q < K) {
-                feed(lv[q], o, w[q + 1], w[q + 2 <= K + 1 ? q + 2 : K + 1], p);
+                feed<FUSED>(lv[q], o, w[q + 1], w[q + 2 <= K + 1 ? q + 2 : K + 1], p);
             } else {
                 const uint64_t m = j < j1 ? w[K + 1].mid & kOut : 0ull;
                 bad |= nan && __builtin_amdgcn_inverse_ballot_w64(m);
@@ -295,6 +362,13 @@ __device__ __forceinline__ void march_wave(const StepArgs &a, int32_t i0, int32_
     for (; c < j0 + K; ++c) column(c, std::false_type{});
     if (!EDGE) {
         arrived(raw);
+        if constexpr (FUSED) {
+#pragma unroll 1
+            for (; c < last; c += 2) {
+                column(c, std::true_type{});
+                column(c + 1, std::true_type{});
+            }
+        }
 #pragma unroll 1
         for (; c <= last; ++c) column(c, std::true_type{});
     } else {
@@ -304,8 +378,14 @@ __device__ __forceinline__ void march_wave(const StepArgs &a, int32_t i0, int32_
     if (bad) atomicOr(a.flag, 1);
 }
 
-// K steps.
-template <typename T, int K>
+// K steps.  FUSED: for lattices that keep the SIMDs full, two columns per
+// turn of the loop and the moves of feed() in fewer instructions.  Where a
+// wave waits on its own chain instead, the fused moves' waits cost more than
+// the instructions they save.  us a step, plain -> fused: porous 4096^2 FP64
+// 116.5 -> 112.0, FP32 69.3 -> 67.5; open 3001 x 5003 FP64 111.7 -> 106.9;
+// porous 8192^2 FP32 261.5 -> 253.8; an ensemble of 60 lattices of up to 256^2
+// FP64 31.2 -> 28.7, of 8 of them FP32 6.6 -> 7.0.
+template <typename T, int K, bool FUSED>
 __global__ __launch_bounds__(kBlockRows) void march_kernel(StepArgs a, MarchPlan m)
 {
     constexpr int32_t kRows = 64 - 2 * K;
@@ -330,7 +410,7 @@ __global__ __launch_bounds__(kBlockRows) void march_kernel(StepArgs a, MarchPlan
             j0 = right ? nc - (K + 1) : 0;
             j1 = right ? nc : K + 1;
         }
-        march_wave<T, K, true>(a, stripe * kRows - K, j0, j1, lane);
+        march_wave<T, K, FUSED, true>(a, stripe * kRows - K, j0, j1, lane);
         return;
     }
     t -= m.edge_waves;
@@ -338,6 +418,6 @@ __global__ __launch_bounds__(kBlockRows) void march_kernel(StepArgs a, MarchPlan
     const int32_t j0 = K + 1 + chunk * m.cols;
     const int32_t end = nc - (K + 1);
     if (j0 >= end) return;
-    march_wave<T, K, false>(a, (m.top + t - chunk * inner) * kRows - K, j0, min(j0 + m.cols, end), lane);
+    march_wave<T, K, FUSED, false>(a, (m.top + t - chunk * inner) * kRows - K, j0, min(j0 + m.cols, end), lane);
 }
 

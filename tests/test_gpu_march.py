@@ -120,11 +120,12 @@ def test_nan_is_reported(storage):
     lat.close()
 
 
+@pytest.mark.parametrize("big", [[], [(900, 1300)]])
 @pytest.mark.parametrize("storage", [L.F64, L.F32_SHIFTED])
-def test_ensemble_same_bits_as_single_steps(storage):
+def test_ensemble_same_bits_as_single_steps(storage, big):
     """Samples of every small size beside larger ones, all kinds of
     perimeter: the ensemble's marching launches against its single steps."""
-    shapes = [(3, 3), (5, 9), (57, 10), (56, 11), (64, 12), (113, 40), (300, 200), (129, 700)]
+    shapes = [(3, 3), (5, 9), (57, 10), (56, 11), (64, 12), (113, 40), (300, 200), (129, 700)] + big
     rng = np.random.default_rng(17)
     classes = [random_class(rng, nr, nc, 0.15) for nr, nc in shapes]
     states = [state(rng, nc, nr) for nr, nc in shapes]
