@@ -219,7 +219,7 @@ hipError_t launch_reduce_partials(double *partials, int64_t nblocks, int32_t nco
 // Lattices below these node counts take tiles (tile_steps), FP64 and FP32
 // lattices from there on marching waves; ensembles take marching waves from
 // kMarchMinNodes nodes in all.
-constexpr int64_t kTileMaxNodes = 300000, kTileMaxNodesF16 = (int64_t)1 << 19;
+constexpr int64_t kTileMaxNodes = 300000, kTileMaxNodesF16 = (int64_t)3 << 19;
 constexpr int64_t kMarchMinNodes = (int64_t)1 << 17, kBatchFusedNodes = (int64_t)1 << 20;
 // Steps per launch of the marching kernel for this lattice (0: not for it),
 // and such a launch: `steps` steps (2 .. march_steps) without new prescribed

@@ -2289,52 +2289,56 @@ hipError_t launch_march(int32_t storage, int32_t steps, const StepArgs &a, hipSt
 namespace {
 
 struct TileShape {
-    int32_t side, halo;  // halo 0: no tiles for this lattice
+    int32_t rows, cols, halo;  // halo 0: no tiles for this lattice
 };
 
 int64_t tiles_of(const StepArgs &a, TileShape t)
 {
-    const int64_t n = t.side - 2 * t.halo;
-    return ((a.g.nr + n - 1) / n) * ((a.g.nc + n - 1) / n);
+    const int64_t r = t.rows - 2 * t.halo, c = t.cols - 2 * t.halo;
+    return ((a.g.nr + r - 1) / r) * ((a.g.nc + c - 1) / c);
 }
 
 // As many steps a launch as leave one tile per CU: more steps share a
-// launch's fixed cost, and a second tile on a CU costs what it saves.  The
-// 24 x 24 region steps faster (1.3 us against 1.55 in FP64) and holds 6
-// steps where the lattice is small enough; then 32 x 32.  Beyond one tile
-// per CU, two; then 4 steps.  Measured, us a step in FP64: 129^2 24 x 24 at
-// 4 / 6 / 8 steps 2.52 / 2.12 / 2.54, 32 x 32 at 10 2.15; 200^2 24 x 24 at
-// 5 2.76, 32 x 32 at 8 2.67; 400^2 32 x 32 at 4 / 6 / 8 5.5 / 5.0 / 5.8;
-// 251 x 1003 7.1 / 7.9 / 8.3.  From about 300000 nodes the marching waves
-// are as fast (FP64 / FP32: 1400 x 200 march 7.8 / 5.6, porous 500 x 700 7.6
-// / 5.7; 500^2 tiles 7.0 / 4.9); FP16, which has none, stays until single
-// steps are (700^2 8.5 against 12.4, 1000^2 16.4).
+// launch's fixed cost, and a second tile on a CU costs what it saves.  Smaller
+// regions step faster (waves per SIMD: 24 x 24 two to three, 32 x 24 three, 32
+// x 32 four) but hold fewer steps: the shapes are tried from the fastest per
+// step on.  Beyond one tile
+// per CU 8- and 4-byte elements part: two 32 x 24 tiles of FP32 or FP16 run
+// on a CU side by side.  Measured, us a step (steps a launch): 129^2 FP64
+// 32 x 24 1.85 (9), 32 x 20 1.84 (7), 32 x 16 1.95 (6), 24 x 24 2.05 (7), 32 x
+// 32 2.15 (10), FP32 1.45, 1.53, -, 1.60, 1.65; 65^2 FP64 24 x 24 1.75 (8), 32
+// x 24 1.86 (9); 160^2 24 x 24 1.92 (7), 32 x 24 2.01 (8); 200^2 FP64 32 x 24 2.27 (7), 32
+// x 32 2.50 (7); 300^2 FP64 32 x 32 3.26 (6), 32 x 24 3.71 (4); 251 x 1003 FP32
+// 32 x 24 4.63 (5), 4.88 (6), 32 x 32 5.14 (4), FP64 7.97 (4), 7.23 (4).  From
+// about 300000 nodes the marching waves are as fast (FP64 / FP32: 1400 x 200
+// march 7.8 / 5.6, porous 500 x 700 7.6 / 5.7); FP16, which has none, stays
+// until single steps are: 700^2 6.7 against 12.4, 1000^2 11.0 against 16.3,
+// 1500^2 about 24 either way.
 TileShape tile_shape(int32_t storage, const StepArgs &a)
 {
     const int64_t nodes = (int64_t)a.g.nr * a.g.nc;
-    if (nodes >= (storage == kF16 ? kTileMaxNodesF16 : kTileMaxNodes)) return {0, 0};
-    for (int32_t halo = 8; halo >= 6; --halo)
-        if (tiles_of(a, {24, halo}) <= a.cus) return {24, halo};
-    for (int32_t per_cu : {1, 2})
-        for (int32_t halo = 10; halo >= 4; --halo)
-            if (tiles_of(a, {32, halo}) <= (int64_t)per_cu * a.cus) return {32, halo};
-    return {32, 4};
+    if (nodes >= (storage == kF16 ? kTileMaxNodesF16 : kTileMaxNodes)) return {0, 0, 0};
+    constexpr TileShape kOnePerCu[] = {{24, 24, 8}, {32, 24, 9}, {24, 24, 7}, {32, 24, 8}, {32, 24, 7}, {32, 32, 9},
+                                       {32, 32, 8}, {32, 32, 7}, {32, 32, 6}, {32, 32, 5}, {32, 32, 4}};
+    for (const TileShape &t : kOnePerCu)
+        if ((t.halo > 4 || storage == kF64) && tiles_of(a, t) <= a.cus) return t;
+    if (storage != kF64) {
+        if (tiles_of(a, {32, 24, 6}) <= 3 * (int64_t)a.cus) return {32, 24, 6};
+        return {32, 24, storage == kF16 && tiles_of(a, {32, 24, 5}) > 4 * (int64_t)a.cus ? 4 : 5};
+    }
+    for (int32_t halo = 7; halo > 4; --halo)
+        if (tiles_of(a, {32, 32, halo}) <= 2 * (int64_t)a.cus) return {32, 32, halo};
+    return {32, 32, 4};
 }
 
-template <typename T>
+template <typename T, bool PS>
 hipError_t launch_tile_t(const StepArgs &a, TileShape t, int32_t steps, hipStream_t s)
 {
-    const int32_t n = t.side - 2 * t.halo, ti = (a.g.nr + n - 1) / n;
-    const dim3 grid((unsigned)tiles_of(a, t)), block((unsigned)(t.side * t.side));
-    if constexpr (sizeof(T) == 8) {
-        if (a.psbb) {
-            if (t.side == 24) hipLaunchKernelGGL((tile_kernel<T, 24, true>), grid, block, 0, s, a, steps, t.halo, ti);
-            else hipLaunchKernelGGL((tile_kernel<T, 32, true>), grid, block, 0, s, a, steps, t.halo, ti);
-            return hipGetLastError();
-        }
-    }
-    if (t.side == 24) hipLaunchKernelGGL((tile_kernel<T, 24>), grid, block, 0, s, a, steps, t.halo, ti);
-    else hipLaunchKernelGGL((tile_kernel<T, 32>), grid, block, 0, s, a, steps, t.halo, ti);
+    const int32_t n = t.rows - 2 * t.halo, ti = (a.g.nr + n - 1) / n;
+    const dim3 grid((unsigned)tiles_of(a, t)), block((unsigned)(t.rows * t.cols));
+    if (t.rows == 24) hipLaunchKernelGGL((tile_kernel<T, 24, 24, PS>), grid, block, 0, s, a, steps, t.halo, ti);
+    else if (t.cols == 24) hipLaunchKernelGGL((tile_kernel<T, 32, 24, PS>), grid, block, 0, s, a, steps, t.halo, ti);
+    else hipLaunchKernelGGL((tile_kernel<T, 32, 32, PS>), grid, block, 0, s, a, steps, t.halo, ti);
     return hipGetLastError();
 }
 
@@ -2349,9 +2353,9 @@ hipError_t launch_tile(int32_t storage, int32_t steps, const StepArgs &a0, hipSt
     const TileShape t = tile_shape(storage, a);
     if (steps < 1 || steps > t.halo) return hipErrorInvalidValue;
     switch (storage) {
-    case kF64: return launch_tile_t<double>(a, t, steps, s);
-    case kF32: return launch_tile_t<float>(a, t, steps, s);
-    default: return launch_tile_t<_Float16>(a, t, steps, s);
+    case kF64: return a.psbb ? launch_tile_t<double, true>(a, t, steps, s) : launch_tile_t<double, false>(a, t, steps, s);
+    case kF32: return launch_tile_t<float, false>(a, t, steps, s);
+    default: return launch_tile_t<_Float16, false>(a, t, steps, s);
     }
 }
 

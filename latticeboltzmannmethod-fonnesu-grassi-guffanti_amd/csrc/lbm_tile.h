@@ -17,31 +17,31 @@
 // domain hold those values in LDS and are never overwritten, so the gather
 // needs no case for them.
 //
-// What bounds it: latency.  A launch costs about 4.6 us (FP64, S = 24) and
-// 1.3 us a step (a gather from LDS, a barrier, the collision's dependent
-// chain, a store, a barrier).  us a step, single steps -> tiles: 129^2
-// cavity FP64 7.7 -> 2.1, FP32 7.1 -> 1.5, FP16 7.9 -> 1.7; channel 40 x 96
-// FP64 7.0 -> 1.7; 300^2 FP64 9.1 -> 3.3; 251 x 1003 FP32 9.6 -> 5.1.
+// What bounds it: latency.  A launch costs about 5 us and a step 1.2 us in
+// FP64 (a gather from LDS, a barrier, the collision's dependent chain, a
+// store, a barrier).  us a step, single steps -> tiles: 129^2 cavity FP64 7.7
+// -> 1.85, FP32 7.1 -> 1.45, FP16 7.9 -> 1.7; channel 40 x 96 FP64 7.0 -> 1.7;
+// 300^2 FP64 9.1 -> 3.3; 251 x 1003 FP32 9.6 -> 4.6.
 //
 // Same arithmetic per node as the step kernels, same bits.
 // PS: partially saturated obstacles (FP64).  A node keeps the populations
 // that enter it through its obstacle slots, and their weights, in registers
 // (psbb_gather, psbb_update); its carried values alternate between two
 // buffers like the state, since the tiles around it read the old ones.
-template <typename T, int kTileSide, bool PS = false>
-__global__ __launch_bounds__(kTileSide * kTileSide) void tile_kernel(StepArgs a, int32_t steps, int32_t halo, int32_t tiles_i)
+template <typename T, int kRows, int kCols, bool PS = false>
+__global__ __launch_bounds__(kRows * kCols) void tile_kernel(StepArgs a, int32_t steps, int32_t halo, int32_t tiles_i)
 {
-    constexpr int kTileNodes = kTileSide * kTileSide;
+    constexpr int kTileNodes = kRows * kCols;
     __shared__ T F[9 * kTileNodes];
     __shared__ uint8_t kind[kTileNodes];  // 0 dry, 1 wet, 2 outside the domain
-    const int32_t nr = a.g.nr, nc = a.g.nc, side = kTileSide - 2 * halo;
+    const int32_t nr = a.g.nr, nc = a.g.nc;
     const int32_t tj = (int32_t)blockIdx.x / tiles_i, ti = (int32_t)blockIdx.x - tj * tiles_i;
     const int32_t pos = threadIdx.x;
-    const int32_t rj = pos / kTileSide, ri = pos - rj * kTileSide;
-    const int32_t i = ti * side - halo + ri, j = tj * side - halo + rj;
+    const int32_t rj = pos / kRows, ri = pos - rj * kRows;
+    const int32_t i = ti * (kRows - 2 * halo) - halo + ri, j = tj * (kCols - 2 * halo) - halo + rj;
     const bool inside = (uint32_t)i < (uint32_t)nr && (uint32_t)j < (uint32_t)nc;
     // distance from the region's border: the node is valid for that many steps
-    const int32_t depth = min(min(ri, kTileSide - 1 - ri), min(rj, kTileSide - 1 - rj));
+    const int32_t depth = min(min(ri, kRows - 1 - ri), min(rj, kCols - 1 - rj));
 
     bool wet = false;
     int32_t own = 0;
@@ -114,8 +114,8 @@ __global__ __launch_bounds__(kTileSide * kTileSide) void tile_kernel(StepArgs a,
 #pragma unroll
     for (int d = 1; d < 9; ++d) {
         const int32_t si = ri - kOffI[d], sj = rj - kOffJ[d];
-        const bool in = (uint32_t)si < (uint32_t)kTileSide && (uint32_t)sj < (uint32_t)kTileSide;
-        const int32_t sp = in ? sj * kTileSide + si : pos;
+        const bool in = (uint32_t)si < (uint32_t)kRows && (uint32_t)sj < (uint32_t)kCols;
+        const int32_t sp = in ? sj * kRows + si : pos;
         src[d] = kind[sp] != 0 ? d * kTileNodes + sp : kOpp[d] * kTileNodes + pos;
     }
 #pragma unroll 1
