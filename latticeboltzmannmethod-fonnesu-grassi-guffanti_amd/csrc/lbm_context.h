@@ -65,6 +65,8 @@ struct lbm_ctx {
     double *d_bc[2] = {nullptr, nullptr};
     double *h_bc_pin = nullptr;  // bc_slots slots of [3][E], used in turn
     int bc_slots = 0, bc_slot = 0;
+    double *h_out = nullptr;  // behind the slots: kOutDoubles results the kernels write for the host
+    static constexpr int kOutDoubles = 8;
     bool bc_pending = false;
     hipEvent_t bc_ev[2] = {nullptr, nullptr};  // last reader of each half of the slots
     int bc_cur = 0, bc_prev = 0;

@@ -233,6 +233,8 @@ hipError_t launch_march(int32_t storage, int32_t steps, const StepArgs &a, hipSt
 int32_t tile_steps(int32_t storage, const StepArgs &a);
 hipError_t launch_tile(int32_t storage, int32_t steps, const StepArgs &a, hipStream_t s);
 int64_t readout_blocks(const StepArgs &a);
+// Parts of a [3][n] field to host memory the device can write (either nullptr).
+hipError_t launch_copy_fields(const double *macro, int64_t n, double *rho, double *u, hipStream_t s);
 // rho = 1, u = 0 over a field of n nodes ([3][n] doubles).
 hipError_t launch_fill_macro(double *macro, int64_t n, hipStream_t s);
 

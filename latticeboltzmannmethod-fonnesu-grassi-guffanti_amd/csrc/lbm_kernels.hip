@@ -1893,6 +1893,20 @@ __global__ __launch_bounds__(kBlockRows) void fill_macro(double *macro, int64_t 
     macro[2 * n + q] = 0.0;
 }
 
+// Copies a [3][n] field's parts to rho (n doubles) and u (2 n), either
+// nullptr: page-locked host memory, for fields too small to be worth a copy
+// engine's start (download_fields).
+__global__ __launch_bounds__(kBlockRows) void copy_fields(const double *macro, int64_t n, double *rho, double *u)
+{
+    const int64_t q = (int64_t)blockIdx.x * kBlockRows + threadIdx.x;
+    if (q >= 3 * n) return;
+    if (q < n) {
+        if (rho) rho[q] = macro[q];
+    } else if (u) {
+        u[q - n] = macro[q];
+    }
+}
+
 // Compact index of wet node (i, j), any thread.
 __device__ __forceinline__ int64_t cidx_of(const Geometry &g, int64_t i, int64_t j)
 {
@@ -2469,6 +2483,13 @@ hipError_t launch_lift_drag(int32_t storage, const StepArgs &a0, const void *fst
     case kF32: hipLaunchKernelGGL(lift_drag<float>, grid, block, 0, s, a, ij, masks, n, per_point, partials); break;
     default: hipLaunchKernelGGL(lift_drag<_Float16>, grid, block, 0, s, a, ij, masks, n, per_point, partials); break;
     }
+    return hipGetLastError();
+}
+
+hipError_t launch_copy_fields(const double *macro, int64_t n, double *rho, double *u, hipStream_t s)
+{
+    const int64_t nb = (3 * n + kBlockRows - 1) / kBlockRows;
+    hipLaunchKernelGGL(copy_fields, dim3((unsigned)nb), dim3(kBlockRows), 0, s, macro, n, rho, u);
     return hipGetLastError();
 }
 

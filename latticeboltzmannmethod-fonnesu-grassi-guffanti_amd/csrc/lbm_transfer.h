@@ -14,6 +14,9 @@ namespace lbm {
 hipError_t copy_to_host(int device, void *dst, const void *src, size_t bytes, hipStream_t s);
 hipError_t copy_to_device(int device, void *dst, const void *src, size_t bytes, hipStream_t s);
 
+// The device's view of page-locked host memory (nullptr for other memory).
+void *device_view(const void *host);
+
 // Contexts alive: the page-locked chunks the copies go through are shared by
 // all of them and freed with the last one.
 void transfer_retain();

@@ -116,6 +116,16 @@ hipError_t copy_to_device(int device, void *dst, const void *src, size_t bytes, 
     return copy(device, dst, src, bytes, hipMemcpyHostToDevice, s);
 }
 
+void *device_view(const void *host)
+{
+    hipPointerAttribute_t at{};
+    if (hipPointerGetAttributes(&at, host) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    return at.type == hipMemoryTypeHost ? at.devicePointer : nullptr;
+}
+
 void transfer_retain()
 {
     std::lock_guard<std::mutex> lock(g_refs_mu);

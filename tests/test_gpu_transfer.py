@@ -62,3 +62,33 @@ def test_threads():
     for t in threads:
         t.join()
     assert not bad
+
+
+# 24 bytes a node: either side of the size up to which a kernel writes the fields
+@pytest.mark.parametrize("nr,nc", [(3, 3), (209, 209), (210, 209), (600, 400)])
+def test_fields_into_page_locked_memory(nr, nc):
+    n = nr * nc
+    ptr = C.c_void_p()
+    assert L.lib().lbm_host_alloc(3 * n * 8, C.byref(ptr)) == 0
+    buf = np.frombuffer((C.c_double * (3 * n)).from_address(ptr.value))
+    with L.Lattice(box(nr, nc), storage=L.F64, tau=0.8) as lat:
+        lat.upload_populations(state(np.random.default_rng(nr), nc, nr))
+        for k in range(3):
+            lat.step(2, L.STEP_MACRO)
+            rho, u = lat.macro()
+            buf[:] = -1.0
+            lat.wait(lat.macro_async(buf[:n].reshape(nc, nr), buf[n:].reshape(2, nc, nr)))
+            assert np.array_equal(buf[:n].reshape(nc, nr), rho) and np.array_equal(buf[n:].reshape(2, nc, nr), u)
+        # either part alone, and one of them in pageable memory
+        t = C.c_int64()
+        dp = C.POINTER(C.c_double)
+        own = np.empty((nc, nr))
+        buf[:] = -1.0
+        assert L.lib().lbm_download_macro_async(lat._h, None, C.cast(ptr.value + 8 * n, dp), C.byref(t)) == 0
+        lat.wait(t.value)
+        assert np.array_equal(buf[n:].reshape(2, nc, nr), u) and (buf[:n] == -1.0).all()
+        assert L.lib().lbm_download_macro_async(lat._h, own.ctypes.data_as(dp), C.cast(ptr.value + 8 * n, dp),
+                                                C.byref(t)) == 0
+        lat.wait(t.value)
+        assert np.array_equal(own, rho)
+    assert L.lib().lbm_host_free(ptr) == 0
