@@ -301,9 +301,10 @@ int lbm_get_scale(lbm_ctx *ctx, double *scale);
  * lane's neighbour addressing read from a table built on first use (4 bytes
  * per wet node and step more traffic, far fewer instructions per wave).
  * Results are the same bits for every shape.  With 0 (the default), steps
- * without new prescribed values may run several to a launch (FP64 and FP32
- * storage, blocked layout); a shape set here is a launch of one step.  No
- * counterpart in the reference (a tuning knob of this engine). */
+ * run several to a launch where the lattice allows it (small lattices;
+ * larger ones in FP64 and FP32 storage); a shape set here is a launch of one
+ * step.  No counterpart in the reference (a tuning knob of
+ * this engine). */
 enum { LBM_LAUNCH_WET_RUNS = 64, LBM_LAUNCH_RUN_TABLE = 65 };
 int lbm_set_launch(lbm_ctx *ctx, int32_t segments);
 int lbm_get_launch(lbm_ctx *ctx, int32_t *segments);
@@ -320,7 +321,8 @@ int lbm_get_occupancy(lbm_ctx *ctx, int32_t *groups_per_cu);
 
 /* Times each launch shape (1, 2, 4, 8 segments, wet runs, tabled wet runs)
  * at each occupancy (no limit, 7 down to 3 work-groups per compute unit),
- * and launches of several steps where the lattice takes them, over `steps` launches (every launch rewrites the spare buffer from the
+ * and launches of several steps where the lattice takes them, over `steps`
+ * launches (every launch rewrites the spare buffer from the
  * current state, so the state does not change) and keeps the fastest
  * pair for single steps, and several steps per launch if they are faster
  * still.  Reports the shape of the single steps and the time per step

@@ -3,8 +3,8 @@
 // A batch keeps, per sample, two complete step-argument sets (one per
 // buffer parity) in device memory and a tile table (sample, column, first
 // row of R 64-row segments) covering every tile that holds a wet node.
-// One time step of the whole ensemble is one launch of batch_kernel, a
-// persistent grid that walks the table.  Runs of steps replay a captured
+// One time step of the whole ensemble is one launch of batch_kernel, with
+// one wave per tile or a persistent grid that walks the table.  Runs of steps replay a captured
 // HIP graph of an even number of launches, so a replay leaves the buffer
 // parity unchanged.  Steps without new prescribed values run kBatchMarchSteps
 // to a launch (batch_march_kernel) where every sample is blocked FP64 or

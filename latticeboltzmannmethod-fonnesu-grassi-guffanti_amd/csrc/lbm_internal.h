@@ -223,7 +223,7 @@ constexpr int64_t kTileMaxNodes = 300000, kTileMaxNodesF16 = (int64_t)3 << 19;
 constexpr int64_t kMarchMinNodes = (int64_t)1 << 17, kBatchFusedNodes = (int64_t)1 << 20;
 // Steps per launch of the marching kernel for this lattice (0: not for it),
 // and such a launch: `steps` steps (2 .. march_steps) without new prescribed
-// values from fin (F*) to fout, blocked layout.
+// values from fin (F*) to fout.
 int32_t march_steps(int32_t storage, const StepArgs &a);
 hipError_t launch_march(int32_t storage, int32_t steps, const StepArgs &a, hipStream_t s);
 // Steps per launch of the tile kernel for this lattice (0: not for it), and

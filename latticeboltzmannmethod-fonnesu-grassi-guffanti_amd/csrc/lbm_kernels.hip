@@ -1,7 +1,9 @@
 // gfx950 kernels of the D2Q9 engine.
 //
-// One fused kernel per time step, pull scheme, A-B buffers holding the
-// post-collision populations F* of the previous step.  For a wet node x
+// Fused time steps, pull scheme, A-B buffers holding the post-collision
+// populations F* of the previous step: several steps per launch (marching
+// waves, lbm_march.h; tiles in LDS for small lattices, lbm_tile.h), or one
+// step per launch through the step kernels below.  For a wet node x
 // and direction d with source s = x - c_d (c_d = the push offset of d in
 // the reference's stream, BGKCollision.hpp:179-187):
 //   s wet            -> P_d(x) = F*_d(s)                 (stream)
@@ -1633,8 +1635,8 @@ __global__ __launch_bounds__(kBlockRows) void batch_march_kernel(BatchArgs bt)
     const int j0 = __builtin_amdgcn_readfirstlane(e[2]);
     const int j1 = __builtin_amdgcn_readfirstlane(e[3]);
     const StepArgs a = args_at(bt, s);
-    if (j1 < 0) march_wave<T, K, FUSED, true>(a, i0, j0, j1 & 0x7fffffff, lane);
-    else march_wave<T, K, FUSED, false>(a, i0, j0, j1, lane);
+    if (j1 < 0) march_wave<T, K, FUSED, true, false>(a, i0, j0, j1 & 0x7fffffff, lane);
+    else march_wave<T, K, FUSED, false, false>(a, i0, j0, j1, lane);
 }
 
 // The time-step kernel of a batch of independent lattices: a persistent
@@ -2092,13 +2094,18 @@ hipError_t launch_march_t(StepArgs a, hipStream_t s)
     const int64_t chunks = inner > 0 ? (a.g.nc - 2 * (K + 1) + m.cols - 1) / m.cols : 0;
     a.nblocks = (m.edge_waves + inner * chunks + kBlockRows / 64 - 1) / (kBlockRows / 64);
     const dim3 grid((unsigned)a.nblocks), block(kBlockRows);
-    if constexpr (K == 5) {  // large lattices only
-        hipLaunchKernelGGL((march_kernel<T, K, true>), grid, block, 0, s, a, m);
-    } else if constexpr (K == 4) {
-        if (march_large(a)) hipLaunchKernelGGL((march_kernel<T, K, true>), grid, block, 0, s, a, m);
-        else hipLaunchKernelGGL((march_kernel<T, K, false>), grid, block, 0, s, a, m);
-    } else {
-        hipLaunchKernelGGL((march_kernel<T, K, false>), grid, block, 0, s, a, m);
+    // K = 5: large lattices only.  Lattices in planes, which are large unless
+    // that layout was asked for, have the fused copy only at K = 4.
+    const bool fused = K == 5 || (K == 4 && (march_large(a) || !a.block_mask));
+    if constexpr (K >= 4) {
+        if (fused && !a.block_mask) hipLaunchKernelGGL((march_kernel<T, K, true, true>), grid, block, 0, s, a, m);
+        else if (fused) hipLaunchKernelGGL((march_kernel<T, K, true, false>), grid, block, 0, s, a, m);
+    }
+    if constexpr (K <= 4) {
+        if (!fused && a.block_mask) hipLaunchKernelGGL((march_kernel<T, K, false, false>), grid, block, 0, s, a, m);
+    }
+    if constexpr (K < 4) {
+        if (!a.block_mask) hipLaunchKernelGGL((march_kernel<T, K, false, true>), grid, block, 0, s, a, m);
     }
     return hipGetLastError();
 }
@@ -2283,13 +2290,13 @@ hipError_t launch_batch_step(int32_t storage, bool gather, int32_t R, const Batc
 int32_t march_steps(int32_t storage, const StepArgs &a)
 {
     const int64_t nodes = (int64_t)a.g.nr * a.g.nc;
-    if (storage == kF16 || a.psbb || !a.block_mask || nodes < kTileMaxNodes) return 0;
+    if (storage == kF16 || a.psbb || nodes < kTileMaxNodes) return 0;
     return storage == kF64 && march_large(a) ? 5 : 4;
 }
 
 hipError_t launch_march(int32_t storage, int32_t steps, const StepArgs &a, hipStream_t s)
 {
-    if (storage == kF16 || a.psbb || !a.block_mask) return hipErrorInvalidValue;
+    if (storage == kF16 || a.psbb) return hipErrorInvalidValue;
     const bool f64 = storage == kF64;
     switch (steps) {
     case 2: return f64 ? launch_march_t<double, 2>(a, s) : launch_march_t<float, 2>(a, s);

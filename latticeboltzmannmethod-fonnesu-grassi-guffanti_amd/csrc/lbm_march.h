@@ -242,44 +242,56 @@ __device__ __forceinline__ int close_edge(const StepArgs &a, int i, int j, T *p,
     return policy;
 }
 
-// One 64-row window's elements in memory, blocked layout: a scalar base at
-// the 64-node block of the window's first wet row, and the byte offset of
-// this lane's node from it (the window's nodes fall in two blocks at most).
-template <typename T>
+// One 64-row window's elements in memory: a scalar base at the 64-node block
+// of the window's first wet row, and the byte offset of this lane's node from
+// it (the window's nodes fall in two blocks at most).  The directions lie 64
+// elements apart (blocked) or, PLANES, a plane apart: a scalar base each,
+// formed by adding.  Lattices of 4 GiB and more a buffer lie in planes.  us a
+// step, one step a launch (tuned) -> this: open 8192^2 FP64 1583 -> 484 (420
+// would be blocked FP64's time per node); 2100^2 FP64 36.2 against 35.5
+// blocked, FP32 23.7 against 22.6.
+template <typename T, bool PLANES>
 __device__ __forceinline__ int64_t win_base(const Win &w)
 {
-    return (int64_t)(w.base >> 6) * (int64_t)(9 * 64 * sizeof(T));
+    return (int64_t)(w.base >> 6) * (int64_t)((PLANES ? 1 : 9) * 64 * sizeof(T));
 }
 
-template <typename T>
+template <typename T, bool PLANES>
 __device__ __forceinline__ uint32_t win_offset(const Win &w)
 {
     const uint32_t r = __builtin_amdgcn_mbcnt_hi((uint32_t)(w.mid >> 32),
                                                  __builtin_amdgcn_mbcnt_lo((uint32_t)w.mid, (uint32_t)w.base & 63u));
-    return (r + 8u * (r & 64u)) * (uint32_t)sizeof(T);
+    return (PLANES ? r : r + 8u * (r & 64u)) * (uint32_t)sizeof(T);
 }
 
 // The 9 stored populations of the window's nodes.
-template <typename T>
+template <typename T, bool PLANES>
 __device__ __forceinline__ void win_load(const StepArgs &a, const Win &w, T *raw)
 {
-    const LBM_GLOBAL char *base = (const LBM_GLOBAL char *)a.fin + win_base<T>(w);
-    const uint32_t off = win_offset<T>(w);
+    const LBM_GLOBAL char *base = (const LBM_GLOBAL char *)a.fin + win_base<T, PLANES>(w);
+    const uint32_t off = win_offset<T, PLANES>(w);
+    const int64_t apart = PLANES ? a.g.plane * (int64_t)sizeof(T) : (int64_t)(64 * sizeof(T));
 #pragma unroll
-    for (int d = 0; d < 9; ++d) raw[d] = *(const LBM_GLOBAL T *)(base + d * 64 * (int)sizeof(T) + off);
+    for (int d = 0; d < 9; ++d, base += apart) raw[d] = *(const LBM_GLOBAL T *)(base + off);
 }
 
 // Stores o for the lanes of m, without a branch: the other lanes' offsets
 // lie outside the buffer descriptor's range, so their writes are dropped.
-template <typename T>
+template <typename T, bool PLANES>
 __device__ __forceinline__ void win_store(const StepArgs &a, const Win &w, uint64_t m, const T *o)
 {
-    char *base = (char *)a.fout + win_base<T>(w);
-    const uint32_t off = __builtin_amdgcn_inverse_ballot_w64(m) ? win_offset<T>(w) : 0x40000000u;
-    const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(base, 0, 2 * 9 * 64 * (int)sizeof(T), 0x00027000);
+    char *base = (char *)a.fout + win_base<T, PLANES>(w);
+    const uint32_t off = __builtin_amdgcn_inverse_ballot_w64(m) ? win_offset<T, PLANES>(w) : 0x40000000u;
+    auto rsrc = __builtin_amdgcn_make_buffer_rsrc(base, 0, (PLANES ? 2 : 2 * 9) * 64 * (int)sizeof(T), 0x00027000);
 #pragma unroll
     for (int d = 0; d < 9; ++d) {
-        const int at = d * 64 * (int)sizeof(T);
+        if constexpr (PLANES) {
+            if (d > 0) {
+                base += a.g.plane * (int64_t)sizeof(T);
+                rsrc = __builtin_amdgcn_make_buffer_rsrc(base, 0, 2 * 64 * (int)sizeof(T), 0x00027000);
+            }
+        }
+        const int at = PLANES ? 0 : d * 64 * (int)sizeof(T);
         if constexpr (sizeof(T) == 8) {
             typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
             __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, o[d]), rsrc, (int)off + (at & 4095),
@@ -314,7 +326,7 @@ __device__ __forceinline__ bool march_collide(const StepArgs &a, T *p, const Win
     else return collide_shifted<false, false>(a, p, policy, v, 0, j, o);
 }
 
-template <typename T, int K, bool FUSED, bool EDGE>
+template <typename T, int K, bool FUSED, bool EDGE, bool PLANES>
 __device__ __forceinline__ void march_wave(const StepArgs &a, int32_t i0, int32_t j0, int32_t j1, int lane)
 {
     constexpr uint64_t kOut = ((1ull << (64 - 2 * K)) - 1ull) << K;  // lanes whose rows this wave owns
@@ -328,7 +340,7 @@ __device__ __forceinline__ void march_wave(const StepArgs &a, int32_t i0, int32_
     for (int q = 0; q < K; ++q) lv[q] = Level<T>{};
     T raw[9];
     w[0] = window(load_words(a.g, first, i0), i0);
-    win_load(a, w[0], raw);
+    win_load<T, PLANES>(a, w[0], raw);
     WinWords nw = load_words(a.g, EDGE ? min(first + 1, nc) : first + 1, i0);
     bool bad = false;
     // one column: c enters, column c - K leaves (all levels active)
@@ -340,7 +352,7 @@ __device__ __forceinline__ void march_wave(const StepArgs &a, int32_t i0, int32_
         w[0] = window(nw, i0);
         nw = load_words(a.g, EDGE ? min(c + 2, nc) : c + 2, i0);
         feed<FUSED>(lv[0], raw, w[1], w[2], p);
-        win_load(a, w[0], raw);
+        win_load<T, PLANES>(a, w[0], raw);
 #pragma unroll
         for (int q = 1; q <= K; ++q) {
             // level q of column c - q
@@ -353,7 +365,7 @@ __device__ __forceinline__ void march_wave(const StepArgs &a, int32_t i0, int32_
             } else {
                 const uint64_t m = j < j1 ? w[K + 1].mid & kOut : 0ull;
                 bad |= nan && __builtin_amdgcn_inverse_ballot_w64(m);
-                win_store(a, w[K + 1], m, o);
+                win_store<T, PLANES>(a, w[K + 1], m, o);
             }
         }
     };
@@ -385,7 +397,7 @@ __device__ __forceinline__ void march_wave(const StepArgs &a, int32_t i0, int32_
 // 116.5 -> 112.0, FP32 69.3 -> 67.5; open 3001 x 5003 FP64 111.7 -> 106.9;
 // porous 8192^2 FP32 261.5 -> 253.8; an ensemble of 60 lattices of up to 256^2
 // FP64 31.2 -> 28.7, of 8 of them FP32 6.6 -> 7.0.
-template <typename T, int K, bool FUSED>
+template <typename T, int K, bool FUSED, bool PLANES>
 __global__ __launch_bounds__(kBlockRows) void march_kernel(StepArgs a, MarchPlan m)
 {
     constexpr int32_t kRows = 64 - 2 * K;
@@ -410,7 +422,7 @@ __global__ __launch_bounds__(kBlockRows) void march_kernel(StepArgs a, MarchPlan
             j0 = right ? nc - (K + 1) : 0;
             j1 = right ? nc : K + 1;
         }
-        march_wave<T, K, FUSED, true>(a, stripe * kRows - K, j0, j1, lane);
+        march_wave<T, K, FUSED, true, PLANES>(a, stripe * kRows - K, j0, j1, lane);
         return;
     }
     t -= m.edge_waves;
@@ -418,6 +430,6 @@ __global__ __launch_bounds__(kBlockRows) void march_kernel(StepArgs a, MarchPlan
     const int32_t j0 = K + 1 + chunk * m.cols;
     const int32_t end = nc - (K + 1);
     if (j0 >= end) return;
-    march_wave<T, K, FUSED, false>(a, (m.top + t - chunk * inner) * kRows - K, j0, min(j0 + m.cols, end), lane);
+    march_wave<T, K, FUSED, false, PLANES>(a, (m.top + t - chunk * inner) * kRows - K, j0, min(j0 + m.cols, end), lane);
 }
 

@@ -145,3 +145,26 @@ def test_ensemble_same_bits_as_single_steps(storage, big):
             lat.close()
     for shape, x, y in zip(shapes, *out):
         assert np.array_equal(x, y), shape
+
+
+@pytest.mark.parametrize("storage", [L.F64, L.F32_SHIFTED])
+@pytest.mark.parametrize("nr,nc", [(56, 5370), (113, 2670), (30100, 10), (2051, 2047)])
+def test_planes(nr, nc, storage):
+    """The layout of lattices beyond 4 GiB a buffer, asked for: one stripe of
+    windows, several, all windows on the perimeter, and the large lattices'
+    launches, at every remainder of a launch."""
+    rng = np.random.default_rng(nr + nc)
+    cls = random_class(rng, nr, nc, 0.15)
+    p0 = state(rng, nc, nr)
+    for n in (3, 4, 5, 10, 46):
+        out = []
+        for options, flags in ((L.OPT_PLANAR_LAYOUT, 0), (L.OPT_PLANAR_LAYOUT, L.STEP_NO_GRAPH)):
+            lat = L.Lattice(cls, tau=0.8, inlet_policy=L.ZOUHE_PRESSURE, outlet_policy=L.OPEN_NOOP, storage=storage,
+                            options=options)
+            lat.set_open_values(0, rho=np.full(len(lat.open_nodes(0)), 1.001))
+            assert lat.layout() == L.LAYOUT_PLANES
+            lat.upload_populations(p0)
+            lat.step(n, flags)
+            out.append(lat.populations())
+            lat.close()
+        assert np.array_equal(*out), n
