@@ -1,7 +1,7 @@
 """Throughput of the D2Q9 time step on one MI355X.
 
-A "step" is one lattice-Boltzmann time step (one launch of the fused step
-kernel) over the whole workload.  Default workload: the 8192 x 8192 random
+A "step" is one lattice-Boltzmann time step over the whole workload
+(FP64 and FP32 lattices advance several of them per launch).  Default workload: the 8192 x 8192 random
 porous medium (discs r in [4, 16], 30 % solid, BGK tau 0.8, Zou-He pressure
 inlet 1.001 / outlet 1.000), populations resident in HBM before the timed
 region.  The headline value is the MLUPS of the FP32 shifted-population
@@ -12,18 +12,22 @@ against the FP64 run, and their FP64-reduced mass difference, are stated.
 
 The ensemble line advances 512 independent porous lattices (rows and
 columns in {128, ..., 1024}, porosity in [0.5, 0.9], discs r in [3, 12])
-with one step-kernel launch per step, HIP-graph replay and the autotuned
-tile shape, in FP32; its per-sample Darcy permeabilities (FP64 GPU
+in FP32 with HIP-graph replay and the autotuned launch (several steps per
+launch, or one over tiles); its per-sample Darcy permeabilities (FP64 GPU
 reductions) are checked against an FP64 ensemble.
 
-MLUPS = wet nodes * steps / time / 1e6.  Algorithmic HBM bytes per step =
-wet nodes * 18 * sizeof(storage) + NR*NC/8 (bit-packed wet mask); the
-roofline fraction divides the achieved rate by MI355X's 8 TB/s; the rate of
+MLUPS = wet nodes * steps / time / 1e6.  Algorithmic HBM bytes per launch =
+wet nodes * 18 * sizeof(storage) + NR*NC/8 (bit-packed wet mask); per step
+that is divided by the steps one launch takes (steps_per_launch), since the
+populations are read and written once per launch.  The roofline fraction
+divides the rate of those bytes by MI355X's 8 TB/s.  one_step_gbs is the
+rate that one step per launch would need for the same MLUPS: it passes
+8 TB/s where several steps share a launch.  The rate of
 a plain 16-byte-per-lane copy kernel over one FP32 population buffer's
 volume is measured in the same run and reported beside it as the practical
-ceiling of a stream (copy_ceiling, frac_of_copy).  The step
-kernel is the only kernel in the timed region, so its average duration is
-the event-timed region divided by the number of steps.
+ceiling of a stream (copy_ceiling, frac_of_copy).  The step kernels are the
+only kernels in the timed region, so the time per step is the event-timed
+region divided by the number of steps.
 
 The CPU baseline is the repo's CPU oracle in the reference's step structure
 (list-driven sweeps, three population tensors, the by-value rho / u copies
@@ -170,6 +174,27 @@ def random_state(wl):
     return _RANDOM_STATE[wl.name]
 
 
+def steps_per_launch(wl, storage):
+    """Time steps per launch of the library's rule for lattices beyond the
+    tiles' size (300,000 nodes): marching waves take 4 steps of FP64 and
+    FP32 lattices, 5 of FP64 lattices of at least 2^22 nodes; FP16 lattices
+    take one.  None for smaller lattices, whose tiles take 4 to 9 steps."""
+    nodes = wl.nr * wl.nc
+    if nodes < (3 << 19 if storage == L.F16_SHIFTED else 300000):
+        return None
+    if storage == L.F16_SHIFTED:
+        return 1
+    return 5 if storage == L.F64 and nodes >= 1 << 22 else 4
+
+
+def warm_graphs(step):
+    """Captures the step graphs of both buffer parities (a graph holds at
+    most 72 steps)."""
+    step(80, L.STEP_CHECK)
+    step(1, L.STEP_CHECK)
+    step(80, L.STEP_CHECK)
+
+
 def time_storage(wl, name, steps, warmup, ev):
     storage, options = VARIANTS[name]
     lat = wl.make_lattice(storage, options=options)
@@ -177,7 +202,7 @@ def time_storage(wl, name, steps, warmup, ev):
         lat.upload_populations(random_state(wl))
     lat.step(warmup, L.STEP_CHECK)
     segments, _ = lat.autotune(steps=5)
-    lat.step(2 * 32, L.STEP_CHECK)              # capture and warm the step graphs
+    warm_graphs(lat.step)
     lat.synchronize()
     stream = lat.stream_handle()
     t0 = time.perf_counter()
@@ -188,13 +213,29 @@ def time_storage(wl, name, steps, warmup, ev):
     nwet = wl.wet_count()
     per_step_s = ms / 1e3 / steps
     mlups = nwet / per_step_s / 1e6
-    alg = W.algorithmic_bytes(wl, storage)
+    per_launch = steps_per_launch(wl, storage)
+    one_step = W.algorithmic_bytes(wl, storage)
+    alg = one_step / (per_launch or 1)
     achieved = alg / per_step_s / 1e9
+    if per_launch is not None and per_launch > 1:
+        traffic = measured_traffic(f"{wl.name}/{name}/K{per_launch}", "march_kernel")
+        traffic = None if traffic is None else traffic / per_launch
+    elif per_launch == 1:
+        traffic = measured_traffic(f"{wl.name}/{name}/R{segments}/o{lat.occupancy()}")
+    else:
+        traffic = None
     return lat, dict(storage=name, mlups=mlups, mlups_all_nodes=wl.nr * wl.nc / per_step_s / 1e6,
-                     ms_per_step=ms / steps, wall_s=wall, alg_bytes_per_step=alg, achieved_gbs=achieved,
-                     frac=achieved / HBM_PEAK_GBS, segments=segments, occupancy=lat.occupancy(),
+                     ms_per_step=ms / steps, wall_s=wall, steps_per_launch=per_launch, alg_bytes_per_step=alg,
+                     achieved_gbs=achieved, frac=achieved / HBM_PEAK_GBS, one_step_gbs=one_step / per_step_s / 1e9,
+                     segments=segments, occupancy=lat.occupancy(),
                      layout="blocked" if lat.layout() == L.LAYOUT_BLOCKED else "planes",
-                     traffic_bytes_per_step=measured_traffic(f"{wl.name}/{name}/R{segments}/o{lat.occupancy()}"))
+                     traffic_bytes_per_step=traffic)
+
+
+def launch_text(r):
+    if r["steps_per_launch"] == 1:
+        return f"launch {r['segments']}, occupancy {r['occupancy'] or 'full'}"
+    return f"{r['steps_per_launch'] or 'several'} steps per launch"
 
 
 def physical_cores():
@@ -295,7 +336,7 @@ def bench_cavity_trt(args, ev):
         lats[s] = lat
         log(f"  cavity_trt4096 {s}: {r['mlups']:.1f} MLUPS, {r['ms_per_step']:.4f} ms/step, "
             f"{r['achieved_gbs']:.0f} GB/s = {100 * r['frac']:.1f}% of 8 TB/s "
-            f"(launch {r['segments']}, occupancy {r['occupancy'] or 'full'})")
+            f"({launch_text(r)})")
     errors = None
     if args.c4_error_steps > 0:
         t1 = time.perf_counter()
@@ -325,36 +366,38 @@ def bench_open(args, ev):
         lat.close()
         log(f"  open8192 {s}: {r['mlups']:.1f} MLUPS, {r['ms_per_step']:.4f} ms/step, "
             f"{r['achieved_gbs']:.0f} GB/s = {100 * r['frac']:.1f}% of 8 TB/s "
-            f"(launch {r['segments']}, occupancy {r['occupancy'] or 'full'}, {r['layout']})")
+            f"({launch_text(r)}, {r['layout']})")
     return dict(workload=wl.name, wet_nodes=wl.wet_count(), collision="BGK", storages=results)
 
 
 def bench_ensemble(args, ev):
-    """Many independent porous lattices of uneven sizes advanced by one
-    persistent launch per step (lbm_batch), HIP-graph step loop, tile shape
-    from the autotuner."""
+    """Many independent porous lattices of uneven sizes advanced together
+    (lbm_batch), 4 steps per launch, HIP-graph step loop; the tile shape and
+    grid of single steps come from the autotuner too."""
     t0 = time.perf_counter()
     wls = W.ensemble(n_samples=args.ensemble_samples)
     wet = sum(w.wet_count() for w in wls)
-    alg = sum(W.algorithmic_bytes(w, L.F32_SHIFTED) for w in wls)
+    per_launch = 4
+    one_step = sum(W.algorithmic_bytes(w, L.F32_SHIFTED) for w in wls)
+    alg = one_step / per_launch
     lats = [w.make_lattice(L.F32_SHIFTED) for w in wls]
     log(f"ensemble: {len(wls)} samples, {wet} wet nodes (built in {time.perf_counter() - t0:.1f}s)")
     b = L.Batch(lats)
     b.step(args.warmup, L.STEP_CHECK)
     seg, blocks, tuned_ms = b.autotune(steps=5)
-    b.step(2 * 32, L.STEP_CHECK)                 # capture and warm the graphs
+    warm_graphs(b.step)
     b.synchronize()
     ms = ev.time_ms(b.stream_handle(), lambda: b.step(args.steps))
     b.step(0, L.STEP_CHECK)
     per_step_s = ms / 1e3 / args.steps
     res = dict(samples=len(wls), wet_nodes=wet, storage="f32", mlups=wet / per_step_s / 1e6,
-               ms_per_step=ms / args.steps, alg_bytes_per_step=alg, achieved_gbs=alg / per_step_s / 1e9,
-               frac=alg / per_step_s / 1e9 / HBM_PEAK_GBS, segments=seg, blocks=blocks, graph_steps=32,
-               traffic_bytes_per_step=(measured_traffic(f"ensemble{len(wls)}/f32/R{seg}", "batch_kernel")
-                                       if blocks == 0 else None))
+               ms_per_step=ms / args.steps, steps_per_launch=per_launch, alg_bytes_per_step=alg,
+               achieved_gbs=alg / per_step_s / 1e9, frac=alg / per_step_s / 1e9 / HBM_PEAK_GBS,
+               one_step_gbs=one_step / per_step_s / 1e9, segments=seg, blocks=blocks)
+    traffic = measured_traffic(f"ensemble{len(wls)}/f32/K{per_launch}", "batch_march_kernel")
+    res["traffic_bytes_per_step"] = None if traffic is None else traffic / per_launch
     log(f"  ensemble f32: {res['mlups']:.1f} MLUPS, {res['ms_per_step']:.4f} ms/step, {res['achieved_gbs']:.0f} GB/s "
-        f"= {100 * res['frac']:.1f}% of 8 TB/s (R={seg}, "
-        f"{'one wave per tile' if blocks == 0 else f'{blocks} persistent work-groups'})")
+        f"= {100 * res['frac']:.1f}% of 8 TB/s ({per_launch} steps per launch)")
     if args.ensemble_check_steps > 0:
         # per-sample Darcy permeability (FP64 GPU reductions) of the FP32
         # ensemble against the FP64 ensemble (the oracle-pinned path)
@@ -441,13 +484,14 @@ def main():
         lat, r = time_storage(wl, s, args.steps, args.warmup, ev)
         r["frac_of_copy"] = r["achieved_gbs"] / ceiling["gbs"]
         if patterns:
-            # the dense pattern of the layout the lattice got
+            # the dense pattern of the layout the lattice got, in the bytes
+            # that the launches move
             pat = "blocked_pull" if lat.layout() == L.LAYOUT_BLOCKED else "ab_pull"
             r["frac_of_pattern"] = r["achieved_gbs"] / patterns[s[:3]][pat]
         results[s] = r
         log(f"  {r['storage']}: {r['mlups']:.1f} MLUPS, {r['ms_per_step']:.4f} ms/step, "
             f"{r['achieved_gbs']:.0f} GB/s = {100 * r['frac']:.1f}% of 8 TB/s, "
-            f"{100 * r['frac_of_copy']:.0f}% of the copy ceiling")
+            f"{100 * r['frac_of_copy']:.0f}% of the copy ceiling ({launch_text(r)})")
         lats[s] = lat
     errors = None
     error_steps = wl.steps if args.error_steps is None else args.error_steps
@@ -488,7 +532,8 @@ def main():
                    "storage": head, "collision": "BGK" if wl.collision == L.BGK else "TRT",
                    "parallelism": "single GPU"},
         "roofline": {"bound": "hbm", "achieved": round(r["achieved_gbs"], 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": round(r["frac"], 4), "traffic": r["traffic_bytes_per_step"]},
+                     "frac": round(r["frac"], 4), "traffic": r["traffic_bytes_per_step"],
+                     "steps_per_launch": r["steps_per_launch"], "one_step_gbs": round(r["one_step_gbs"], 1)},
         "cpu_baseline": cpu,
         "copy_ceiling": {k: (round(v, 1) if isinstance(v, float) else v) for k, v in ceiling.items()},
         "access_patterns": patterns,
