@@ -146,7 +146,6 @@ struct MarchPlan {
     int32_t edge_chunks;     // waves per edge stripe
     int32_t edge_row_waves;  // waves of the edge stripes
     int32_t edge_waves;      // and with the first and last columns of the others, rounded up to whole work-groups
-    int32_t xcd_chunk;       // work-groups per XCD chunk (xcd_remap)
 };
 
 // A batch step: per sample two complete argument sets, args[2 s + p] for

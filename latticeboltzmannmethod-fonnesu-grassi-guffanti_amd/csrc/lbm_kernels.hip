@@ -2067,7 +2067,6 @@ MarchPlan march_plan(const StepArgs &a)
     const int64_t inner = m.stripes - m.top - m.bottom, free_cols = a.g.nc - 2 * (K + 1);
     m.edge_row_waves = (m.top + m.bottom) * m.edge_chunks;
     m.edge_waves = (int32_t)((m.edge_row_waves + 2 * inner + 3) & ~(int64_t)3);
-    m.xcd_chunk = std::max(1, m.stripes / 4);  // about one chunk of columns per XCD
     m.cols = kMarchMinCols;
     if (inner > 0) {
         const int64_t chip = a.cus * 4 * kMarchWaves<T>;

@@ -397,11 +397,20 @@ __device__ __forceinline__ void march_wave(const StepArgs &a, int32_t i0, int32_
 // 116.5 -> 112.0, FP32 69.3 -> 67.5; open 3001 x 5003 FP64 111.7 -> 106.9;
 // porous 8192^2 FP32 261.5 -> 253.8; an ensemble of 60 lattices of up to 256^2
 // FP64 31.2 -> 28.7, of 8 of them FP32 6.6 -> 7.0.
+//
+// The XCDs take the waves in chunks of 8 work-groups: 32 stripes of one chunk
+// of columns.  us a step with about one chunk of columns per XCD -> 8 (three
+// rounds in turn, spread 0.4 %): TRT cavity 4096^2 FP32 78.4 -> 76.6; open
+// 4096^2 FP32 76.7 -> 75.2; channel 1400 x 4000 FP32 26.2 -> 25.8, 512 x 2048
+// FP32 7.9 -> 7.8; porous media and FP64 the same.  4, 6, 10 and 12 lie
+// between.
+constexpr uint32_t kMarchXcdChunk = 8;
+
 template <typename T, int K, bool FUSED, bool PLANES>
 __global__ __launch_bounds__(kBlockRows) void march_kernel(StepArgs a, MarchPlan m)
 {
     constexpr int32_t kRows = 64 - 2 * K;
-    const uint32_t b = xcd_remap(blockIdx.x, (uint32_t)a.nblocks, (uint32_t)m.xcd_chunk);
+    const uint32_t b = xcd_remap(blockIdx.x, (uint32_t)a.nblocks, kMarchXcdChunk);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     int32_t t = (int32_t)b * (kBlockRows / 64) + wave;
