@@ -27,7 +27,7 @@
 // and latency (two waves per SIMD: nine values per level stay in
 // registers).  us a step, before (one step a launch, tuned) -> K = 4 (FP32),
 // 5 (FP64): porous 8192^2 FP32 561 -> 254; open 4096^2 FP64 419 -> 121; TRT
-// cavity 4096^2 FP32 194 -> 78, FP64 416 -> 157; porous 4096^2 FP64 303 -> 112.
+// cavity 4096^2 FP32 194 -> 77, FP64 416 -> 157; porous 4096^2 FP64 303 -> 112.
 // K = 2 / 3 / 4 / 5 on the porous 4096^2 (before FUSED): FP64 211 / 146 / 119
 // / 114, FP32 121 / 78 / 71 / 74: the launch stays near 550 us (FP64) up to K = 4, where
 // memory binds it, and the lanes and columns lost to the window's ends
