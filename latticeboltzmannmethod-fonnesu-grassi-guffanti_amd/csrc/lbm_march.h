@@ -22,7 +22,8 @@
 // perimeter nodes (EDGE); the prescribed values are those of the current
 // step throughout, so the launch is for steps without new values.
 //
-// What bounds it: in FP32 the VALU (busy throughout; 122 instructions per
+// What bounds it: in FP32 the VALU (busy throughout on porous media, 0.85 on
+// unobstructed ones, which load at 4.5 TB/s meanwhile; 122 instructions per
 // level and lane, of which the collision takes 110), in FP64 the VALU at 0.8
 // and latency (two waves per SIMD: nine values per level stay in
 // registers).  us a step, before (one step a launch, tuned) -> K = 4 (FP32),
