@@ -86,6 +86,9 @@ hipError_t copy(int device, void *dst, const void *src, size_t bytes, hipMemcpyK
         }
         g_chunks = (char *)p;
     }
+    // The steps queued before the copy are waited for here, by this thread
+    // alone: a run of many steps would otherwise hold every lane for its length.
+    if (const hipError_t e = hipStreamSynchronize(s); e != hipSuccess) return e;
     hipError_t res[kLanes];
     std::thread threads[kLanes];
     auto lane = [&](int k) {

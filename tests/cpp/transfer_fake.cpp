@@ -1,0 +1,132 @@
+// Host code of the transfers (csrc/lbm_transfer.hip, included as C++) over a
+// stand-in for the HIP runtime: one stream whose copies run when somebody
+// waits for them, so that what is still in flight can be seen.  Run with a
+// scenario's name; exits 0 if it holds.
+#include "../../latticeboltzmannmethod-fonnesu-grassi-guffanti_amd/csrc/lbm_transfer.hip"
+
+#include <cstdio>
+#include <cstdlib>
+#include <string>
+#include <vector>
+
+namespace {
+
+struct Copy {
+    void *dst;
+    const void *src;
+    size_t n;
+};
+
+std::mutex mu;
+std::vector<Copy> queue;         // copies in flight
+bool earlier = false;            // steps queued before the call are still running
+bool lane_waited = false;        // a copy was queued, or waited for, behind those steps
+bool fail_records = false;
+const char *pinned = nullptr;    // page-locked range
+size_t pinned_bytes = 0;
+
+void drain()
+{
+    for (const Copy &c : queue) std::memcpy(c.dst, c.src, c.n);
+    queue.clear();
+    earlier = false;
+}
+
+}  // namespace
+
+extern "C" {
+
+hipError_t hipMemcpyAsync(void *dst, const void *src, size_t n, hipMemcpyKind, hipStream_t)
+{
+    std::lock_guard<std::mutex> lock(mu);
+    lane_waited |= earlier;
+    queue.push_back({dst, src, n});
+    return hipSuccess;
+}
+
+hipError_t hipStreamSynchronize(hipStream_t)
+{
+    std::lock_guard<std::mutex> lock(mu);
+    drain();
+    return hipSuccess;
+}
+
+hipError_t hipEventSynchronize(hipEvent_t)
+{
+    std::lock_guard<std::mutex> lock(mu);
+    lane_waited |= earlier;
+    drain();
+    return hipSuccess;
+}
+
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return fail_records ? hipErrorUnknown : hipSuccess; }
+
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned)
+{
+    *e = (hipEvent_t) new char;
+    return hipSuccess;
+}
+
+hipError_t hipEventDestroy(hipEvent_t e)
+{
+    delete (char *)e;
+    return hipSuccess;
+}
+
+hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipGetLastError(void) { return hipSuccess; }
+
+hipError_t hipHostMalloc(void **p, size_t n, unsigned)
+{
+    *p = std::malloc(n);
+    return hipSuccess;
+}
+
+hipError_t hipHostFree(void *p)
+{
+    std::free(p);
+    return hipSuccess;
+}
+
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t *at, const void *p)
+{
+    *at = hipPointerAttribute_t{};
+    const char *c = (const char *)p;
+    const bool in = c >= pinned && c < pinned + pinned_bytes;
+    at->type = in ? hipMemoryTypeHost : hipMemoryTypeUnregistered;
+    at->devicePointer = in ? (void *)p : nullptr;
+    return hipSuccess;
+}
+
+}  // extern "C"
+
+int main(int argc, char **argv)
+{
+    const std::string what = argc > 1 ? argv[1] : "";
+    const size_t n = (size_t)13 << 20;  // several rounds of the chunks and a remainder
+    std::vector<char> a(n + 123), b(n + 123, 0);
+    for (size_t k = 0; k < a.size(); ++k) a[k] = (char)(k * 2654435761u >> 13);
+    lbm::transfer_retain();
+    int bad = 0;
+    auto require = [&](bool ok, const char *text) {
+        if (!ok) {
+            std::printf("%s: %s\n", what.c_str(), text);
+            bad = 1;
+        }
+    };
+    if (what == "bytes") {
+        require(lbm::copy_to_host(0, b.data(), a.data(), a.size(), nullptr) == hipSuccess, "down failed");
+        require(a == b, "down differs");
+        std::fill(b.begin(), b.end(), 0);
+        require(lbm::copy_to_device(0, b.data(), a.data(), a.size(), nullptr) == hipSuccess, "up failed");
+        require(a == b, "up differs");
+    } else if (what == "earlier") {
+        earlier = true;
+        require(lbm::copy_to_host(0, b.data(), a.data(), a.size(), nullptr) == hipSuccess, "down failed");
+        require(!lane_waited, "the lanes waited for the stream's earlier work");
+    } else {
+        require(false, "unknown scenario");
+    }
+    lbm::transfer_release();
+    return bad;
+}
