@@ -102,9 +102,12 @@ hipError_t copy(int device, void *dst, const void *src, size_t bytes, hipMemcpyK
     lane(0);
     for (int k = started; k < kLanes; ++k) lane(k);
     for (int k = 1; k < started; ++k) threads[k].join();
+    // A lane that failed may have left its chunk, or its caller's memory, to
+    // a copy in flight: all of them end before the chunks are given back.
+    const hipError_t end = hipStreamSynchronize(s);
     for (const hipError_t e : res)
         if (e != hipSuccess) return e;
-    return hipStreamSynchronize(s);
+    return end;
 }
 
 }  // namespace

@@ -124,6 +124,16 @@ int main(int argc, char **argv)
         earlier = true;
         require(lbm::copy_to_host(0, b.data(), a.data(), a.size(), nullptr) == hipSuccess, "down failed");
         require(!lane_waited, "the lanes waited for the stream's earlier work");
+    } else if (what == "failure") {
+        for (const bool up : {false, true}) {
+            fail_records = true;
+            const hipError_t e = up ? lbm::copy_to_device(0, b.data(), a.data(), a.size(), nullptr)
+                                    : lbm::copy_to_host(0, b.data(), a.data(), a.size(), nullptr);
+            require(e != hipSuccess, "the failure was not reported");
+            require(queue.empty(), "copies to or from the chunks still in flight after a failed lane");
+            fail_records = false;
+            drain();
+        }
     } else {
         require(false, "unknown scenario");
     }

@@ -37,3 +37,9 @@ def test_lanes_start_behind_earlier_work(driver):
     """The threads start once the stream has reached the copy: they do not
     wait for the steps queued before it."""
     _holds(driver, "earlier")
+
+
+def test_failed_lane_leaves_nothing_in_flight(driver):
+    """After a lane has failed, the copies of all lanes are waited for before
+    the chunks can be taken by another call or freed."""
+    _holds(driver, "failure")
