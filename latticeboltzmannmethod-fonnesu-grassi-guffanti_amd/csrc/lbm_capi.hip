@@ -1321,7 +1321,8 @@ int lbm_download_macro_async(lbm_ctx *c, double *rho, double *u, int64_t *ticket
     // them over the link.  Two copies on another stream took 55 us for 40 x
     // 96 nodes, this 17.
     if (3 * N * sizeof(double) <= kKernelCopyBytes) {
-        double *dr = rho ? (double *)device_view(rho) : nullptr, *du = u ? (double *)device_view(u) : nullptr;
+        double *dr = rho ? (double *)device_view(rho, N * sizeof(double)) : nullptr;
+        double *du = u ? (double *)device_view(u, 2 * N * sizeof(double)) : nullptr;
         if ((!rho || dr) && (!u || du)) {
             HIP_TRY(launch_copy_fields(m, (int64_t)N, dr, du, c->stream));
             return new_ticket(c, c->stream, ticket);

@@ -14,8 +14,9 @@ namespace lbm {
 hipError_t copy_to_host(int device, void *dst, const void *src, size_t bytes, hipStream_t s);
 hipError_t copy_to_device(int device, void *dst, const void *src, size_t bytes, hipStream_t s);
 
-// The device's view of page-locked host memory (nullptr for other memory).
-void *device_view(const void *host);
+// The device's view of `bytes` of page-locked host memory (nullptr unless the
+// first and the last byte lie in one).
+void *device_view(const void *host, size_t bytes);
 
 // Contexts alive: the page-locked chunks the copies go through are shared by
 // all of them and freed with the last one.

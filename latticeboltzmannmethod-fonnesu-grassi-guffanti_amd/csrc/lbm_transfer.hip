@@ -122,14 +122,28 @@ hipError_t copy_to_device(int device, void *dst, const void *src, size_t bytes, 
     return copy(device, dst, src, bytes, hipMemcpyHostToDevice, s);
 }
 
-void *device_view(const void *host)
+namespace {
+
+// Where the device sees one byte of page-locked host memory.
+char *device_byte(const char *host)
 {
     hipPointerAttribute_t at{};
     if (hipPointerGetAttributes(&at, host) != hipSuccess) {
         (void)hipGetLastError();
         return nullptr;
     }
-    return at.type == hipMemoryTypeHost ? at.devicePointer : nullptr;
+    return at.type == hipMemoryTypeHost ? (char *)at.devicePointer : nullptr;
+}
+
+}  // namespace
+
+void *device_view(const void *host, size_t bytes)
+{
+    // Only a part of the caller's memory may be page-locked (hipHostRegister):
+    // a kernel that wrote past it would fault, where a copy is an error.
+    char *first = device_byte((const char *)host);
+    if (!first || bytes == 0) return first;
+    return device_byte((const char *)host + bytes - 1) == first + bytes - 1 ? first : nullptr;
 }
 
 void transfer_retain()

@@ -134,6 +134,14 @@ int main(int argc, char **argv)
             fail_records = false;
             drain();
         }
+    } else if (what == "view") {
+        pinned = a.data();
+        pinned_bytes = 4096;
+        require(lbm::device_view(a.data(), 4096) == a.data(), "page-locked memory has no view");
+        require(lbm::device_view(a.data() + 8, 8) == a.data() + 8, "a part of it has no view");
+        require(!lbm::device_view(a.data(), 4097), "memory whose end is pageable has a view");
+        require(!lbm::device_view(a.data() + 4088, 16), "memory whose second half is pageable has a view");
+        require(!lbm::device_view(b.data(), 8), "pageable memory has a view");
     } else {
         require(false, "unknown scenario");
     }

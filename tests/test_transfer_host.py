@@ -43,3 +43,8 @@ def test_failed_lane_leaves_nothing_in_flight(driver):
     """After a lane has failed, the copies of all lanes are waited for before
     the chunks can be taken by another call or freed."""
     _holds(driver, "failure")
+
+
+def test_device_view_covers_the_whole_range(driver):
+    """A kernel may write host memory only if all of it is page-locked."""
+    _holds(driver, "view")
