@@ -174,19 +174,6 @@ def random_state(wl):
     return _RANDOM_STATE[wl.name]
 
 
-def steps_per_launch(wl, storage):
-    """Time steps per launch of the library's rule for lattices beyond the
-    tiles' size (300,000 nodes): marching waves take 4 steps of FP64 and
-    FP32 lattices, 5 of FP64 lattices of at least 2^22 nodes; FP16 lattices
-    take one.  None for smaller lattices, whose tiles take 4 to 9 steps."""
-    nodes = wl.nr * wl.nc
-    if nodes < (3 << 19 if storage == L.F16_SHIFTED else 300000):
-        return None
-    if storage == L.F16_SHIFTED:
-        return 1
-    return 5 if storage == L.F64 and nodes >= 1 << 22 else 4
-
-
 def warm_graphs(step):
     """Captures the step graphs of both buffer parities (a graph holds at
     most 72 steps)."""
@@ -213,17 +200,15 @@ def time_storage(wl, name, steps, warmup, ev):
     nwet = wl.wet_count()
     per_step_s = ms / 1e3 / steps
     mlups = nwet / per_step_s / 1e6
-    per_launch = steps_per_launch(wl, storage)
+    per_launch = lat.steps_per_launch()
     one_step = W.algorithmic_bytes(wl, storage)
-    alg = one_step / (per_launch or 1)
+    alg = one_step / per_launch
     achieved = alg / per_step_s / 1e9
-    if per_launch is not None and per_launch > 1:
+    if per_launch > 1:
         traffic = measured_traffic(f"{wl.name}/{name}/K{per_launch}", "march_kernel")
         traffic = None if traffic is None else traffic / per_launch
-    elif per_launch == 1:
-        traffic = measured_traffic(f"{wl.name}/{name}/R{segments}/o{lat.occupancy()}")
     else:
-        traffic = None
+        traffic = measured_traffic(f"{wl.name}/{name}/R{segments}/o{lat.occupancy()}")
     return lat, dict(storage=name, mlups=mlups, mlups_all_nodes=wl.nr * wl.nc / per_step_s / 1e6,
                      ms_per_step=ms / steps, wall_s=wall, steps_per_launch=per_launch, alg_bytes_per_step=alg,
                      achieved_gbs=achieved, frac=achieved / HBM_PEAK_GBS, one_step_gbs=one_step / per_step_s / 1e9,
@@ -235,7 +220,7 @@ def time_storage(wl, name, steps, warmup, ev):
 def launch_text(r):
     if r["steps_per_launch"] == 1:
         return f"launch {r['segments']}, occupancy {r['occupancy'] or 'full'}"
-    return f"{r['steps_per_launch'] or 'several'} steps per launch"
+    return f"{r['steps_per_launch']} steps per launch"
 
 
 def physical_cores():
@@ -372,14 +357,12 @@ def bench_open(args, ev):
 
 def bench_ensemble(args, ev):
     """Many independent porous lattices of uneven sizes advanced together
-    (lbm_batch), 4 steps per launch, HIP-graph step loop; the tile shape and
-    grid of single steps come from the autotuner too."""
+    (lbm_batch), HIP-graph step loop; the steps per launch, and the tile shape
+    and grid of single steps, come from the autotuner."""
     t0 = time.perf_counter()
     wls = W.ensemble(n_samples=args.ensemble_samples)
     wet = sum(w.wet_count() for w in wls)
-    per_launch = 4
     one_step = sum(W.algorithmic_bytes(w, L.F32_SHIFTED) for w in wls)
-    alg = one_step / per_launch
     lats = [w.make_lattice(L.F32_SHIFTED) for w in wls]
     log(f"ensemble: {len(wls)} samples, {wet} wet nodes (built in {time.perf_counter() - t0:.1f}s)")
     b = L.Batch(lats)
@@ -389,6 +372,8 @@ def bench_ensemble(args, ev):
     b.synchronize()
     ms = ev.time_ms(b.stream_handle(), lambda: b.step(args.steps))
     b.step(0, L.STEP_CHECK)
+    per_launch = b.steps_per_launch()
+    alg = one_step / per_launch
     per_step_s = ms / 1e3 / args.steps
     res = dict(samples=len(wls), wet_nodes=wet, storage="f32", mlups=wet / per_step_s / 1e6,
                ms_per_step=ms / args.steps, steps_per_launch=per_launch, alg_bytes_per_step=alg,

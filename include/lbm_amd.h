@@ -303,13 +303,28 @@ int lbm_get_scale(lbm_ctx *ctx, double *scale);
  * Results are the same bits for every shape.  With 0 (the default), steps
  * run several to a launch where the lattice allows it (small lattices;
  * larger ones in FP64 and FP32 storage); a shape set here is a launch of one
- * step.  No counterpart in the reference (a tuning knob of
- * this engine). */
+ * step.  lbm_get_launch reports the shape of single steps, which also take
+ * the steps that several to a launch leave over.  No counterpart in the
+ * reference (a tuning knob of this engine). */
 enum { LBM_LAUNCH_WET_RUNS = 64, LBM_LAUNCH_RUN_TABLE = 65 };
 int lbm_set_launch(lbm_ctx *ctx, int32_t segments);
 int lbm_get_launch(lbm_ctx *ctx, int32_t *segments);
 
-/* Occupancy of the step kernels: at most `groups_per_cu` work-groups (of
+/* Time steps per launch: at most `steps` (as many as the lattice's kernels
+ * take: 4 to 9 for small lattices, 4 or 5 for larger ones in FP64 and FP32
+ * storage, 1 otherwise), 1 for single steps, or 0 for the library's choice
+ * by size and shape, the default.  The value read is the number that a run
+ * of many steps takes per launch now; lbm_set_launch (0: the library's
+ * choice, a shape: 1) and lbm_autotune (what it measured fastest) set it
+ * too.  A tuned choice is kept by reading lbm_get_launch,
+ * lbm_get_occupancy and lbm_get_steps_per_launch, and brought back by
+ * setting them in that order.  Results are the same bits for every value.
+ * No counterpart in the reference. */
+int lbm_set_steps_per_launch(lbm_ctx *ctx, int32_t steps);
+int lbm_get_steps_per_launch(lbm_ctx *ctx, int32_t *steps);
+
+/* Occupancy of the kernels that take one step (launches of several steps
+ * run as many work-groups as fit): at most `groups_per_cu` work-groups (of
  * four waves) per compute unit, 2 to 7, or 0 for as many as their
  * registers allow (8 for most shapes).  Fewer waves in flight can move more
  * bytes per second.  Until set or tuned it is 7 (FP32, FP16 storage) or 5
@@ -325,8 +340,9 @@ int lbm_get_occupancy(lbm_ctx *ctx, int32_t *groups_per_cu);
  * launches (every launch rewrites the spare buffer from the
  * current state, so the state does not change) and keeps the fastest
  * pair for single steps, and several steps per launch if they are faster
- * still.  Reports the shape of the single steps and the time per step
- * (outputs may be NULL); lbm_get_occupancy reports the occupancy.  LBM_ERR_STATE for a context
+ * still.  Reports the shape of the single steps and the time per step of
+ * the choice (outputs may be NULL); lbm_get_occupancy and
+ * lbm_get_steps_per_launch report the rest of the choice.  LBM_ERR_STATE for a context
  * that belongs to an ensemble (the ensemble has its own,
  * lbm_batch_autotune) and for a lattice with partially saturated
  * bounce-back (it has one launch shape).  No counterpart in the
@@ -369,6 +385,12 @@ int lbm_batch_destroy(lbm_batch *batch);
  * table (as lbm_set_launch for one lattice). */
 int lbm_batch_set_launch(lbm_batch *batch, int32_t segments, int64_t blocks);
 int lbm_batch_get_launch(lbm_batch *batch, int32_t *segments, int64_t *blocks);
+
+/* Time steps per launch of the ensemble, as lbm_set_steps_per_launch: 0 =
+ * the library's choice (the default), 1 = single steps (what
+ * lbm_batch_set_launch sets), 4 and more = 4 where all samples allow it. */
+int lbm_batch_set_steps_per_launch(lbm_batch *batch, int32_t steps);
+int lbm_batch_get_steps_per_launch(lbm_batch *batch, int32_t *steps);
 
 /* Autotuner: times every candidate tile shape and grid (one wave per tile,
  * or 2, 4, 8, 16 persistent work-groups per compute unit; and wet-run

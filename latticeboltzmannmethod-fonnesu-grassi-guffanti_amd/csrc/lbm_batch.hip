@@ -65,10 +65,12 @@ struct lbm_batch {
     // wet-run table (launch shape kRunLaunch): every sample's runs
     int32_t *d_runs = nullptr;
     int64_t nruns = 0;
-    // marching waves (several steps per launch); march: they are in use
+    // marching waves (several steps per launch); march: they are in use,
+    // unless max_steps (steps per launch at most, 0 = the rule) forbids them
     int32_t *d_marches = nullptr;
     int64_t nmarches = 0;
     bool march = false;
+    int32_t max_steps = 0;
     bool fused = false;
     // "first" = each sample's arguments as lbm_step would build them for its
     // next step; "steady" = the same with the previous prescribed values set
@@ -222,6 +224,14 @@ int build_runs(lbm_batch *b)
     return LBM_OK;
 }
 
+void set_max_steps(lbm_batch *b, int32_t steps)
+{
+    const bool march = b->nmarches > 0 && (steps == 0 || steps >= kBatchMarchSteps);
+    if (march != b->march) drop_graphs(b);
+    b->march = march;
+    b->max_steps = steps;
+}
+
 // Table of the marching waves.  Chunks of columns: the longest of these
 // that fill three quarters of the chip's waves (each wave recomputes the 2 K
 // columns at its ends), and the shortest for ensembles that never do.  us a
@@ -247,8 +257,8 @@ int build_marches(lbm_batch *b)
     b->nmarches = (int64_t)table.size() / 4;
     HIP_TRY(hipMalloc(&b->d_marches, table.size() * sizeof(int32_t)));
     HIP_TRY(hipMemcpy(b->d_marches, table.data(), table.size() * sizeof(int32_t), hipMemcpyHostToDevice));
-    b->march = true;
     b->fused = nodes >= kBatchFusedNodes;
+    set_max_steps(b, 0);
     return LBM_OK;
 }
 
@@ -442,10 +452,26 @@ int lbm_batch_set_launch(lbm_batch *b, int32_t segments, int64_t blocks)
         int r = build_tiles(b, tiles_R);
         if (r) return r;
     }
-    if (nb != b->blocks || segments != b->R || b->march) drop_graphs(b);
+    if (nb != b->blocks || segments != b->R) drop_graphs(b);
     b->R = segments;
     b->blocks = nb;
-    b->march = false;
+    set_max_steps(b, 1);
+    return LBM_OK;
+}
+
+int lbm_batch_set_steps_per_launch(lbm_batch *b, int32_t steps)
+{
+    if (!b) return fail(LBM_ERR_INVALID, "null batch");
+    if (steps < 0) return fail(LBM_ERR_INVALID, "steps must be >= 0");
+    HIP_TRY(hipSetDevice(b->device));
+    set_max_steps(b, steps);
+    return LBM_OK;
+}
+
+int lbm_batch_get_steps_per_launch(lbm_batch *b, int32_t *steps)
+{
+    if (!b || !steps) return fail(LBM_ERR_INVALID, "null argument");
+    *steps = b->march ? kBatchMarchSteps : 1;
     return LBM_OK;
 }
 
@@ -498,7 +524,7 @@ int lbm_batch_autotune(lbm_batch *b, int32_t steps, int32_t *segments, int64_t *
     if (r) return r;
     b->R = best_R;
     b->blocks = best_nb;
-    b->march = false;
+    set_max_steps(b, 1);
     if (b->nmarches > 0) {  // several steps per launch against the best single step
         const BatchArgs ba = batch_args(b, b->steady, b->phase);
         HIP_TRY(launch_batch_march(b->storage, ba, b->stream));
@@ -510,7 +536,7 @@ int lbm_batch_autotune(lbm_batch *b, int32_t steps, int32_t *segments, int64_t *
         HIP_TRY(hipEventElapsedTime(&ms, b->t0, b->t1));
         if (ms / kBatchMarchSteps < best) {
             best = ms / kBatchMarchSteps;
-            b->march = true;
+            set_max_steps(b, kBatchMarchSteps);
         }
     }
     drop_graphs(b);

@@ -135,10 +135,11 @@ struct Launching {
 
 Launching launching(const lbm_ctx *c)
 {
-    if (c->multi) {
+    const int32_t most = c->max_steps == 0 ? INT32_MAX : c->max_steps;
+    if (most > 1) {
         const StepArgs a = make_args(c);
-        if (const int32_t k = tile_steps(c->storage, a)) return {Launching::kTile, k};
-        if (const int32_t k = march_steps(c->storage, a)) return {Launching::kMarch, k};
+        if (const int32_t k = tile_steps(c->storage, a)) return {Launching::kTile, std::min(k, most)};
+        if (const int32_t k = march_steps(c->storage, a)) return {Launching::kMarch, std::min(k, most)};
     }
     return {Launching::kSingle, 1};
 }
@@ -1168,8 +1169,25 @@ int lbm_set_launch(lbm_ctx *c, int32_t segments)
         if (r) return r;
     }
     c->segments = segments;
-    c->multi = segments == 0;
+    c->max_steps = segments == 0 ? 0 : 1;
     drop_graphs(c);
+    return LBM_OK;
+}
+
+int lbm_set_steps_per_launch(lbm_ctx *c, int32_t steps)
+{
+    if (!c) return fail(LBM_ERR_INVALID, "null context");
+    if (steps < 0) return fail(LBM_ERR_INVALID, "steps must be >= 0");
+    c->max_steps = steps;
+    drop_graphs(c);
+    return LBM_OK;
+}
+
+int lbm_get_steps_per_launch(lbm_ctx *c, int32_t *steps)
+{
+    if (!c || !steps) return fail(LBM_ERR_INVALID, "null argument");
+    if (!c->has_geom) return fail(LBM_ERR_STATE, "no geometry");
+    *steps = launching(c).steps;
     return LBM_OK;
 }
 
@@ -1255,11 +1273,11 @@ int lbm_autotune(lbm_ctx *c, int32_t steps, int32_t *segments, double *ms_per_st
         }
     }
     // several steps per launch against the best single step
-    const bool was_multi = c->multi;
-    c->multi = true;
+    const int32_t was = c->max_steps;
+    c->max_steps = INT32_MAX;
     const Launching how = launching(c);
-    c->multi = was_multi;
-    bool multi = false;
+    c->max_steps = was;
+    int32_t tuned = 1;
     if (how.kind != Launching::kSingle) {
         auto launch = [&] {
             return how.kind == Launching::kTile ? launch_tile(c->storage, how.steps, a, c->stream)
@@ -1274,7 +1292,7 @@ int lbm_autotune(lbm_ctx *c, int32_t steps, int32_t *segments, double *ms_per_st
         if (err == hipSuccess) err = hipEventElapsedTime(&ms, t0, t1);
         if (err == hipSuccess && ms / (float)how.steps < best) {
             best = ms / (float)how.steps;
-            multi = true;
+            tuned = how.steps;
         }
     }
     (void)hipEventDestroy(t0);
@@ -1282,7 +1300,7 @@ int lbm_autotune(lbm_ctx *c, int32_t steps, int32_t *segments, double *ms_per_st
     if (err != hipSuccess) return fail(LBM_ERR_HIP, "autotune: %s", hipGetErrorString(err));
     c->segments = best_R;
     c->occupancy = best_occ;
-    c->multi = multi;
+    c->max_steps = tuned;
     drop_graphs(c);
     if (segments) *segments = best_R;
     if (ms_per_step) *ms_per_step = best / steps;

@@ -118,9 +118,9 @@ struct lbm_ctx {
     struct lbm_batch *batch = nullptr;
     // 64-row segments per wave of the step kernel (0 = default_segments)
     int32_t segments = 0;
-    // several steps per launch where nothing asks for single ones: off while
-    // a shape is set by hand, or where the autotuner measured it slower
-    bool multi = true;
+    // steps per launch at most: 0 = the library's rule, 1 = single steps (a
+    // shape set by hand, or the autotuner measured several slower)
+    int32_t max_steps = 0;
     int32_t cus = 256;  // compute units of the device
     // partially saturated bounce-back of the wet obstacles (lbm_set_partial_bounce_back)
     bool psbb = false;

@@ -48,9 +48,9 @@ EXPORTED = [
     "lbm_get_stream",
     "lbm_get_scale", "lbm_geometry_cavity", "lbm_geometry_channel", "lbm_geometry_add_disc",
     "lbm_geometry_porous", "lbm_set_launch", "lbm_get_launch", "lbm_set_occupancy", "lbm_get_occupancy",
-    "lbm_get_layout",
+    "lbm_set_steps_per_launch", "lbm_get_steps_per_launch", "lbm_get_layout",
     "lbm_autotune", "lbm_batch_create", "lbm_batch_destroy", "lbm_batch_set_launch", "lbm_batch_get_launch",
-    "lbm_batch_autotune", "lbm_batch_step", "lbm_batch_reduce", "lbm_batch_info", "lbm_batch_get_stream",
+    "lbm_batch_set_steps_per_launch", "lbm_batch_get_steps_per_launch", "lbm_batch_autotune", "lbm_batch_step", "lbm_batch_reduce", "lbm_batch_info", "lbm_batch_get_stream",
     "lbm_batch_synchronize", "lbm_copy_bandwidth", "lbm_pattern_bandwidth",
 ]
 
@@ -124,6 +124,8 @@ def lib():
                                     i64p],
             "lbm_set_launch": [vp, C.c_int32],
             "lbm_get_launch": [vp, i32p],
+            "lbm_set_steps_per_launch": [vp, C.c_int32],
+            "lbm_get_steps_per_launch": [vp, i32p],
             "lbm_set_occupancy": [vp, C.c_int32],
             "lbm_get_layout": [vp, i32p],
             "lbm_get_occupancy": [vp, i32p],
@@ -132,6 +134,8 @@ def lib():
             "lbm_batch_destroy": [vp],
             "lbm_batch_set_launch": [vp, C.c_int32, C.c_int64],
             "lbm_batch_get_launch": [vp, i32p, i64p],
+            "lbm_batch_set_steps_per_launch": [vp, C.c_int32],
+            "lbm_batch_get_steps_per_launch": [vp, i32p],
             "lbm_batch_autotune": [vp, C.c_int32, i32p, i64p, dp],
             "lbm_batch_step": [vp, C.c_int64, C.c_uint32],
             "lbm_batch_reduce": [vp, dp],
@@ -379,6 +383,16 @@ class Lattice:
         _check(lib().lbm_get_launch(self._h, C.byref(r)))
         return r.value
 
+    def set_steps_per_launch(self, steps):
+        """At most that many time steps per launch, 1 = single steps, 0 = the
+        library's choice (lbm_set_steps_per_launch)."""
+        _check(lib().lbm_set_steps_per_launch(self._h, steps))
+
+    def steps_per_launch(self):
+        r = C.c_int32(0)
+        _check(lib().lbm_get_steps_per_launch(self._h, C.byref(r)))
+        return r.value
+
     def layout(self):
         """LAYOUT_BLOCKED or LAYOUT_PLANES (lbm_get_layout)."""
         r = C.c_int32(0)
@@ -386,8 +400,8 @@ class Lattice:
         return r.value
 
     def set_occupancy(self, groups_per_cu):
-        """Work-groups per compute unit of the step kernels (2..7), 0 = no
-        limit; until set or tuned, the storage format's default (occupancy())."""
+        """Work-groups per compute unit of the kernels that take one step
+        (2..7), 0 = no limit; until set or tuned, the storage format's default (occupancy())."""
         _check(lib().lbm_set_occupancy(self._h, groups_per_cu))
 
     def occupancy(self):
@@ -396,8 +410,9 @@ class Lattice:
         return r.value
 
     def autotune(self, steps=5):
-        """Fastest launch shape and occupancy (lbm_autotune); returns the shape
-        and its ms per step (occupancy() gives the occupancy)."""
+        """Fastest launch (lbm_autotune); returns the shape of single steps and
+        the choice's ms per step (occupancy() and steps_per_launch() give the
+        rest of the choice)."""
         r, ms = C.c_int32(0), C.c_double(0)
         _check(lib().lbm_autotune(self._h, steps, C.byref(r), C.byref(ms)))
         return r.value, ms.value
@@ -453,6 +468,16 @@ class Batch:
         r, b = C.c_int32(0), C.c_int64(0)
         _check(lib().lbm_batch_get_launch(self._h, C.byref(r), C.byref(b)))
         return r.value, b.value
+
+    def set_steps_per_launch(self, steps):
+        """1 = single steps, 4 = four per launch where the samples allow it, 0 =
+        the library's choice (lbm_batch_set_steps_per_launch)."""
+        _check(lib().lbm_batch_set_steps_per_launch(self._h, steps))
+
+    def steps_per_launch(self):
+        r = C.c_int32(0)
+        _check(lib().lbm_batch_get_steps_per_launch(self._h, C.byref(r)))
+        return r.value
 
     def autotune(self, steps=5):
         r, b, ms = C.c_int32(0), C.c_int64(0), C.c_double(0)

@@ -1,0 +1,86 @@
+"""Steps per launch: what is in use can be read, set by hand and brought back,
+for a lattice and for an ensemble; the results keep their bits."""
+import numpy as np
+import pytest
+
+import lbm_amd as L
+from test_gpu_march import POLICIES, make, random_class, state
+
+pytestmark = pytest.mark.gpu
+
+# tiles, marching waves of 4 steps, and of 5 (FP64)
+SIZES = [(129, 130), (560, 541), (2060, 2040)]
+
+
+@pytest.mark.parametrize("storage", [L.F64, L.F32_SHIFTED])
+@pytest.mark.parametrize("nr,nc", SIZES)
+def test_lattice(nr, nc, storage):
+    rng = np.random.default_rng(nr)
+    cls = random_class(rng, nr, nc, 0.1)
+    p0 = state(rng, nc, nr)
+    lat = make(cls, np.random.default_rng(1), storage, L.BGK, POLICIES[:2])
+    default = lat.steps_per_launch()
+    assert default > 1
+    lat.set_launch(2)
+    assert lat.steps_per_launch() == 1
+    lat.set_launch(0)
+    assert lat.steps_per_launch() == default
+    with pytest.raises(L.LbmError):
+        lat.set_steps_per_launch(-1)
+    want = None
+    for k in (1, 2, 3, 4, default, 100, 0):
+        lat.set_steps_per_launch(k)
+        assert lat.steps_per_launch() == min(k or default, default)
+        lat.upload_populations(p0)
+        lat.step(93)
+        p = lat.populations()
+        want = p if want is None else want
+        assert np.array_equal(p, want), k
+    # a tuned choice, on another lattice of the same geometry
+    lat.autotune(2)
+    tuned = lat.launch(), lat.occupancy(), lat.steps_per_launch()
+    other = make(cls, np.random.default_rng(1), storage, L.BGK, POLICIES[:2])
+    other.set_launch(tuned[0])
+    other.set_occupancy(tuned[1])
+    other.set_steps_per_launch(tuned[2])
+    assert (other.launch(), other.occupancy(), other.steps_per_launch()) == tuned
+    other.upload_populations(p0)
+    other.step(93)
+    assert np.array_equal(other.populations(), want)
+    lat.close()
+    other.close()
+
+
+def test_ensemble():
+    rng = np.random.default_rng(3)
+    shapes = [(300, 200), (129, 700), (200, 250)]
+    lats = [make(random_class(rng, nr, nc, 0.1), np.random.default_rng(k), L.F32_SHIFTED, L.TRT, POLICIES[:2])
+            for k, (nr, nc) in enumerate(shapes)]
+    states = [state(rng, nc, nr) for nr, nc in shapes]
+    with L.Batch(lats) as b:
+        default = b.steps_per_launch()
+        segments, blocks = b.launch()
+        b.set_launch(segments, blocks)
+        assert b.steps_per_launch() == 1
+        out = []
+        for k, n in ((1, 1), (3, 1), (4, 4), (100, 4), (0, default)):
+            b.set_steps_per_launch(k)
+            assert b.steps_per_launch() == n
+            for lat, p in zip(lats, states):
+                lat.upload_populations(p)
+            b.step(45)
+            out.append([lat.populations() for lat in lats])
+        for x in out[1:]:
+            assert all(np.array_equal(p, q) for p, q in zip(out[0], x))
+        b.set_launch(segments, blocks)
+        b.set_steps_per_launch(0)
+        assert b.steps_per_launch() == default
+    for lat in lats:
+        lat.close()
+
+
+def test_without_geometry_it_is_an_error():
+    import ctypes as C
+    with L.Lattice(L.geometry_channel(40, 96), storage=L.F16_SHIFTED) as lat:
+        assert lat.steps_per_launch() > 1
+    assert L.lib().lbm_get_steps_per_launch(None, C.byref(C.c_int32())) == L.ERR_INVALID
