@@ -241,17 +241,17 @@ void set_max_steps(lbm_batch *b, int32_t steps)
 int build_marches(lbm_batch *b)
 {
     int64_t nodes = 0;
-    std::vector<StepArgs> args;
+    std::vector<LatticeShape> shapes;
     for (const lbm_ctx *c : b->samples) {
         if (c->storage == kF16 || !c->blocked) return LBM_OK;
         nodes += c->nr * c->nc;
-        args.push_back(make_args(c));
+        shapes.push_back(shape_of(c));
     }
     if (nodes < kMarchMinNodes) return LBM_OK;
     std::vector<int32_t> table;
     const int64_t chip = (int64_t)b->cus * 4 * (b->storage == kF64 ? 2 : 3);
     for (int32_t cols : {64, 32, 16, 12, 8, 6}) {
-        march_table(args.data(), (int64_t)args.size(), cols, table);
+        march_table(shapes.data(), (int64_t)shapes.size(), kBatchMarchSteps, cols, table);
         if ((int64_t)table.size() / 4 >= chip * 3 / 4) break;
     }
     b->nmarches = (int64_t)table.size() / 4;

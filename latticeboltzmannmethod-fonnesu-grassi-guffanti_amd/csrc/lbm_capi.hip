@@ -96,9 +96,6 @@ StepArgs make_args(const lbm_ctx *c)
     a.nruns = c->nruns;
     a.perim = c->d_perim;
     a.nperim = c->nperim;
-    a.wet_top = c->wet_top;
-    a.wet_bottom = c->wet_bottom;
-    a.cus = c->cus;
     a.trun = c->d_trun;
     a.tlane = c->d_tlane;
     a.psbb = c->psbb ? 1 : 0;
@@ -107,6 +104,11 @@ StepArgs make_args(const lbm_ctx *c)
     a.ps_b = c->d_ps_b;
     set_input(c, a, c->cur);
     return a;
+}
+
+LatticeShape shape_of(const lbm_ctx *c)
+{
+    return {c->storage, c->psbb, c->nr, c->nc, c->wet_top, c->wet_bottom, c->cus};
 }
 
 int flush_bc(lbm_ctx *c)
@@ -137,9 +139,9 @@ Launching launching(const lbm_ctx *c)
 {
     const int32_t most = c->max_steps == 0 ? INT32_MAX : c->max_steps;
     if (most > 1) {
-        const StepArgs a = make_args(c);
-        if (const int32_t k = tile_steps(c->storage, a)) return {Launching::kTile, std::min(k, most)};
-        if (const int32_t k = march_steps(c->storage, a)) return {Launching::kMarch, std::min(k, most)};
+        const LatticeShape a = shape_of(c);
+        if (const int32_t k = tile_shape(a).halo) return {Launching::kTile, std::min(k, most)};
+        if (const int32_t k = march_steps(a)) return {Launching::kMarch, std::min(k, most)};
     }
     return {Launching::kSingle, 1};
 }
@@ -167,8 +169,8 @@ hipError_t launch_steps(const lbm_ctx *c, Launching::Kind kind, int in, int32_t 
         a.bc_new = c->d_bc[c->bc_cur];
     }
     switch (kind) {
-    case Launching::kTile: return launch_tile(c->storage, k, a, c->stream);
-    case Launching::kMarch: return launch_march(c->storage, k, a, c->stream);
+    case Launching::kTile: return launch_tile(c->storage, k, a, tile_shape(shape_of(c)), c->stream);
+    case Launching::kMarch: return launch_march(c->storage, k, a, march_plan(shape_of(c), k), c->stream);
     default: return launch_step(c->storage, true, a, c->stream, c->segments);
     }
 }
@@ -1280,8 +1282,9 @@ int lbm_autotune(lbm_ctx *c, int32_t steps, int32_t *segments, double *ms_per_st
     int32_t tuned = 1;
     if (how.kind != Launching::kSingle) {
         auto launch = [&] {
-            return how.kind == Launching::kTile ? launch_tile(c->storage, how.steps, a, c->stream)
-                                                : launch_march(c->storage, how.steps, a, c->stream);
+            return how.kind == Launching::kTile
+                       ? launch_tile(c->storage, how.steps, a, tile_shape(shape_of(c)), c->stream)
+                       : launch_march(c->storage, how.steps, a, march_plan(shape_of(c), how.steps), c->stream);
         };
         if (err == hipSuccess) err = launch();
         if (err == hipSuccess) err = hipEventRecord(t0, c->stream);

@@ -138,6 +138,9 @@ namespace lbm {
 // storage scale); the caller sets fin/fout/macro.
 StepArgs make_args(const lbm_ctx *c);
 
+// What the launch rules look at.
+LatticeShape shape_of(const lbm_ctx *c);
+
 // Queues the copy of prescribed values that are still waiting for their step.
 int flush_bc(lbm_ctx *c);
 

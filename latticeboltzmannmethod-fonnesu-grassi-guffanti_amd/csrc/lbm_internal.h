@@ -5,13 +5,12 @@
 
 #include <hip/hip_runtime.h>
 #include <cstdint>
-#include <vector>
 
 #include "../../include/lbm_amd.h"
+#include "lbm_plan.h"
 
 namespace lbm {
 
-enum Storage : int32_t { kF64 = 0, kF32 = 1, kF16 = 2 };
 enum Policy : int32_t { kVelocity = 0, kPressure = 1, kNoop = 2 };
 enum EdgeKind : uint8_t { kEdgePlain = 0, kEdgeInlet = 1, kEdgeOutlet = 2 };
 
@@ -74,8 +73,6 @@ struct StepArgs {
     int32_t esize;          // bytes per stored population
     int32_t wpc;            // step kernel: waves per column
     int64_t nblocks;
-    int32_t wet_top, wet_bottom;  // row 0 / row NR-1 holds a wet node
-    int32_t cus;            // host side: compute units of the device
     double bgk_t, bgk_omt;              // 1/tau, 1 - 1/tau
     double trt_inv_te, trt_a, trt_b;    // 1/tau+, 0.5/tau+, 0.5/tau-
     float sh_a, sh_b;                   // shifted paths: 0.5/tau+, 0.5/tau- (BGK: both 0.5/tau)
@@ -137,17 +134,6 @@ constexpr uint32_t occupancy_lds(int32_t groups_per_cu)
     return groups_per_cu >= 2 && groups_per_cu <= 7 ? 163840u / (uint32_t)(groups_per_cu + 1) + 64u : 0u;
 }
 
-// How a launch of the marching kernel deals its waves (march_kernel).
-struct MarchPlan {
-    int32_t stripes;         // stripes of rows
-    int32_t top, bottom;     // of these, the first / last ones, whose windows hold wet nodes of row 0 / NR-1
-    int32_t cols;            // columns per wave
-    int32_t edge_cols;       // columns per wave of the edge stripes
-    int32_t edge_chunks;     // waves per edge stripe
-    int32_t edge_row_waves;  // waves of the edge stripes
-    int32_t edge_waves;      // and with the first and last columns of the others, rounded up to whole work-groups
-};
-
 // A batch step: per sample two complete argument sets, args[2 s + p] for
 // buffer parity p (p = 0: input in the sample's current buffer).
 struct BatchArgs {
@@ -170,11 +156,9 @@ struct BatchArgs {
     int32_t fused;  // enough nodes to keep the SIMDs full (march_kernel)
 };
 
-// Steps per launch of an ensemble's marching waves, their table over chunks
-// of `cols` columns (a[s]: any of sample s's arguments), and a launch: the
-// samples blocked and without new prescribed values.
+// Steps per launch of an ensemble's marching waves, and a launch of their
+// table (march_table): the samples blocked and without new prescribed values.
 constexpr int32_t kBatchMarchSteps = 4;
-void march_table(const StepArgs *a, int64_t samples, int32_t cols, std::vector<int32_t> &table);
 hipError_t launch_batch_march(int32_t storage, const BatchArgs &b, hipStream_t s);
 
 // Per-sample FP64 sums (readout's five) of a batch's current state:
@@ -215,22 +199,13 @@ hipError_t launch_lift_drag(int32_t storage, const StepArgs &a, const void *fsta
 // behind them holds room for kFoldBlocks more.
 constexpr int64_t kFoldBlocks = 256;
 hipError_t launch_reduce_partials(double *partials, int64_t nblocks, int32_t ncomp, double *out, hipStream_t s);
-// Lattices below these node counts take tiles (tile_steps), FP64 and FP32
-// lattices from there on marching waves; ensembles take marching waves from
-// kMarchMinNodes nodes in all.
-constexpr int64_t kTileMaxNodes = 300000, kTileMaxNodesF16 = (int64_t)3 << 19;
-constexpr int64_t kMarchMinNodes = (int64_t)1 << 17, kBatchFusedNodes = (int64_t)1 << 20;
-// Steps per launch of the marching kernel for this lattice (0: not for it),
-// and such a launch: `steps` steps (2 .. march_steps) without new prescribed
-// values from fin (F*) to fout.
-int32_t march_steps(int32_t storage, const StepArgs &a);
-hipError_t launch_march(int32_t storage, int32_t steps, const StepArgs &a, hipStream_t s);
-// Steps per launch of the tile kernel for this lattice (0: not for it), and
-// such a launch of 1 .. tile_steps steps from fin (F*) to fout.  The first
-// gather is closed with bc_prev, everything after takes bc_cur (in host
-// memory: copied to a.bc_new); a.macro is written by the last step.
-int32_t tile_steps(int32_t storage, const StepArgs &a);
-hipError_t launch_tile(int32_t storage, int32_t steps, const StepArgs &a, hipStream_t s);
+// A launch of `steps` steps (2 .. march_steps) without new prescribed values
+// from fin (F*) to fout, dealt as march_plan says for that number.
+hipError_t launch_march(int32_t storage, int32_t steps, const StepArgs &a, const MarchPlan &m, hipStream_t s);
+// A launch of 1 .. t.halo steps from fin (F*) to fout, t the lattice's tiles.
+// The first gather is closed with bc_prev, everything after takes bc_cur (in
+// host memory: copied to a.bc_new); a.macro is written by the last step.
+hipError_t launch_tile(int32_t storage, int32_t steps, const StepArgs &a, TileShape t, hipStream_t s);
 int64_t readout_blocks(const StepArgs &a);
 // Parts of a [3][n] field to host memory the device can write (either nullptr).
 hipError_t launch_copy_fields(const double *macro, int64_t n, double *rho, double *u, hipStream_t s);

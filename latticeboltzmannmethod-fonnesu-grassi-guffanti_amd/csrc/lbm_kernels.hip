@@ -2024,78 +2024,14 @@ hipError_t launch_step_t(bool gather, StepArgs a, hipStream_t s)
     return launch_perimeter<T>(a, s);
 }
 
-// Waves per SIMD the marching kernels' registers allow.
-template <typename T>
-constexpr int64_t kMarchWaves = sizeof(T) == 8 ? 2 : 3;
-
-// Deals the columns to waves.  A wave computes cols + 2 K columns' levels
-// for cols columns of results, so long chunks waste less, but the waves
-// should fill the chip a whole number of times (every wave takes about the
-// same time): the longest chunk of at most kMarchCols columns that does.
-// Small lattices: as many chunks as fit on the chip at once, of at least
-// kMarchMinCols columns.  Measured at K = 4, us a step by cols: FP64
-// 4096^2 open 141.8 (40), 143.6 (56, 2.6 fills), 136.0 (78, 2 fills), 169
-// (146, 1 fill); porous 8192^2 FP32 278 (32), 271 (64), 273 (128); FP64
-// 512 x 2048 16.0 (8), 14.3 (12), 17.2 (16).
-constexpr int64_t kMarchCols = 80, kMarchMinCols = 6;
-
-// Stripes of rows of K-step windows, and which of them hold wet nodes of
-// the first or last row.
-MarchPlan march_stripes(const StepArgs &a, int32_t K)
-{
-    const int32_t rows = 64 - 2 * K, nr = a.g.nr;
-    MarchPlan m{};
-    m.stripes = (nr + rows - 1) / rows;
-    if (a.g.nc < 2 * (K + 1) + 1) {  // no column is free of the first and last columns' influence
-        m.top = m.stripes;
-    } else {
-        m.top = a.wet_top ? 1 : 0;
-        if (a.wet_bottom)
-            for (int32_t q = m.stripes - 1; q >= m.top && q * rows - K + 64 >= nr; --q) ++m.bottom;
-    }
-    // edge waves are slower and start first: short ones, shorter still
-    // where the whole launch is short
-    m.edge_cols = (int64_t)nr * a.g.nc < (int64_t)1 << 21 ? 2 : 8;
-    m.edge_chunks = (a.g.nc + m.edge_cols - 1) / m.edge_cols;
-    return m;
-}
-
 template <typename T, int K>
-MarchPlan march_plan(const StepArgs &a)
+hipError_t launch_march_t(StepArgs a, const MarchPlan &m, hipStream_t s)
 {
-    MarchPlan m = march_stripes(a, K);
-    const int64_t inner = m.stripes - m.top - m.bottom, free_cols = a.g.nc - 2 * (K + 1);
-    m.edge_row_waves = (m.top + m.bottom) * m.edge_chunks;
-    m.edge_waves = (int32_t)((m.edge_row_waves + 2 * inner + 3) & ~(int64_t)3);
-    m.cols = kMarchMinCols;
-    if (inner > 0) {
-        const int64_t chip = a.cus * 4 * kMarchWaves<T>;
-        for (int64_t fills = 1;; ++fills) {
-            const int64_t chunks = (fills * chip - m.edge_waves) / inner;
-            if (chunks < 1) continue;
-            const int64_t cols = (free_cols + chunks - 1) / chunks;
-            if (cols > kMarchCols) continue;
-            m.cols = (int32_t)std::max(cols, kMarchMinCols);
-            break;
-        }
-    }
-    return m;
-}
-
-// Lattices whose waves keep the SIMDs full.
-bool march_large(const StepArgs &a) { return (int64_t)a.g.nr * a.g.nc >= (int64_t)1 << 22; }
-
-template <typename T, int K>
-hipError_t launch_march_t(StepArgs a, hipStream_t s)
-{
-    const MarchPlan m = march_plan<T, K>(a);
-    const int64_t inner = m.stripes - m.top - m.bottom;
-    const int64_t chunks = inner > 0 ? (a.g.nc - 2 * (K + 1) + m.cols - 1) / m.cols : 0;
-    a.nblocks = (m.edge_waves + inner * chunks + kBlockRows / 64 - 1) / (kBlockRows / 64);
+    a.nblocks = (m.waves + kBlockRows / 64 - 1) / (kBlockRows / 64);
     const dim3 grid((unsigned)a.nblocks), block(kBlockRows);
     // K = 5: large lattices only.  Lattices in planes, which are large unless
     // that layout was asked for, have the fused copy only at K = 4.
-    const bool fused = K == 5 || (K == 4 && (march_large(a) || !a.block_mask));
+    const bool fused = K == 5 || (K == 4 && ((int64_t)a.g.nr * a.g.nc >= kMarchLargeNodes || !a.block_mask));
     if constexpr (K >= 4) {
         if (fused && !a.block_mask) hipLaunchKernelGGL((march_kernel<T, K, true, true>), grid, block, 0, s, a, m);
         else if (fused) hipLaunchKernelGGL((march_kernel<T, K, true, false>), grid, block, 0, s, a, m);
@@ -2281,81 +2217,27 @@ hipError_t launch_batch_step(int32_t storage, bool gather, int32_t R, const Batc
     }
 }
 
-// A launch of marching waves takes at least the time one wave needs for its
-// columns (30 us at K = 4 in FP64, half of it in FP32; more where the top
-// or bottom row is wet): small lattices take tiles (tile_shape).  FP64 at
-// K = 5 is 5-7 % faster than K = 4 on 4096^2 (BGK; the same in TRT) and
-// slower on small lattices.
-int32_t march_steps(int32_t storage, const StepArgs &a)
-{
-    const int64_t nodes = (int64_t)a.g.nr * a.g.nc;
-    if (storage == kF16 || a.psbb || nodes < kTileMaxNodes) return 0;
-    return storage == kF64 && march_large(a) ? 5 : 4;
-}
-
-hipError_t launch_march(int32_t storage, int32_t steps, const StepArgs &a, hipStream_t s)
+hipError_t launch_march(int32_t storage, int32_t steps, const StepArgs &a, const MarchPlan &m, hipStream_t s)
 {
     if (storage == kF16 || a.psbb) return hipErrorInvalidValue;
     const bool f64 = storage == kF64;
     switch (steps) {
-    case 2: return f64 ? launch_march_t<double, 2>(a, s) : launch_march_t<float, 2>(a, s);
-    case 3: return f64 ? launch_march_t<double, 3>(a, s) : launch_march_t<float, 3>(a, s);
-    case 4: return f64 ? launch_march_t<double, 4>(a, s) : launch_march_t<float, 4>(a, s);
-    case 5: return f64 ? launch_march_t<double, 5>(a, s) : hipErrorInvalidValue;
+    case 2: return f64 ? launch_march_t<double, 2>(a, m, s) : launch_march_t<float, 2>(a, m, s);
+    case 3: return f64 ? launch_march_t<double, 3>(a, m, s) : launch_march_t<float, 3>(a, m, s);
+    case 4: return f64 ? launch_march_t<double, 4>(a, m, s) : launch_march_t<float, 4>(a, m, s);
+    case 5: return f64 ? launch_march_t<double, 5>(a, m, s) : hipErrorInvalidValue;
     default: return hipErrorInvalidValue;
     }
 }
 
 namespace {
 
-struct TileShape {
-    int32_t rows, cols, halo;  // halo 0: no tiles for this lattice
-};
-
-int64_t tiles_of(const StepArgs &a, TileShape t)
-{
-    const int64_t r = t.rows - 2 * t.halo, c = t.cols - 2 * t.halo;
-    return ((a.g.nr + r - 1) / r) * ((a.g.nc + c - 1) / c);
-}
-
-// As many steps a launch as leave one tile per CU: more steps share a
-// launch's fixed cost, and a second tile on a CU costs what it saves.  Smaller
-// regions step faster (waves per SIMD: 24 x 24 two to three, 32 x 24 three, 32
-// x 32 four) but hold fewer steps: the shapes are tried from the fastest per
-// step on.  Beyond one tile
-// per CU 8- and 4-byte elements part: two 32 x 24 tiles of FP32 or FP16 run
-// on a CU side by side.  Measured, us a step (steps a launch): 129^2 FP64
-// 32 x 24 1.85 (9), 32 x 20 1.84 (7), 32 x 16 1.95 (6), 24 x 24 2.05 (7), 32 x
-// 32 2.15 (10), FP32 1.45, 1.53, -, 1.60, 1.65; 65^2 FP64 24 x 24 1.75 (8), 32
-// x 24 1.86 (9); 160^2 24 x 24 1.92 (7), 32 x 24 2.01 (8); 200^2 FP64 32 x 24 2.27 (7), 32
-// x 32 2.50 (7); 300^2 FP64 32 x 32 3.26 (6), 32 x 24 3.71 (4); 251 x 1003 FP32
-// 32 x 24 4.63 (5), 4.88 (6), 32 x 32 5.14 (4), FP64 7.97 (4), 7.23 (4).  From
-// about 300000 nodes the marching waves are as fast (FP64 / FP32: 1400 x 200
-// march 7.8 / 5.6, porous 500 x 700 7.6 / 5.7); FP16, which has none, stays
-// until single steps are: 700^2 6.7 against 12.4, 1000^2 11.0 against 16.3,
-// 1500^2 about 24 either way.
-TileShape tile_shape(int32_t storage, const StepArgs &a)
-{
-    const int64_t nodes = (int64_t)a.g.nr * a.g.nc;
-    if (nodes >= (storage == kF16 ? kTileMaxNodesF16 : kTileMaxNodes)) return {0, 0, 0};
-    constexpr TileShape kOnePerCu[] = {{24, 24, 8}, {32, 24, 9}, {24, 24, 7}, {32, 24, 8}, {32, 24, 7}, {32, 32, 9},
-                                       {32, 32, 8}, {32, 32, 7}, {32, 32, 6}, {32, 32, 5}, {32, 32, 4}};
-    for (const TileShape &t : kOnePerCu)
-        if ((t.halo > 4 || storage == kF64) && tiles_of(a, t) <= a.cus) return t;
-    if (storage != kF64) {
-        if (tiles_of(a, {32, 24, 6}) <= 3 * (int64_t)a.cus) return {32, 24, 6};
-        return {32, 24, storage == kF16 && tiles_of(a, {32, 24, 5}) > 4 * (int64_t)a.cus ? 4 : 5};
-    }
-    for (int32_t halo = 7; halo > 4; --halo)
-        if (tiles_of(a, {32, 32, halo}) <= 2 * (int64_t)a.cus) return {32, 32, halo};
-    return {32, 32, 4};
-}
-
 template <typename T, bool PS>
 hipError_t launch_tile_t(const StepArgs &a, TileShape t, int32_t steps, hipStream_t s)
 {
     const int32_t n = t.rows - 2 * t.halo, ti = (a.g.nr + n - 1) / n;
-    const dim3 grid((unsigned)tiles_of(a, t)), block((unsigned)(t.rows * t.cols));
+    const int32_t nj = t.cols - 2 * t.halo, tj = (a.g.nc + nj - 1) / nj;
+    const dim3 grid((unsigned)ti * (unsigned)tj), block((unsigned)(t.rows * t.cols));
     if (t.rows == 24) hipLaunchKernelGGL((tile_kernel<T, 24, 24, PS>), grid, block, 0, s, a, steps, t.halo, ti);
     else if (t.cols == 24) hipLaunchKernelGGL((tile_kernel<T, 32, 24, PS>), grid, block, 0, s, a, steps, t.halo, ti);
     else hipLaunchKernelGGL((tile_kernel<T, 32, 32, PS>), grid, block, 0, s, a, steps, t.halo, ti);
@@ -2364,45 +2246,15 @@ hipError_t launch_tile_t(const StepArgs &a, TileShape t, int32_t steps, hipStrea
 
 }  // namespace
 
-int32_t tile_steps(int32_t storage, const StepArgs &a) { return tile_shape(storage, a).halo; }
-
-hipError_t launch_tile(int32_t storage, int32_t steps, const StepArgs &a0, hipStream_t s)
+hipError_t launch_tile(int32_t storage, int32_t steps, const StepArgs &a0, TileShape t, hipStream_t s)
 {
     StepArgs a = a0;
     set_planes(a);
-    const TileShape t = tile_shape(storage, a);
     if (steps < 1 || steps > t.halo) return hipErrorInvalidValue;
     switch (storage) {
     case kF64: return a.psbb ? launch_tile_t<double, true>(a, t, steps, s) : launch_tile_t<double, false>(a, t, steps, s);
     case kF32: return launch_tile_t<float, false>(a, t, steps, s);
     default: return launch_tile_t<_Float16, false>(a, t, steps, s);
-    }
-}
-
-void march_table(const StepArgs *a, int64_t samples, int32_t cols, std::vector<int32_t> &table)
-{
-    constexpr int32_t K = kBatchMarchSteps, rows = 64 - 2 * K;
-    table.clear();
-    auto add = [&](int64_t s, int32_t stripe, int32_t j0, int32_t j1, bool edge) {
-        table.insert(table.end(), {(int32_t)s, stripe * rows - K, j0, edge ? (int32_t)(j1 | (1u << 31)) : j1});
-    };
-    for (int64_t s = 0; s < samples; ++s) {
-        const MarchPlan m = march_stripes(a[s], K);
-        const int32_t nc = a[s].g.nc;
-        for (int32_t q = 0; q < m.stripes; ++q) {
-            if (q < m.top || q >= m.stripes - m.bottom) {
-                for (int32_t j = 0; j < nc; j += m.edge_cols) add(s, q, j, std::min(j + m.edge_cols, nc), true);
-            } else {
-                add(s, q, 0, K + 1, true);
-                add(s, q, nc - (K + 1), nc, true);
-            }
-        }
-    }
-    for (int64_t s = 0; s < samples; ++s) {
-        const MarchPlan m = march_stripes(a[s], K);
-        const int32_t end = a[s].g.nc - (K + 1);
-        for (int32_t j = K + 1; j < end; j += cols)
-            for (int32_t q = m.top; q < m.stripes - m.bottom; ++q) add(s, q, j, std::min(j + cols, end), false);
     }
 }
 

@@ -1,0 +1,118 @@
+// The launch rules (csrc/lbm_plan.cpp) at a prompt: one request a line, one
+// answer a line.
+//   shape STORAGE PSBB NR NC TOP BOTTOM CUS   the lattice of what follows
+//   steps                    march_steps, rows, columns and halo of its tiles
+//   plan K                   the numbers of march_plan
+//   cover K                  whether each row and column of a launch of K
+//                            steps belongs to one wave, in the kernel's numbering
+//   add / table K COLS       adds the lattice to an ensemble / the waves of its
+//                            table, and whether they cover every sample once
+#include "../../latticeboltzmannmethod-fonnesu-grassi-guffanti_amd/csrc/lbm_plan.h"
+
+#include <algorithm>
+#include <iostream>
+#include <sstream>
+#include <string>
+
+using namespace lbm;
+
+namespace {
+
+// Rows and columns that a window stores, and those its loads reach.
+struct Cover {
+    int64_t nr, nc;
+    std::vector<uint8_t> hits;
+    bool ok = true;
+    Cover(int64_t r, int64_t c) : nr(r), nc(c), hits((size_t)(r * c), 0) {}
+    void wave(const LatticeShape &a, int32_t K, int64_t i0, int64_t j0, int64_t j1, bool edge)
+    {
+        if (j0 < 0 || j1 > nc || j0 >= j1) ok = false;
+        // a window of the inner copy takes no perimeter node in any level
+        if (!edge && (j0 - K < 1 || j1 + K > nc - 1)) ok = false;
+        if (!edge && ((a.wet_top && i0 <= 0) || (a.wet_bottom && i0 + 64 >= nr))) ok = false;
+        for (int64_t j = std::max<int64_t>(j0, 0); j < std::min(j1, nc); ++j)
+            for (int64_t i = std::max<int64_t>(i0 + K, 0); i < std::min(i0 + 64 - K, nr); ++i)
+                if (hits[(size_t)(j * nr + i)]++) ok = false;
+    }
+    bool whole() const { return ok && std::all_of(hits.begin(), hits.end(), [](uint8_t h) { return h == 1; }); }
+};
+
+// The waves of march_kernel, numbered as it numbers them.
+bool covered(const LatticeShape &a, int32_t K)
+{
+    const MarchPlan m = march_plan(a, K);
+    const int64_t rows = 64 - 2 * K, inner = m.stripes - m.top - m.bottom;
+    const int64_t blocks = (m.waves + 3) / 4;
+    Cover c(a.nr, a.nc);
+    for (int64_t w = 0; w < 4 * blocks; ++w) {
+        int64_t t = w;
+        if (t < m.edge_waves) {
+            if (t < m.edge_row_waves) {
+                const int64_t q = t / m.edge_chunks, j0 = (t - q * m.edge_chunks) * m.edge_cols;
+                const int64_t stripe = q < m.top ? q : m.stripes - m.bottom + (q - m.top);
+                c.wave(a, K, stripe * rows - K, j0, std::min<int64_t>(j0 + m.edge_cols, a.nc), true);
+            } else {
+                t -= m.edge_row_waves;
+                if (t >= 2 * inner) continue;
+                const bool right = t >= inner;
+                const int64_t stripe = m.top + (right ? t - inner : t);
+                c.wave(a, K, stripe * rows - K, right ? a.nc - (K + 1) : 0, right ? a.nc : K + 1, true);
+            }
+            continue;
+        }
+        t -= m.edge_waves;
+        if (inner == 0) return false;  // the kernel would divide by it
+        const int64_t chunk = t / inner, j0 = K + 1 + chunk * m.cols, end = a.nc - (K + 1);
+        if (j0 >= end) continue;
+        c.wave(a, K, (m.top + t - chunk * inner) * rows - K, j0, std::min<int64_t>(j0 + m.cols, end), false);
+    }
+    return c.whole();
+}
+
+}  // namespace
+
+int main()
+{
+    LatticeShape a{};
+    std::vector<LatticeShape> samples;
+    std::string line, what;
+    while (std::getline(std::cin, line)) {
+        std::istringstream in(line);
+        in >> what;
+        int32_t K = 0, cols = 0;
+        if (what == "shape") {
+            in >> a.storage >> a.psbb >> a.nr >> a.nc >> a.wet_top >> a.wet_bottom >> a.cus;
+            continue;
+        }
+        if (what == "add") {
+            samples.push_back(a);
+            continue;
+        }
+        if (what == "steps") {
+            const TileShape t = tile_shape(a);
+            std::cout << march_steps(a) << " " << t.rows << " " << t.cols << " " << t.halo;
+        } else if (what == "plan") {
+            in >> K;
+            const MarchPlan m = march_plan(a, K);
+            std::cout << m.stripes << " " << m.top << " " << m.bottom << " " << m.cols << " " << m.edge_cols << " "
+                      << m.edge_row_waves << " " << m.edge_waves << " " << m.waves;
+        } else if (what == "cover") {
+            in >> K;
+            std::cout << covered(a, K);
+        } else if (what == "table") {
+            in >> K >> cols;
+            std::vector<int32_t> table;
+            march_table(samples.data(), (int64_t)samples.size(), K, cols, table);
+            bool ok = true;
+            for (size_t s = 0; s < samples.size(); ++s) {
+                Cover c(samples[s].nr, samples[s].nc);
+                for (size_t k = 0; k < table.size(); k += 4)
+                    if (table[k] == (int32_t)s)
+                        c.wave(samples[s], K, table[k + 1], table[k + 2], table[k + 3] & 0x7fffffff, table[k + 3] < 0);
+                ok = ok && c.whole();
+            }
+            std::cout << table.size() / 4 << " " << ok;
+        }
+        std::cout << std::endl;
+    }
+}

@@ -1,0 +1,61 @@
+"""The launch rules (csrc/lbm_plan.cpp), on the CPU: what they deal out covers
+every node once, and which launch they choose."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+from conftest import PKG, ROOT
+
+F64, F32, F16 = range(3)
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    if shutil.which("g++") is None:
+        pytest.skip("needs g++")
+    exe = str(tmp_path_factory.mktemp("rules") / "launch_rules")
+    r = subprocess.run(["g++", "-std=c++20", "-O1", "-g", os.path.join(ROOT, "tests", "cpp", "launch_rules.cpp"),
+                        os.path.join(PKG, "csrc", "lbm_plan.cpp"), "-o", exe], capture_output=True, text=True,
+                       timeout=300)
+    assert r.returncode == 0, r.stderr[-3000:]
+
+    def ask(*lines):
+        r = subprocess.run([exe], input="\n".join(lines) + "\n", capture_output=True, text=True, timeout=120)
+        assert r.returncode == 0, r.stderr[-3000:]
+        return [[int(x) for x in ln.split()] for ln in r.stdout.splitlines()]
+
+    return ask
+
+
+def shape(storage, nr, nc, top=False, bottom=False, psbb=False, cus=256):
+    return f"shape {storage} {int(psbb)} {nr} {nc} {int(top)} {int(bottom)} {cus}"
+
+
+# rows at the windows' ends for every K (60, 58, 56 and 54 stored rows), columns
+# around the ones that the first and last columns influence
+ROWS = (1, 3, 53, 54, 55, 56, 57, 59, 60, 61, 64, 65, 108, 109, 112, 113, 161, 162, 163, 1100)
+COLS = (3, 6, 7, 8, 9, 10, 11, 12, 13, 14, 20, 61, 700)
+
+
+@pytest.mark.parametrize("K", [2, 3, 4, 5])
+@pytest.mark.parametrize("storage", [F64, F32])
+def test_waves_cover_the_lattice(rules, storage, K):
+    asked, lines = [], []
+    for nr in ROWS:
+        for nc in COLS:
+            for top, bottom in ((0, 0), (1, 0), (0, 1), (1, 1)):
+                asked.append((nr, nc, top, bottom))
+                lines += [shape(storage, nr, nc, top, bottom, cus=256 if nr % 2 else 32), f"cover {K}"]
+    for case, (ok,) in zip(asked, rules(*lines)):
+        assert ok, case
+
+
+@pytest.mark.parametrize("cols", [64, 16, 6])
+def test_ensemble_waves_cover_the_samples(rules, cols):
+    lines = []
+    for k, (nr, nc) in enumerate([(3, 3), (5, 9), (57, 10), (56, 11), (64, 12), (113, 40), (300, 200), (129, 700)]):
+        lines += [shape(F32, nr, nc, k % 2, k % 3 == 0), "add"]
+    waves, ok = rules(*lines, f"table 4 {cols}")[0]
+    assert ok and waves > 0
