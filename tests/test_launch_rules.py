@@ -59,3 +59,20 @@ def test_ensemble_waves_cover_the_samples(rules, cols):
         lines += [shape(F32, nr, nc, k % 2, k % 3 == 0), "add"]
     waves, ok = rules(*lines, f"table 4 {cols}")[0]
     assert ok and waves > 0
+
+
+LIDS = [(3, 106666), (16, 62500), (30, 9999), (50, 8000), (50, 20000), (64, 15625), (120, 9000)]
+
+
+@pytest.mark.parametrize("storage", [F64, F32])
+def test_perimeter_waves_do_not_fill_the_chip_with_halo_columns(rules, storage):
+    """A wave of a perimeter window computes 2 K columns beside those it
+    stores: short ones only while they leave room on the chip."""
+    chip = 256 * 4 * (2 if storage == F64 else 3)
+    for nr, nc in LIDS:
+        for bottom in (False, True):
+            (_, _, _, _, edge_cols, edge_row_waves, _, _), = rules(shape(storage, nr, nc, True, bottom), "plan 4")
+            assert edge_cols >= 2 and (edge_cols == 8 or edge_row_waves <= chip), (nr, nc, bottom)
+    # the same for an ensemble's table: 300 lattices of two stripes, one on the perimeter
+    waves, ok = rules(*[shape(storage, 64, 64, True), "add"] * 300, "table 4 64")[0]
+    assert ok and waves - 300 * 3 <= 300 * 8
