@@ -232,12 +232,7 @@ void set_max_steps(lbm_batch *b, int32_t steps)
     b->max_steps = steps;
 }
 
-// Table of the marching waves.  Chunks of columns: the longest of these
-// that fill three quarters of the chip's waves (each wave recomputes the 2 K
-// columns at its ends), and the shortest for ensembles that never do.  us a
-// step by columns (64 / 32 / 16 / 8): 32 lattices of up to 1024^2 FP32 48.6 /
-// 47.6 / 50.9 / 57.6; 20 of up to 512^2 24.1 / 18.4 / 14.8 / 15.4; 60 of up to
-// 256^2 FP64 35.0 / 26.6 / 27.2 / 26.2.
+// Table of the marching waves.
 int build_marches(lbm_batch *b)
 {
     int64_t nodes = 0;
@@ -249,11 +244,7 @@ int build_marches(lbm_batch *b)
     }
     if (nodes < kMarchMinNodes) return LBM_OK;
     std::vector<int32_t> table;
-    const int64_t chip = (int64_t)b->cus * 4 * (b->storage == kF64 ? 2 : 3);
-    for (int32_t cols : {64, 32, 16, 12, 8, 6}) {
-        march_table(shapes.data(), (int64_t)shapes.size(), kBatchMarchSteps, cols, table);
-        if ((int64_t)table.size() / 4 >= chip * 3 / 4) break;
-    }
+    march_table(shapes.data(), (int64_t)shapes.size(), kBatchMarchSteps, table);
     b->nmarches = (int64_t)table.size() / 4;
     HIP_TRY(hipMalloc(&b->d_marches, table.size() * sizeof(int32_t)));
     HIP_TRY(hipMemcpy(b->d_marches, table.data(), table.size() * sizeof(int32_t), hipMemcpyHostToDevice));

@@ -18,7 +18,10 @@ int64_t march_waves(int32_t storage) { return storage == kF64 ? 2 : 3; }
 // kMarchMinCols columns.  Measured at K = 4, us a step by cols: FP64
 // 4096^2 open 141.8 (40), 143.6 (56, 2.6 fills), 136.0 (78, 2 fills), 169
 // (146, 1 fill); porous 8192^2 FP32 278 (32), 271 (64), 273 (128); FP64
-// 512 x 2048 16.0 (8), 14.3 (12), 17.2 (16).
+// 512 x 2048 16.0 (8), 14.3 (12), 17.2 (16).  A fill that the edge waves
+// leave less than a fifth of is no reason for a long chunk: its few waves
+// would run on alone for most of the launch (FP64, first row wet, 200 x 5000:
+// 27.0 with one of 40 columns, 22.7 with the next fill's 9).
 constexpr int64_t kMarchCols = 80, kMarchMinCols = 6;
 
 // Waves the device holds at once.
@@ -83,16 +86,49 @@ MarchPlan march_plan(const LatticeShape &a, int32_t K)
     m.cols = kMarchMinCols;
     if (inner > 0) {
         for (int64_t fills = 1;; ++fills) {
-            const int64_t chunks = (fills * chip - m.edge_waves) / inner;
+            const int64_t slots = fills * chip - m.edge_waves, chunks = slots / inner;
             if (chunks < 1) continue;
             const int64_t cols = (free_cols + chunks - 1) / chunks;
-            if (cols > kMarchCols) continue;
+            if (cols > kMarchCols || (cols > kMarchCols / 2 && slots < chip / 5)) continue;
             m.cols = (int32_t)std::max(cols, kMarchMinCols);
             break;
         }
     }
     m.waves = m.edge_waves + (inner > 0 ? inner * ((free_cols + m.cols - 1) / m.cols) : 0);
     return m;
+}
+
+namespace {
+
+// Columns that a marching wave computes, weighted by how long one takes: the
+// perimeter's closures wait for loads of their own at every level.
+double march_work(const int32_t *wave, int32_t K)
+{
+    const bool edge = wave[3] < 0;
+    return ((wave[3] & 0x7fffffff) - wave[2] + 2 * K) * (edge ? 1.75 : 1.0);
+}
+
+}  // namespace
+
+// Chunks of columns: the longest of these whose waves keep three quarters of
+// the chip busy for as long as one of them takes (each wave recomputes the 2 K
+// columns at its ends), and the shortest for ensembles that never do.  us a
+// step by columns (64 / 32 / 16 / 8): 32 lattices of up to 1024^2 FP32 48.6 /
+// 47.6 / 50.9 / 57.6; 20 of up to 512^2 24.1 / 18.4 / 14.8 / 15.4; 60 of up to
+// 256^2 FP64 35.0 / 26.6 / 27.2 / 26.2.  It is the work that counts and not the
+// number of waves: perimeter waves are many and short.  Counted alike they
+// made the others long, single steps / counted alike / this: 20 lattices of
+// 129^2 with a wet first row FP64 18.1 / 23.9 / 13.3, and last row 20.9 / 47.1
+// / 16.0; 60 of 64^2 17.2 / 41.6 / 14.3; 16 porous ones of 512^2 92.1 / 47.4 /
+// 35.5.
+void march_table(const LatticeShape *a, int64_t samples, int32_t K, std::vector<int32_t> &table)
+{
+    for (int32_t cols : {64, 32, 16, 12, 8, 6}) {
+        march_table(a, samples, K, cols, table);
+        double work = 0.0;
+        for (size_t k = 0; k < table.size(); k += 4) work += march_work(&table[k], K);
+        if (samples == 0 || work >= 0.75 * (double)march_chip(a[0]) * (cols + 2 * K)) return;
+    }
 }
 
 void march_table(const LatticeShape *a, int64_t samples, int32_t K, int32_t cols, std::vector<int32_t> &table)

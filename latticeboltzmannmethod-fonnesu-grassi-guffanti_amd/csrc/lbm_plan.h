@@ -44,9 +44,11 @@ struct MarchPlan {
 int32_t march_steps(const LatticeShape &a);
 MarchPlan march_plan(const LatticeShape &a, int32_t K);
 
-// Waves of an ensemble's marching launch of K steps over chunks of `cols`
-// columns: per wave, 4 int32 -- sample, first row of the window, columns
+// Waves of an ensemble's marching launch of K steps, the columns of the
+// windows without perimeter nodes in chunks of `cols`, or in chunks chosen
+// here: per wave, 4 int32 -- sample, first row of the window, columns
 // [j0, j1) (sign bit of j1: perimeter window).
+void march_table(const LatticeShape *a, int64_t samples, int32_t K, std::vector<int32_t> &table);
 void march_table(const LatticeShape *a, int64_t samples, int32_t K, int32_t cols, std::vector<int32_t> &table);
 
 // Region of a tile, and the steps per launch it holds (halo 0: no tiles for

@@ -6,7 +6,9 @@
 //   cover K                  whether each row and column of a launch of K
 //                            steps belongs to one wave, in the kernel's numbering
 //   add / table K COLS       adds the lattice to an ensemble / the waves of its
-//                            table, and whether they cover every sample once
+//                            table, whether they cover every sample once, and
+//                            the longest wave without perimeter nodes
+//                            (COLS 0: the library's choice)
 #include "../../latticeboltzmannmethod-fonnesu-grassi-guffanti_amd/csrc/lbm_plan.h"
 
 #include <algorithm>
@@ -102,8 +104,12 @@ int main()
         } else if (what == "table") {
             in >> K >> cols;
             std::vector<int32_t> table;
-            march_table(samples.data(), (int64_t)samples.size(), K, cols, table);
+            if (cols) march_table(samples.data(), (int64_t)samples.size(), K, cols, table);
+            else march_table(samples.data(), (int64_t)samples.size(), K, table);
             bool ok = true;
+            int32_t longest = 0;
+            for (size_t k = 0; k < table.size(); k += 4)
+                if (table[k + 3] >= 0) longest = std::max(longest, table[k + 3] - table[k + 2]);
             for (size_t s = 0; s < samples.size(); ++s) {
                 Cover c(samples[s].nr, samples[s].nc);
                 for (size_t k = 0; k < table.size(); k += 4)
@@ -111,7 +117,7 @@ int main()
                         c.wave(samples[s], K, table[k + 1], table[k + 2], table[k + 3] & 0x7fffffff, table[k + 3] < 0);
                 ok = ok && c.whole();
             }
-            std::cout << table.size() / 4 << " " << ok;
+            std::cout << table.size() / 4 << " " << ok << " " << longest;
         }
         std::cout << std::endl;
     }

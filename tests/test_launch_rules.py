@@ -52,13 +52,13 @@ def test_waves_cover_the_lattice(rules, storage, K):
         assert ok, case
 
 
-@pytest.mark.parametrize("cols", [64, 16, 6])
+@pytest.mark.parametrize("cols", [64, 16, 6, 0])
 def test_ensemble_waves_cover_the_samples(rules, cols):
     lines = []
     for k, (nr, nc) in enumerate([(3, 3), (5, 9), (57, 10), (56, 11), (64, 12), (113, 40), (300, 200), (129, 700)]):
         lines += [shape(F32, nr, nc, k % 2, k % 3 == 0), "add"]
-    waves, ok = rules(*lines, f"table 4 {cols}")[0]
-    assert ok and waves > 0
+    waves, ok, longest = rules(*lines, f"table 4 {cols}")[0]
+    assert ok and waves > 0 and longest <= (cols or 64)
 
 
 LIDS = [(3, 106666), (16, 62500), (30, 9999), (50, 8000), (50, 20000), (64, 15625), (120, 9000)]
@@ -74,5 +74,20 @@ def test_perimeter_waves_do_not_fill_the_chip_with_halo_columns(rules, storage):
             (_, _, _, _, edge_cols, edge_row_waves, _, _), = rules(shape(storage, nr, nc, True, bottom), "plan 4")
             assert edge_cols >= 2 and (edge_cols == 8 or edge_row_waves <= chip), (nr, nc, bottom)
     # the same for an ensemble's table: 300 lattices of two stripes, one on the perimeter
-    waves, ok = rules(*[shape(storage, 64, 64, True), "add"] * 300, "table 4 64")[0]
+    waves, ok, _ = rules(*[shape(storage, 64, 64, True), "add"] * 300, "table 4 64")[0]
     assert ok and waves - 300 * 3 <= 300 * 8
+
+
+def test_long_chunks_only_where_they_fill_the_chip(rules):
+    """Perimeter waves take slots of the chip, but not for as long as a long
+    chunk takes: they are no reason for one."""
+    for nr, nc in ((200, 5000), (130, 7692)):
+        (_, _, _, cols, _, _, edge_waves, waves), = rules(shape(F64, nr, nc, True), "plan 4")
+        assert cols <= 40 or (waves - edge_waves) >= 2048 // 5, (nr, nc)
+    for storage in (F64, F32):
+        for n, size in ((20, 129), (10, 256), (30, 100)):
+            _, ok, longest = rules(*[shape(storage, size, size, True, True), "add"] * n, "table 4 0")[0]
+            assert ok and longest <= 16, (storage, n, size)
+        # without perimeter rows, enough waves for long chunks
+        _, ok, longest = rules(*[shape(storage, 1024, 1024), "add"] * 12, "table 4 0")[0]
+        assert ok and longest == 64
