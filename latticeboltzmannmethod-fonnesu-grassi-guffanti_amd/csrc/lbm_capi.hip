@@ -108,7 +108,7 @@ StepArgs make_args(const lbm_ctx *c)
 
 LatticeShape shape_of(const lbm_ctx *c)
 {
-    return {c->storage, c->psbb, c->nr, c->nc, c->wet_top, c->wet_bottom, c->cus};
+    return {c->storage, c->psbb, c->nr, c->nc, c->wet_top, c->wet_bottom, c->cus, c->n_wet, c->wet_segments};
 }
 
 int flush_bc(lbm_ctx *c)
@@ -141,7 +141,8 @@ Launching launching(const lbm_ctx *c)
     if (most > 1) {
         const LatticeShape a = shape_of(c);
         if (const int32_t k = tile_shape(a).halo) return {Launching::kTile, std::min(k, most)};
-        if (const int32_t k = march_steps(a)) return {Launching::kMarch, std::min(k, most)};
+        const int32_t k = march_steps(a);
+        if (k > 0 && (c->max_steps > 0 || march_pays(a))) return {Launching::kMarch, std::min(k, most)};
     }
     return {Launching::kSingle, 1};
 }
@@ -752,6 +753,7 @@ int lbm_set_geometry(lbm_ctx *c, const uint8_t *cls)
     for (int k = 0; k < 7; ++k) c->counts[k] = 0;
     c->n_wet = 0;
     c->wet_top = c->wet_bottom = false;
+    c->wet_segments = 0;
     for (int w = 0; w < 2; ++w) { c->open_ij[w].clear(); c->open_e[w].clear(); }
     c->obst_ij.clear();
     c->obst_mask.clear();
@@ -793,6 +795,7 @@ int lbm_set_geometry(lbm_ctx *c, const uint8_t *cls)
             bool prev = false;  // row 64 k - 1 wet
             for (int64_t k = 0; k < nrw; ++k) {
                 const uint64_t m = wet[w0 + k];
+                c->wet_segments += m != 0;
                 if (m && r0 < 0) r0 = 64 * k + __builtin_ctzll(m);
                 count += __builtin_popcountll(m);
                 // stretch starts: wet rows whose row above is dry

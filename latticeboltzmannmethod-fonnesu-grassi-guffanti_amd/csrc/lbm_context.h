@@ -54,6 +54,7 @@ struct lbm_ctx {
     int32_t *d_perim = nullptr;  // perimeter items (column, segment) of the perimeter kernel
     int64_t nperim = 0;
     bool wet_top = false, wet_bottom = false;  // row 0 / row NR-1 holds a wet node
+    int64_t wet_segments = 0;                  // 64-row segments of columns that hold one
     uint8_t *d_edge_kind = nullptr;
     void *d_frozen = nullptr;
     void *d_F[2] = {nullptr, nullptr};

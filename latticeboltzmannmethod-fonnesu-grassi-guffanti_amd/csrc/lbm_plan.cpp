@@ -75,6 +75,34 @@ int32_t march_steps(const LatticeShape &a)
     return a.storage == kF64 && nodes >= kMarchLargeNodes ? 5 : 4;
 }
 
+// A marching launch walks every window of the lattice, wet or not, and its
+// waves at the perimeter store few of the columns that they compute.  The
+// one-step kernels leave dry segments at once.  us a step, one step a launch /
+// marching:
+//  * Mostly dry lattices, single steps below 2^20 nodes where less than half
+//    of the segments hold a wet node: FP64 600^2, fluid in one rectangle of 5 /
+//    20 / 40 % 4.6 / 6.7, 5.2 / 6.9, 6.7 / 7.1, squares of fluid 3 / 10 / 30 %
+//    (10 / 32 / 73 % of the segments) 5.1 / 6.7, 5.7 / 6.8, 7.4 / 7.2; 2000 x
+//    200 FP32 5 % 4.1 / 5.0.  At 1100^2 5 % FP64 the two meet (9.6 / 10.0) and
+//    above marching wins: the one-step kernel's dry waves cost what it saves.
+//  * All windows at the perimeter because the first and the last row are wet:
+//    single steps where the windows are more than the segments (57 to 64 rows,
+//    or K = 5 and 109 to 128): 64 x 15625 FP64 36.7 / 42.4, FP32 24.6 / 28.3, 112
+//    x 44642 FP64 181.9 / 193.2; but 80 x 12500 FP64 44.2 / 41.6.
+//  * Fewer than 2 K + 5 columns, so that no window, or hardly one, is free of
+//    the first and last column: single steps with many solid nodes.  440000 x
+//    10 FP32, 30 % solid 31.7 / 37.1, open 61.9 / 52.1; 400000 x 11 30 % solid
+//    31.9 / 35.8.
+bool march_pays(const LatticeShape &a)
+{
+    const int64_t nodes = a.nr * a.nc, rows = (a.nr + 63) / 64;
+    if (nodes < ((int64_t)1 << 20) && 2 * a.wet_segments < rows * a.nc) return false;
+    const int32_t K = march_steps(a);
+    if (a.nc < 2 * K + 5) return 4 * a.wet >= 3 * nodes;
+    const MarchPlan m = march_stripes(a, K);
+    return m.top + m.bottom < m.stripes || m.stripes <= rows;
+}
+
 MarchPlan march_plan(const LatticeShape &a, int32_t K)
 {
     MarchPlan m = march_stripes(a, K);

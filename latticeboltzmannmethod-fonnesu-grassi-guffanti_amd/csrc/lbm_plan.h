@@ -17,6 +17,7 @@ struct LatticeShape {
     int64_t nr, nc;
     bool wet_top, wet_bottom;   // row 0 / row NR-1 holds a wet node
     int32_t cus;                // compute units of the device
+    int64_t wet, wet_segments;  // wet nodes, and 64-row segments of columns that hold one
 };
 
 // Lattices below these node counts take tiles, FP64 and FP32 lattices from
@@ -43,6 +44,9 @@ struct MarchPlan {
 // and the deal of a launch of K of them.
 int32_t march_steps(const LatticeShape &a);
 MarchPlan march_plan(const LatticeShape &a, int32_t K);
+// Whether such launches are faster than the one-step kernels, by shape and
+// wet nodes.
+bool march_pays(const LatticeShape &a);
 
 // Waves of an ensemble's marching launch of K steps, the columns of the
 // windows without perimeter nodes in chunks of `cols`, or in chunks chosen

@@ -1,7 +1,8 @@
 // The launch rules (csrc/lbm_plan.cpp) at a prompt: one request a line, one
 // answer a line.
-//   shape STORAGE PSBB NR NC TOP BOTTOM CUS   the lattice of what follows
+//   shape STORAGE PSBB NR NC TOP BOTTOM CUS WET SEGMENTS   the lattice of what follows
 //   steps                    march_steps, rows, columns and halo of its tiles
+//   pays                     march_pays
 //   plan K                   the numbers of march_plan
 //   cover K                  whether each row and column of a launch of K
 //                            steps belongs to one wave, in the kernel's numbering
@@ -83,7 +84,8 @@ int main()
         in >> what;
         int32_t K = 0, cols = 0;
         if (what == "shape") {
-            in >> a.storage >> a.psbb >> a.nr >> a.nc >> a.wet_top >> a.wet_bottom >> a.cus;
+            in >> a.storage >> a.psbb >> a.nr >> a.nc >> a.wet_top >> a.wet_bottom >> a.cus >> a.wet >>
+                a.wet_segments;
             continue;
         }
         if (what == "add") {
@@ -93,6 +95,8 @@ int main()
         if (what == "steps") {
             const TileShape t = tile_shape(a);
             std::cout << march_steps(a) << " " << t.rows << " " << t.cols << " " << t.halo;
+        } else if (what == "pays") {
+            std::cout << march_pays(a);
         } else if (what == "plan") {
             in >> K;
             const MarchPlan m = march_plan(a, K);

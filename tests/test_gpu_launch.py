@@ -84,3 +84,23 @@ def test_without_geometry_it_is_an_error():
     with L.Lattice(L.geometry_channel(40, 96), storage=L.F16_SHIFTED) as lat:
         assert lat.steps_per_launch() > 1
     assert L.lib().lbm_get_steps_per_launch(None, C.byref(C.c_int32())) == L.ERR_INVALID
+
+
+@pytest.mark.parametrize("storage", [L.F64, L.F32_SHIFTED])
+def test_mostly_dry_lattices_take_single_steps(storage):
+    """The rule's line, seen from outside, and the same bits either side of it."""
+    nr = nc = 600
+    p0 = state(np.random.default_rng(2), nc, nr)
+    for wet, single in ((0.2, True), (0.8, False)):
+        cls = np.full((nc, nr), L.OBSTACLE, np.uint8)
+        cls[1:int(wet * nc), 1:nr - 1] = L.FLUID
+        lat = L.Lattice(cls, storage=storage, tau=0.8)
+        assert (lat.steps_per_launch() == 1) == single
+        out = []
+        for k in (0, 1, 4):
+            lat.set_steps_per_launch(k)
+            lat.upload_populations(p0)
+            lat.step(45)
+            out.append(lat.populations())
+        assert np.array_equal(out[0], out[1]) and np.array_equal(out[0], out[2])
+        lat.close()

@@ -29,8 +29,11 @@ def rules(tmp_path_factory):
     return ask
 
 
-def shape(storage, nr, nc, top=False, bottom=False, psbb=False, cus=256):
-    return f"shape {storage} {int(psbb)} {nr} {nc} {int(top)} {int(bottom)} {cus}"
+def shape(storage, nr, nc, top=False, bottom=False, psbb=False, cus=256, wet=1.0, segments=1.0):
+    """wet, segments: shares of the nodes that are wet, of the 64-row segments
+    that hold a wet node."""
+    return (f"shape {storage} {int(psbb)} {nr} {nc} {int(top)} {int(bottom)} {cus} {int(wet * nr * nc)} "
+            f"{int(segments * ((nr + 63) // 64) * nc)}")
 
 
 # rows at the windows' ends for every K (60, 58, 56 and 54 stored rows), columns
@@ -91,3 +94,19 @@ def test_long_chunks_only_where_they_fill_the_chip(rules):
         # without perimeter rows, enough waves for long chunks
         _, ok, longest = rules(*[shape(storage, 1024, 1024), "add"] * 12, "table 4 0")[0]
         assert ok and longest == 64
+
+
+@pytest.mark.parametrize("storage", [F64, F32])
+def test_lattices_that_march(rules, storage):
+    """Single steps where marching measured slower: mostly dry lattices below
+    2^20 nodes, and lattices whose windows are all at the perimeter, of more
+    windows than segments or with many solid nodes."""
+    yes = [shape(storage, 560, 541), shape(storage, 600, 600, wet=0.7), shape(storage, 600, 600, wet=0.2, segments=0.55),
+           shape(storage, 1100, 1100, wet=0.1, segments=0.1), shape(storage, 4096, 4096, wet=0.05, segments=0.05),
+           shape(storage, 50, 8000, True), shape(storage, 80, 12500, True, True), shape(storage, 64, 15625, True),
+           shape(storage, 33400, 9), shape(storage, 700, 700, True, True)]
+    no = [shape(storage, 600, 600, wet=0.05, segments=0.06), shape(storage, 600, 600, wet=0.1, segments=0.32),
+          shape(storage, 2000, 200, wet=0.3, segments=0.3), shape(storage, 64, 15625, True, True),
+          shape(storage, 44000, 10, wet=0.6), shape(storage, 400000, 12, wet=0.7)]
+    got = rules(*sum([[s, "pays"] for s in yes + no], []))
+    assert [x for x, in got] == [1] * len(yes) + [0] * len(no)
