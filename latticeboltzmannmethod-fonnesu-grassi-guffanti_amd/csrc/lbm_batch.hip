@@ -69,7 +69,7 @@ struct lbm_batch {
     // unless max_steps (steps per launch at most, 0 = the rule) forbids them
     int32_t *d_marches = nullptr;
     int64_t nmarches = 0;
-    bool march = false;
+    bool march = false, march_pays = false;
     int32_t max_steps = 0;
     bool fused = false;
     // "first" = each sample's arguments as lbm_step would build them for its
@@ -226,7 +226,7 @@ int build_runs(lbm_batch *b)
 
 void set_max_steps(lbm_batch *b, int32_t steps)
 {
-    const bool march = b->nmarches > 0 && (steps == 0 || steps >= kBatchMarchSteps);
+    const bool march = b->nmarches > 0 && (steps == 0 ? b->march_pays : steps >= kBatchMarchSteps);
     if (march != b->march) drop_graphs(b);
     b->march = march;
     b->max_steps = steps;
@@ -246,6 +246,7 @@ int build_marches(lbm_batch *b)
     std::vector<int32_t> table;
     march_table(shapes.data(), (int64_t)shapes.size(), kBatchMarchSteps, table);
     b->nmarches = (int64_t)table.size() / 4;
+    b->march_pays = ensemble_pays(shapes.data(), (int64_t)shapes.size(), kBatchMarchSteps, table);
     HIP_TRY(hipMalloc(&b->d_marches, table.size() * sizeof(int32_t)));
     HIP_TRY(hipMemcpy(b->d_marches, table.data(), table.size() * sizeof(int32_t), hipMemcpyHostToDevice));
     b->fused = nodes >= kBatchFusedNodes;

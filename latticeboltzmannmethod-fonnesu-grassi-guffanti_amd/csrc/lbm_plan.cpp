@@ -192,6 +192,35 @@ void march_table(const LatticeShape *a, int64_t samples, int32_t K, int32_t cols
     }
 }
 
+// A marching launch walks every window, wet or not; an ensemble's one-step
+// kernels have a table of the segments that hold a wet node and take only
+// those.  The launch takes as long as the columns that fall to one slot of the
+// chip (kMarchWaves a SIMD, edge columns a quarter more); four single steps
+// cost a fixed time, one per segment and one per wet node, in the same unit of
+// about 2.5 us.  Fitted to 90 ensembles per format: 131072 to 12 million nodes,
+// lattices of 16 x 16 to 1024^2, 2 to 1000 of them, channels, cavities, porous
+// and mostly dry media, wet first and last rows.  Single steps were up to 6 times
+// faster on 27 of them, and marching up to 2.8 on the others; the rule errs by up
+// to 15 %, where the two are close.  us a step, one step a launch /
+// marching: 16 lattices of 512^2, 5 / 20 / 50 % of each wet, FP64 7.8 / 33.5,
+// 24.5 / 34.1, 50.7 / 34.4; FP32 5.9 / 22.4, 13.6 / 23.2, 26.8 / 23.3.
+bool ensemble_pays(const LatticeShape *a, int64_t samples, int32_t K, const std::vector<int32_t> &table)
+{
+    if (table.empty()) return false;
+    double segments = 0.0, wet = 0.0, columns = 0.0;
+    for (int64_t s = 0; s < samples; ++s) {
+        segments += (double)a[s].wet_segments;
+        wet += (double)a[s].wet;
+    }
+    for (size_t k = 0; k < table.size(); k += 4)
+        columns += ((table[k + 3] & 0x7fffffff) - table[k + 2] + 2 * K) * (table[k + 3] < 0 ? 1.25 : 1.0);
+    const double slots = std::min((double)table.size() / 4, (double)march_chip(a[0]));
+    const double per_cu = 256.0 / a[0].cus;
+    const double single = a[0].storage == kF64 ? 10.0 + (0.8e-3 * segments + 8e-6 * wet) * per_cu
+                                               : 11.0 + (0.3e-3 * segments + 12e-6 * wet) * per_cu;
+    return columns / slots < single;
+}
+
 int64_t tiles_of(const LatticeShape &a, TileShape t)
 {
     const int64_t r = t.rows - 2 * t.halo, c = t.cols - 2 * t.halo;

@@ -54,6 +54,9 @@ bool march_pays(const LatticeShape &a);
 // [j0, j1) (sign bit of j1: perimeter window).
 void march_table(const LatticeShape *a, int64_t samples, int32_t K, std::vector<int32_t> &table);
 void march_table(const LatticeShape *a, int64_t samples, int32_t K, int32_t cols, std::vector<int32_t> &table);
+// Whether an ensemble's launches of that table are faster than its one-step
+// kernels, by the samples' wet nodes.
+bool ensemble_pays(const LatticeShape *a, int64_t samples, int32_t K, const std::vector<int32_t> &table);
 
 // Region of a tile, and the steps per launch it holds (halo 0: no tiles for
 // this lattice).

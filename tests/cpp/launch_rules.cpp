@@ -10,6 +10,7 @@
 //                            table, whether they cover every sample once, and
 //                            the longest wave without perimeter nodes
 //                            (COLS 0: the library's choice)
+//   ensemble K               ensemble_pays
 #include "../../latticeboltzmannmethod-fonnesu-grassi-guffanti_amd/csrc/lbm_plan.h"
 
 #include <algorithm>
@@ -105,6 +106,11 @@ int main()
         } else if (what == "cover") {
             in >> K;
             std::cout << covered(a, K);
+        } else if (what == "ensemble") {
+            in >> K;
+            std::vector<int32_t> table;
+            march_table(samples.data(), (int64_t)samples.size(), K, table);
+            std::cout << ensemble_pays(samples.data(), (int64_t)samples.size(), K, table);
         } else if (what == "table") {
             in >> K >> cols;
             std::vector<int32_t> table;

@@ -104,3 +104,48 @@ def test_mostly_dry_lattices_take_single_steps(storage):
             out.append(lat.populations())
         assert np.array_equal(out[0], out[1]) and np.array_equal(out[0], out[2])
         lat.close()
+
+
+@pytest.mark.parametrize("storage", [L.F64, L.F32_SHIFTED])
+def test_ensembles_of_any_shape_keep_their_bits(storage):
+    """Several steps per launch asked for, whatever the rule says: samples of
+    every small size, mostly dry ones, wet first and last rows."""
+    rng = np.random.default_rng(23)
+    classes = [random_class(rng, nr, nc, 0.15) for nr, nc in [(3, 3), (5, 9), (57, 10), (56, 11), (64, 12), (113, 40),
+                                                              (200, 64), (129, 300)]]
+    for nr, nc in ((300, 200), (128, 400)):
+        dry = np.full((nc, nr), L.OBSTACLE, np.uint8)
+        dry[1:20, 1:nr - 1] = L.FLUID
+        classes.append(dry)
+    lids = np.zeros((250, 64), np.uint8)
+    lids[0] = lids[-1] = L.BOUNDARY
+    lids[1:-1, 0], lids[1:-1, -1] = L.INLET, L.OUTLET
+    classes += [lids] * 3
+    states = [state(rng, *c.shape) for c in classes]
+    out = []
+    for k in (1, 4, 0):
+        lats = [make(c, np.random.default_rng(s), storage, L.BGK, POLICIES[:2]) for s, c in enumerate(classes)]
+        for lat, p in zip(lats, states):
+            lat.upload_populations(p)
+        with L.Batch(lats) as b:
+            b.set_steps_per_launch(k)
+            assert k == 0 or b.steps_per_launch() == k
+            b.step(47)
+        out.append([lat.populations() for lat in lats])
+        for lat in lats:
+            lat.close()
+    for s in range(len(classes)):
+        assert np.array_equal(out[0][s], out[1][s]) and np.array_equal(out[0][s], out[2][s]), classes[s].shape
+
+
+@pytest.mark.parametrize("storage", [L.F64, L.F32_SHIFTED])
+def test_mostly_dry_ensembles_take_single_steps(storage):
+    nr = nc = 512
+    for wet, steps in ((0.1, 1), (1.0, 4)):
+        cls = np.full((nc, nr), L.OBSTACLE, np.uint8)
+        cls[1:int(wet * (nc - 2)), 1:nr - 1] = L.FLUID
+        lats = [L.Lattice(cls, storage=storage, tau=0.8) for _ in range(6)]
+        with L.Batch(lats) as b:
+            assert b.steps_per_launch() == steps
+        for lat in lats:
+            lat.close()

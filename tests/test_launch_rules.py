@@ -110,3 +110,16 @@ def test_lattices_that_march(rules, storage):
           shape(storage, 44000, 10, wet=0.6), shape(storage, 400000, 12, wet=0.7)]
     got = rules(*sum([[s, "pays"] for s in yes + no], []))
     assert [x for x, in got] == [1] * len(yes) + [0] * len(no)
+
+
+@pytest.mark.parametrize("storage", [F64, F32])
+def test_ensembles_that_march(rules, storage):
+    """Single steps where the samples are mostly dry, whose one-step table
+    holds only segments with wet nodes."""
+    for n, size, wet, segments, march in ((32, 700, 0.7, 1.0, 1), (512, 400, 0.6, 1.0, 1), (16, 512, 1.0, 1.0, 1),
+                                          (16, 512, 0.05, 0.05, 0), (12, 1024, 0.05, 0.16, 0), (12, 1024, 0.1, 0.27, 0),
+                                          (64, 128, 0.05, 0.1, 0), (2, 1024, 0.2, 0.22, 0), (16, 512, 0.2, 0.22, 0)):
+        one = shape(storage, size, size, wet=wet, segments=segments)
+        assert rules(*[one, "add"] * n, "ensemble 4")[0] == [march], (n, size, wet)
+    lids = shape(storage, 256, 256, True)
+    assert rules(*[lids, "add"] * 10, "ensemble 4")[0] == [1]
