@@ -3,6 +3,8 @@
 //   shape STORAGE PSBB NR NC TOP BOTTOM CUS WET SEGMENTS   the lattice of what follows
 //   steps                    march_steps, rows, columns and halo of its tiles
 //   pays                     march_pays
+//   tiles                    tiles_pay, and tile_min_steps without and with
+//                            waiting values
 //   plan K                   the numbers of march_plan
 //   cover K                  whether each row and column of a launch of K
 //                            steps belongs to one wave, in the kernel's numbering
@@ -98,6 +100,8 @@ int main()
             std::cout << march_steps(a) << " " << t.rows << " " << t.cols << " " << t.halo;
         } else if (what == "pays") {
             std::cout << march_pays(a);
+        } else if (what == "tiles") {
+            std::cout << tiles_pay(a) << " " << tile_min_steps(a, false) << " " << tile_min_steps(a, true);
         } else if (what == "plan") {
             in >> K;
             const MarchPlan m = march_plan(a, K);

@@ -149,3 +149,36 @@ def test_mostly_dry_ensembles_take_single_steps(storage):
             assert b.steps_per_launch() == steps
         for lat in lats:
             lat.close()
+
+
+@pytest.mark.parametrize("storage,nr,nc", [(L.F64, 100, 120), (L.F64, 300, 310), (L.F32_SHIFTED, 200, 210),
+                                           (L.F32_SHIFTED, 400, 410), (L.F16_SHIFTED, 300, 310),
+                                           (L.F16_SHIFTED, 1230, 1240), (L.F64, 9000, 4)])
+@pytest.mark.parametrize("psbb", [False, True])
+def test_calls_of_few_steps(storage, nr, nc, psbb):
+    """Runs that mix tile launches and single steps, fields and new values
+    among them, against single steps throughout."""
+    if psbb and (storage != L.F64 or nc < 8):
+        pytest.skip("FP64 only")
+    rng = np.random.default_rng(nr)
+    cls = random_class(rng, nr, nc, 0.1)
+    p0 = state(rng, nc, nr)
+    lats = [make(cls, np.random.default_rng(1), storage, L.TRT, POLICIES[:2]) for _ in range(2)]
+    k = len(lats[0].open_nodes(0))
+    b = rng.random(int(lats[0].node_counts()[6]))
+    for lat, flags in zip(lats, (0, L.STEP_NO_GRAPH)):
+        if psbb:
+            lat.set_partial_bounce_back(0.9, b)
+        lat.upload_populations(p0)
+        for n in (1, 1, 2, 1, 10, 1, 3, 2, 11, 73, 1):
+            lat.step(n, flags | (L.STEP_MACRO if n % 2 else 0))
+        for n in (1, 2, 1, 10):
+            lat.set_open_values(0, ux=np.full(k, 0.001 * n))
+            lat.step(n, flags)
+            lat.step(1, flags | L.STEP_MACRO | L.STEP_CHECK)
+    a, c = lats
+    assert np.array_equal(a.populations(), c.populations())
+    for x, y in zip(a.macro(), c.macro()):
+        assert np.array_equal(x, y)
+    for lat in lats:
+        lat.close()

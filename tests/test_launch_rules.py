@@ -123,3 +123,21 @@ def test_ensembles_that_march(rules, storage):
         assert rules(*[one, "add"] * n, "ensemble 4")[0] == [march], (n, size, wet)
     lids = shape(storage, 256, 256, True)
     assert rules(*[lids, "add"] * 10, "ensemble 4")[0] == [1]
+
+
+def test_calls_of_few_steps_in_tiles(rules):
+    """A tile launch of one or two steps only where it is the faster one: the
+    smallest lattices, shallow ones, or with new values waiting."""
+    want = {(F64, 129, 129): (1, 1, 1), (F64, 200, 200): (1, 2, 1), (F64, 545, 545): (1, 2, 1),
+            (F32, 250, 250): (1, 1, 1), (F32, 300, 300): (1, 2, 1), (F32, 545, 545): (1, 2, 1),
+            (F16, 310, 310): (1, 1, 1), (F16, 400, 400): (1, 2, 1), (F16, 600, 600): (1, 2, 1),
+            (F16, 850, 850): (1, 2, 1), (F16, 1240, 1240): (1, 3, 1),
+            (F64, 40, 96): (1, 1, 1), (F64, 96666, 3): (0, 3, 1), (F32, 40000, 5): (1, 3, 1),
+            (F64, 20000, 3): (1, 2, 1), (F64, 10000, 3): (1, 2, 1), (F64, 36250, 8): (1, 2, 1)}
+    got = rules(*sum([[shape(*k), "tiles"] for k in want], []))
+    assert {k: tuple(x) for k, x in zip(want, got)} == want
+    got = rules(*sum([[shape(F64, n, n, psbb=True), "tiles"] for n in (60, 129, 300, 400, 545)], []))
+    assert [tuple(x) for x in got] == [(1, 2, 1)] * 3 + [(1, 3, 1)] * 2
+    # a wet first row makes the one-step kernels slow
+    got = rules(*sum([[shape(st, 3, 20000, True), "tiles"] for st in (F64, F32, F16)], []))
+    assert [x[1] for x in got] == [1, 1, 1]
