@@ -140,9 +140,11 @@ Launching launching(const lbm_ctx *c)
     const int32_t most = c->max_steps == 0 ? INT32_MAX : c->max_steps;
     if (most > 1) {
         const LatticeShape a = shape_of(c);
-        if (const int32_t k = tile_shape(a).halo) return {Launching::kTile, std::min(k, most)};
+        const bool asked = c->max_steps > 0;
+        if (const int32_t k = tile_shape(a).halo; k > 0 && (asked || tiles_pay(a)))
+            return {Launching::kTile, std::min(k, most)};
         const int32_t k = march_steps(a);
-        if (k > 0 && (c->max_steps > 0 || march_pays(a))) return {Launching::kMarch, std::min(k, most)};
+        if (k > 0 && (asked || march_pays(a))) return {Launching::kMarch, std::min(k, most)};
     }
     return {Launching::kSingle, 1};
 }
@@ -1095,7 +1097,8 @@ int lbm_step(lbm_ctx *c, int64_t n, uint32_t flags)
         // values) every launch takes the same steps on alternating buffers:
         // replay a captured loop of them, then launch the rest, as many
         // steps at a time as are left.  Tiles also take the steps with new
-        // values and the one that writes the fields.
+        // values and the one that writes the fields, unless so few are left
+        // that single steps are faster.
         const bool steady = c->state == kFstar && c->bc_prev == c->bc_cur;
         const int64_t left = n - s, plain = left - (macro ? 1 : 0);
         if (!(flags & LBM_STEP_NO_GRAPH)) {
@@ -1116,7 +1119,8 @@ int lbm_step(lbm_ctx *c, int64_t n, uint32_t flags)
                 k = (int32_t)(plain == how.steps + 1 ? plain - 2 : std::min<int64_t>(plain, how.steps));
             } else if (how.kind == Launching::kTile && c->state == kFstar) {
                 k = (int32_t)std::min<int64_t>(left, how.steps);
-                if (macro && k == left) {
+                if (k < std::min(how.steps, tile_min_steps(shape_of(c), c->bc_pending))) k = 0;
+                if (macro && k > 0 && k == left) {
                     int r = claim_macro(c, &fields);
                     if (r) return r;
                 }

@@ -260,4 +260,67 @@ TileShape tile_shape(const LatticeShape &a)
     return {32, 32, 4};
 }
 
+// Lattices of a few columns leave most of each tile outside.  us a step, one
+// step a launch / tiles: 3 columns, 40000 rows FP64 9.5 / 12.0, 96666 rows 14.1
+// / 26.8, FP32 10.0 / 14.1, FP16 10.4 / 15.4; 5 columns, 58000 rows FP64 14.4 /
+// 17.7; but 5 columns, 24000 rows FP32 8.4 / 4.9.
+bool tiles_pay(const LatticeShape &a)
+{
+    return a.nc > 5 || tiles_of(a, tile_shape(a)) <= (a.storage == kF64 ? 6 : 10) * (int64_t)a.cus;
+}
+
+namespace {
+
+// us of one step by the one-step kernels, and of a tile launch of one, of
+// lattices below kTileMaxNodes (FP16: kTileMaxNodesF16), as fitted to 230 of
+// them per format (calls of one step; to 5 % and to 15 to 20 %).
+struct StepCost {
+    double base, segments, wet_segments, perimeter, wet;  // the last four per million
+    double tile_base, tile;                               // per round of one tile per CU
+};
+constexpr StepCost kStepCost[3] = {{8.4, 0, 590, 730, 9.4, 2.9, 5.25},
+                                   {7.0, 430, 0, 450, 5.3, 4.0, 2.47},
+                                   {7.6, 580, 0, 650, 0, 3.9, 2.33}};
+
+double one_step_us(const LatticeShape &a)
+{
+    const StepCost &c = kStepCost[a.storage];
+    const int64_t rows = (a.nr + 63) / 64;
+    const int64_t perimeter = (a.wet_top ? a.nc : 0) + (a.wet_bottom && rows > 1 ? a.nc : 0) + 2 * rows;
+    return c.base + 1e-6 * (c.segments * (double)(rows * a.nc) + c.wet_segments * (double)a.wet_segments +
+                            c.perimeter * (double)perimeter + c.wet * (double)a.wet);
+}
+
+double tile_us(const LatticeShape &a, int64_t tiles)
+{
+    const StepCost &c = kStepCost[a.storage];
+    return c.tile_base + c.tile * std::max(1.0, (double)tiles / a.cus);
+}
+
+}  // namespace
+
+// A launch in tiles loads and stores its halo whatever its steps, so one of a
+// single step, or two, is slower than one-step launches except on the smallest
+// lattices, and on shallow ones, whose perimeter segments are slow in one-step
+// launches.  us a step by calls of one step, one-step kernels / tiles: FP64 129^2
+// 8.5 / 7.4, 200^2 8.8 / 9.4, 545^2 15.2 / 20.7; FP32 250^2 7.9 / 8.1, 545^2 10.7
+// / 14.3; FP16 320^2 9.2 / 9.1, 1240^2 19.6 / 37.4; first row wet, 3 x 20000 FP64
+// 34.9 / 25.1; FP64 with partially saturated obstacles (one kernel a step) 60^2
+// 4.7 / 6.3, 545^2 11.0 / 19.9.  Of two: FP16 1100^2 the same, 1240^2 19.7 / 21.8;
+// 50000 x 4 FP64 12.8 / 18.2; partially saturated 200^2 5.5 / 5.7, 400^2 8.5 / 10.0.
+// Where new values wait, a one-step launch takes their copy, of about 10 us, with
+// it: one step with new values FP16 500^2 32.7 / 14.5, 600^2 31.1 / 14.2 (they
+// wait up to nr + nc = 1365).
+int32_t tile_min_steps(const LatticeShape &a, bool waiting)
+{
+    const int64_t nodes = a.nr * a.nc, tiles = tiles_of(a, tile_shape(a)), cus = a.cus;
+    if (waiting) return 1;
+    if (a.psbb) return tiles <= cus ? 2 : 3;
+    const int64_t small = a.storage == kF64 ? 32768 : a.storage == kF32 ? 65000 : 110000;
+    const double margin = a.storage == kF64 ? 0.78 : 0.9, single = one_step_us(a), tile = tile_us(a, tiles);
+    if (nodes < small && tiles <= (a.storage == kF64 ? 1 : 2) * cus) return 1;
+    if (tiles > cus && tile < margin * single) return 1;
+    return tiles <= (a.nc < 8 ? 5 : 14) * cus || 1.3 * tile < margin * 2.0 * single ? 2 : 3;
+}
+
 }  // namespace lbm
