@@ -1116,7 +1116,8 @@ int lbm_step(lbm_ctx *c, int64_t n, uint32_t flags)
             double *fields = nullptr;
             if (how.kind == Launching::kMarch && steady && plain >= 2) {
                 // no single step is left over where two launches can share the rest
-                k = (int32_t)(plain == how.steps + 1 ? plain - 2 : std::min<int64_t>(plain, how.steps));
+                const bool share = plain == how.steps + 1 && how.steps > 2;
+                k = (int32_t)(share ? plain - 2 : std::min<int64_t>(plain, how.steps));
             } else if (how.kind == Launching::kTile && c->state == kFstar) {
                 k = (int32_t)std::min<int64_t>(left, how.steps);
                 if (k < std::min(how.steps, tile_min_steps(shape_of(c), c->bc_pending))) k = 0;

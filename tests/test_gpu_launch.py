@@ -151,15 +151,13 @@ def test_mostly_dry_ensembles_take_single_steps(storage):
             lat.close()
 
 
-@pytest.mark.parametrize("storage,nr,nc", [(L.F64, 100, 120), (L.F64, 300, 310), (L.F32_SHIFTED, 200, 210),
-                                           (L.F32_SHIFTED, 400, 410), (L.F16_SHIFTED, 300, 310),
-                                           (L.F16_SHIFTED, 1230, 1240), (L.F64, 9000, 4)])
-@pytest.mark.parametrize("psbb", [False, True])
+@pytest.mark.parametrize("storage,nr,nc,psbb", [
+    (L.F64, 100, 120, False), (L.F64, 300, 310, False), (L.F64, 9000, 4, False), (L.F32_SHIFTED, 200, 210, False),
+    (L.F32_SHIFTED, 400, 410, False), (L.F16_SHIFTED, 300, 310, False), (L.F16_SHIFTED, 1230, 1240, False),
+    (L.F64, 100, 120, True), (L.F64, 300, 310, True), (L.F64, 500, 510, True)])
 def test_calls_of_few_steps(storage, nr, nc, psbb):
     """Runs that mix tile launches and single steps, fields and new values
     among them, against single steps throughout."""
-    if psbb and (storage != L.F64 or nc < 8):
-        pytest.skip("FP64 only")
     rng = np.random.default_rng(nr)
     cls = random_class(rng, nr, nc, 0.1)
     p0 = state(rng, nc, nr)
@@ -182,3 +180,26 @@ def test_calls_of_few_steps(storage, nr, nc, psbb):
         assert np.array_equal(x, y)
     for lat in lats:
         lat.close()
+
+
+@pytest.mark.parametrize("storage", [L.F64, L.F32_SHIFTED])
+@pytest.mark.parametrize("options", [0, L.OPT_PLANAR_LAYOUT])
+@pytest.mark.parametrize("nr,nc", [(57, 5301), (64, 4700), (33400, 9), (30100, 10), (27300, 11), (25100, 12), (23100, 13)])
+def test_asked_for_where_the_rule_says_no(nr, nc, options, storage):
+    """Several steps per launch on lattices that take single ones by
+    themselves: narrow ones with many solid nodes, windows all at the
+    perimeter."""
+    rng = np.random.default_rng(nr)
+    cls = random_class(rng, nr, nc, 0.4)
+    p0 = state(rng, nc, nr)
+    out = []
+    for k in (1, 2, 3, 4):
+        lat = L.Lattice(cls, tau=0.8, inlet_policy=L.ZOUHE_PRESSURE, outlet_policy=L.OPEN_NOOP, storage=storage,
+                        options=options)
+        lat.set_steps_per_launch(k)
+        assert lat.steps_per_launch() == k
+        lat.upload_populations(p0)
+        lat.step(44, L.STEP_CHECK)
+        out.append(lat.populations())
+        lat.close()
+    assert all(np.array_equal(out[0], x) for x in out[1:])
