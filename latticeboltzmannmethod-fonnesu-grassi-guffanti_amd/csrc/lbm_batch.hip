@@ -11,7 +11,7 @@
 // FP32, unless a launch shape was set by hand.
 //
 // Parity bookkeeping: sample s's state is in buffer base_cur[s] ^ phase,
-// where phase counts the ensemble's steps mod 2 since the sample's
+// where phase counts the ensemble's launches mod 2 since the sample's
 // arguments were last built; args[2 s + p] reads buffer base_cur[s] ^ p.
 #include <hip/hip_runtime.h>
 

@@ -1897,7 +1897,7 @@ __global__ __launch_bounds__(kBlockRows) void fill_macro(double *macro, int64_t 
 
 // Copies a [3][n] field's parts to rho (n doubles) and u (2 n), either
 // nullptr: page-locked host memory, for fields too small to be worth a copy
-// engine's start (download_fields).
+// engine's start.
 __global__ __launch_bounds__(kBlockRows) void copy_fields(const double *macro, int64_t n, double *rho, double *u)
 {
     const int64_t q = (int64_t)blockIdx.x * kBlockRows + threadIdx.x;

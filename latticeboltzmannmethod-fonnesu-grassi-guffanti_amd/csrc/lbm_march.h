@@ -25,16 +25,20 @@
 // What bounds it: in FP32 the VALU (busy throughout on porous media, 0.85 on
 // unobstructed ones, which load at 4.5 TB/s meanwhile; 122 instructions per
 // level and lane, of which the collision takes 110), in FP64 the VALU at 0.8
-// and latency (two waves per SIMD: nine values per level stay in
-// registers).  us a step, before (one step a launch, tuned) -> K = 4 (FP32),
-// 5 (FP64): porous 8192^2 FP32 561 -> 254; open 4096^2 FP64 419 -> 121; TRT
-// cavity 4096^2 FP32 194 -> 77, FP64 416 -> 157; porous 4096^2 FP64 303 -> 112.
-// K = 2 / 3 / 4 / 5 on the porous 4096^2 (before FUSED): FP64 211 / 146 / 119
-// / 114, FP32 121 / 78 / 71 / 74: the launch stays near 550 us (FP64) up to K = 4, where
-// memory binds it, and the lanes and columns lost to the window's ends
-// outweigh the traffic beyond.  FP16 keeps one step a launch: its rounding
-// takes another 50 instructions per node, and it was at the VALU limit with
-// one step.
+// and latency.  FP64 at K = 5 takes 197 registers, so two waves per SIMD; at
+// K = 4 the fused moves take 164 and three fit, but the columns are dealt for
+// two.  FP32 at K = 4 takes 132 and three waves fit; its copy for planes keeps
+// 68 bytes a lane in scratch memory besides.  us a step, before (one step a
+// launch) -> K = 4 (FP32), 5 (FP64): porous 8192^2 FP32 549 (tuned; 602
+// untuned) -> 252; open 4096^2 FP64 419 -> 121; TRT cavity 4096^2 FP32 194 ->
+// 77, FP64 416 -> 157; porous 4096^2 FP64 303 -> 112.  K = 2 / 3 / 4 / 5 on the
+// porous 4096^2 (without FUSED): FP64 211 / 146 / 119 / 114, FP32 121 / 78 / 71
+// / 74.  In FP64 a launch grows from 420 us at K = 2 to 475 at K = 4, its
+// traffic alike, and to 570 at K = 5: from there on the levels cost what the
+// traffic saves, and the lanes and columns lost to the window's ends more.
+// FP16 keeps one step a launch: its rounding takes another 50 instructions
+// per node, and it was at the VALU limit with one step; marching FP16 has not
+// been built.
 
 // One column's 64-row window of a marching wave (rows i0 .. i0 + 63), all
 // wave-uniform: bit l of mid / up / dn is the wet bit of row i0 + l, of the
@@ -93,10 +97,8 @@ __device__ __forceinline__ T lane_shift(T v)
         u.x = lane_move<CTRL>(u.x);
         u.y = lane_move<CTRL>(u.y);
         return __builtin_bit_cast(T, u);
-    } else if constexpr (sizeof(T) == 4) {
-        return __builtin_bit_cast(T, lane_move<CTRL>(__builtin_bit_cast(uint32_t, v)));
     } else {
-        return __builtin_bit_cast(T, (uint16_t)lane_move<CTRL>(__builtin_bit_cast(uint16_t, v)));
+        return __builtin_bit_cast(T, lane_move<CTRL>(__builtin_bit_cast(uint32_t, v)));
     }
 }
 

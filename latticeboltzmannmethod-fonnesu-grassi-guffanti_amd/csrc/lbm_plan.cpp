@@ -7,7 +7,10 @@ namespace lbm {
 
 namespace {
 
-// Waves per SIMD the marching kernels' registers allow.
+// Waves per SIMD that the columns are dealt for.  The kernels' registers allow
+// as many or more: FP64 two at 5 steps (197 VGPRs) and 4 unfused (194), three
+// at 2, 3 and 4 fused (138, 166, 164); FP32 three at 4 (132 fused, 148), four at 3
+// (119), five at 2 (90).  The chunk lengths below were measured with these.
 int64_t march_waves(int32_t storage) { return storage == kF64 ? 2 : 3; }
 
 // Deals the columns to waves.  A wave computes cols + 2 K columns' levels
@@ -66,8 +69,9 @@ MarchPlan march_stripes(const LatticeShape &a, int32_t K)
 // A launch of marching waves takes at least the time one wave needs for its
 // columns (30 us at K = 4 in FP64, half of it in FP32; more where the top
 // or bottom row is wet): small lattices take tiles (tile_shape).  FP64 at
-// K = 5 is 5-7 % faster than K = 4 on 4096^2 (BGK; the same in TRT) and
-// slower on small lattices.
+// K = 5 against K = 4, us a step (columns dealt for two waves per SIMD in both):
+// porous 4096^2 104.4 / 113.5, TRT cavity 4096^2 141.4 / 150.3, open 3001 x 5003
+// 122.0 / 125.3, 8192^2 523 / 613, 2100^2 40.1 / 40.7; slower on small lattices.
 int32_t march_steps(const LatticeShape &a)
 {
     const int64_t nodes = a.nr * a.nc;
@@ -195,13 +199,13 @@ void march_table(const LatticeShape *a, int64_t samples, int32_t K, int32_t cols
 // A marching launch walks every window, wet or not; an ensemble's one-step
 // kernels have a table of the segments that hold a wet node and take only
 // those.  The launch takes as long as the columns that fall to one slot of the
-// chip (kMarchWaves a SIMD, edge columns a quarter more); four single steps
+// chip (march_waves a SIMD, edge columns a quarter more); four single steps
 // cost a fixed time, one per segment and one per wet node, in the same unit of
 // about 2.5 us.  Fitted to 90 ensembles per format: 131072 to 12 million nodes,
 // lattices of 16 x 16 to 1024^2, 2 to 1000 of them, channels, cavities, porous
 // and mostly dry media, wet first and last rows.  Single steps were up to 6 times
 // faster on 27 of them, and marching up to 2.8 on the others; the rule errs by up
-// to 15 %, where the two are close.  us a step, one step a launch /
+// to 17 %, where the two are close.  us a step, one step a launch /
 // marching: 16 lattices of 512^2, 5 / 20 / 50 % of each wet, FP64 7.8 / 33.5,
 // 24.5 / 34.1, 50.7 / 34.4; FP32 5.9 / 22.4, 13.6 / 23.2, 26.8 / 23.3.
 bool ensemble_pays(const LatticeShape *a, int64_t samples, int32_t K, const std::vector<int32_t> &table)

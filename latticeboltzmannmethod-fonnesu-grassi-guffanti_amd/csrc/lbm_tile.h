@@ -19,15 +19,20 @@
 //
 // What bounds it: latency.  A launch costs about 5 us and a step 1.2 us in
 // FP64 (a gather from LDS, a barrier, the collision's dependent chain, a
-// store, a barrier).  us a step, single steps -> tiles: 129^2 cavity FP64 7.7
-// -> 1.85, FP32 7.1 -> 1.45, FP16 7.9 -> 1.7; channel 40 x 96 FP64 7.0 -> 1.7;
-// 300^2 FP64 9.1 -> 3.3; 251 x 1003 FP32 9.6 -> 4.6.
+// store, a barrier); the vector ALUs are busy for 18 % of a launch on the
+// 129^2 cavity in FP64 (40 % on 251 x 1003 in FP32), the waves wait for 58 %
+// (50 %) of their cycles, and bank conflicts take below 1 % of the LDS's.  us
+// a step in long runs, single steps -> tiles: 129^2 cavity FP64 7.7 -> 1.85,
+// FP32 7.1 -> 1.45, FP16 7.9 -> 1.7; channel 40 x 96 FP64 7.0 -> 1.7; 300^2 FP64
+// 9.1 -> 3.3; 251 x 1003 FP32 9.6 -> 4.6.  Launches of one step or two are
+// another matter (tile_min_steps).
 //
 // Same arithmetic per node as the step kernels, same bits.
 // PS: partially saturated obstacles (FP64).  A node keeps the populations
 // that enter it through its obstacle slots, and their weights, in registers
 // (psbb_gather, psbb_update); its carried values alternate between two
-// buffers like the state, since the tiles around it read the old ones.
+// buffers like the state, since the tiles around it read the old ones.  At 32
+// x 32 two of its registers spill (12 bytes a lane of scratch memory).
 template <typename T, int kRows, int kCols, bool PS = false>
 __global__ __launch_bounds__(kRows * kCols) void tile_kernel(StepArgs a, int32_t steps, int32_t halo, int32_t tiles_i)
 {
