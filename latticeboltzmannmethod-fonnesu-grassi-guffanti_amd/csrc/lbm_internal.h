@@ -73,6 +73,10 @@ struct StepArgs {
     int32_t esize;          // bytes per stored population
     int32_t wpc;            // step kernel: waves per column
     int64_t nblocks;
+    // Unused.  How the kernels' scalar loads of their arguments combine, and in
+    // FP64 which scalars the marching kernels spill, follows from the offsets
+    // of what comes next: these 16 bytes keep those that were measured.
+    int64_t unused[2];
     double bgk_t, bgk_omt;              // 1/tau, 1 - 1/tau
     double trt_inv_te, trt_a, trt_b;    // 1/tau+, 0.5/tau+, 0.5/tau-
     float sh_a, sh_b;                   // shifted paths: 0.5/tau+, 0.5/tau- (BGK: both 0.5/tau)

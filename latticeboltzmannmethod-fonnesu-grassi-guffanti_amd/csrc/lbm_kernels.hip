@@ -2027,7 +2027,7 @@ hipError_t launch_step_t(bool gather, StepArgs a, hipStream_t s)
 template <typename T, int K>
 hipError_t launch_march_t(StepArgs a, const MarchPlan &m, hipStream_t s)
 {
-    a.nblocks = (m.waves + kBlockRows / 64 - 1) / (kBlockRows / 64);
+    a.nblocks = (march_launch_waves(m, a.g.nc, K) + kBlockRows / 64 - 1) / (kBlockRows / 64);
     const dim3 grid((unsigned)a.nblocks), block(kBlockRows);
     // K = 5: large lattices only.  Lattices in planes, which are large unless
     // that layout was asked for, have the fused copy only at K = 4.

@@ -126,7 +126,6 @@ MarchPlan march_plan(const LatticeShape &a, int32_t K)
             break;
         }
     }
-    m.waves = m.edge_waves + (inner > 0 ? inner * ((free_cols + m.cols - 1) / m.cols) : 0);
     return m;
 }
 

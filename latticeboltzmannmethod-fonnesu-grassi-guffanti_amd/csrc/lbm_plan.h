@@ -37,8 +37,13 @@ struct MarchPlan {
     int32_t edge_chunks;     // waves per edge stripe
     int32_t edge_row_waves;  // waves of the edge stripes
     int32_t edge_waves;      // and with the first and last columns of the others, rounded up to whole work-groups
-    int64_t waves;           // all of the launch
 };
+// Waves of a launch of K steps of a lattice of nc columns.
+inline int64_t march_launch_waves(const MarchPlan &m, int64_t nc, int32_t K)
+{
+    const int64_t inner = m.stripes - m.top - m.bottom;
+    return m.edge_waves + (inner > 0 ? inner * ((nc - 2 * (K + 1) + m.cols - 1) / m.cols) : 0);
+}
 
 // Steps per launch of the marching kernel for this lattice (0: not for it),
 // and the deal of a launch of K of them.

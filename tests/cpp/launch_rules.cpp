@@ -48,7 +48,7 @@ bool covered(const LatticeShape &a, int32_t K)
 {
     const MarchPlan m = march_plan(a, K);
     const int64_t rows = 64 - 2 * K, inner = m.stripes - m.top - m.bottom;
-    const int64_t blocks = (m.waves + 3) / 4;
+    const int64_t blocks = (march_launch_waves(m, a.nc, K) + 3) / 4;
     Cover c(a.nr, a.nc);
     for (int64_t w = 0; w < 4 * blocks; ++w) {
         int64_t t = w;
@@ -106,7 +106,7 @@ int main()
             in >> K;
             const MarchPlan m = march_plan(a, K);
             std::cout << m.stripes << " " << m.top << " " << m.bottom << " " << m.cols << " " << m.edge_cols << " "
-                      << m.edge_row_waves << " " << m.edge_waves << " " << m.waves;
+                      << m.edge_row_waves << " " << m.edge_waves << " " << march_launch_waves(m, a.nc, K);
         } else if (what == "cover") {
             in >> K;
             std::cout << covered(a, K);
