@@ -301,8 +301,8 @@ int lbm_get_scale(lbm_ctx *ctx, double *scale);
  * lane's neighbour addressing read from a table built on first use (4 bytes
  * per wet node and step more traffic, far fewer instructions per wave).
  * Results are the same bits for every shape.  With 0 (the default), steps
- * run several to a launch where the lattice allows it (small lattices;
- * larger ones in FP64 and FP32 storage); a shape set here is a launch of one
+ * run several to a launch where the lattice allows it and that is faster
+ * (small lattices; larger ones in FP64 and FP32 storage); a shape set here is a launch of one
  * step.  lbm_get_launch reports the shape of single steps, which also take
  * the steps that several to a launch leave over.  No counterpart in the
  * reference (a tuning knob of this engine). */
