@@ -8,9 +8,10 @@
 
 namespace lbm {
 
-// Copies `bytes` on stream s and waits for them: what hipMemcpyAsync and
-// hipStreamSynchronize do, and done by these for small copies and for
-// page-locked host memory.  `device` is the stream's.
+// Copies `bytes` on stream s: what hipMemcpyAsync does, and done by it for
+// small copies and for page-locked host memory.  To the host the copy is
+// waited for; to the device it may be in flight, and the caller waits for the
+// stream before the memory may change.  `device` is the stream's.
 hipError_t copy_to_host(int device, void *dst, const void *src, size_t bytes, hipStream_t s);
 hipError_t copy_to_device(int device, void *dst, const void *src, size_t bytes, hipStream_t s);
 

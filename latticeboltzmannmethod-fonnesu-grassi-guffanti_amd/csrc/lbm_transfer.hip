@@ -44,7 +44,7 @@ bool pageable(const void *p)
 hipError_t plain(void *dst, const void *src, size_t bytes, hipMemcpyKind kind, hipStream_t s)
 {
     const hipError_t e = hipMemcpyAsync(dst, src, bytes, kind, s);
-    return e != hipSuccess ? e : hipStreamSynchronize(s);
+    return e != hipSuccess || kind == hipMemcpyHostToDevice ? e : hipStreamSynchronize(s);
 }
 
 // One lane's chunks of a copy.

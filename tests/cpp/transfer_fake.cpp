@@ -22,6 +22,7 @@ std::vector<Copy> queue;         // copies in flight
 bool earlier = false;            // steps queued before the call are still running
 bool lane_waited = false;        // a copy was queued, or waited for, behind those steps
 bool fail_records = false;
+int waits = 0;                   // for the whole stream
 const char *pinned = nullptr;    // page-locked range
 size_t pinned_bytes = 0;
 
@@ -47,6 +48,7 @@ hipError_t hipMemcpyAsync(void *dst, const void *src, size_t n, hipMemcpyKind, h
 hipError_t hipStreamSynchronize(hipStream_t)
 {
     std::lock_guard<std::mutex> lock(mu);
+    ++waits;
     drain();
     return hipSuccess;
 }
@@ -119,7 +121,11 @@ int main(int argc, char **argv)
         require(a == b, "down differs");
         std::fill(b.begin(), b.end(), 0);
         require(lbm::copy_to_device(0, b.data(), a.data(), a.size(), nullptr) == hipSuccess, "up failed");
+        (void)hipStreamSynchronize(nullptr);  // the caller's part
         require(a == b, "up differs");
+    } else if (what == "queued") {
+        require(lbm::copy_to_device(0, b.data(), a.data(), 1 << 20, nullptr) == hipSuccess, "up failed");
+        require(waits == 0 && queue.size() == 1 && queue[0].n == 1 << 20, "a small upload was waited for");
     } else if (what == "earlier") {
         earlier = true;
         require(lbm::copy_to_host(0, b.data(), a.data(), a.size(), nullptr) == hipSuccess, "down failed");

@@ -48,3 +48,8 @@ def test_failed_lane_leaves_nothing_in_flight(driver):
 def test_device_view_covers_the_whole_range(driver):
     """A kernel may write host memory only if all of it is page-locked."""
     _holds(driver, "view")
+
+
+def test_small_uploads_are_queued(driver):
+    """The caller queues the kernel that reads them and waits once, behind it."""
+    _holds(driver, "queued")
