@@ -105,7 +105,7 @@ hipError_t hipPointerGetAttributes(hipPointerAttribute_t *at, const void *p)
 int main(int argc, char **argv)
 {
     const std::string what = argc > 1 ? argv[1] : "";
-    const size_t n = (size_t)13 << 20;  // several rounds of the chunks and a remainder
+    const size_t n = (size_t)29 << 20;  // several rounds of the chunks and a remainder
     std::vector<char> a(n + 123), b(n + 123, 0);
     for (size_t k = 0; k < a.size(); ++k) a[k] = (char)(k * 2654435761u >> 13);
     lbm::transfer_retain();
@@ -126,6 +126,12 @@ int main(int argc, char **argv)
     } else if (what == "queued") {
         require(lbm::copy_to_device(0, b.data(), a.data(), 1 << 20, nullptr) == hipSuccess, "up failed");
         require(waits == 0 && queue.size() == 1 && queue[0].n == 1 << 20, "a small upload was waited for");
+    } else if (what == "thresholds") {
+        // 8 MB: worth the threads on the way down, not on the way up
+        const size_t m = (size_t)8 << 20;
+        require(lbm::copy_to_device(0, b.data(), a.data(), m, nullptr) == hipSuccess, "up failed");
+        require(queue.size() == 1 && queue[0].n == m, "an upload of 8 MB was cut into chunks");
+        drain();
     } else if (what == "earlier") {
         earlier = true;
         require(lbm::copy_to_host(0, b.data(), a.data(), a.size(), nullptr) == hipSuccess, "down failed");

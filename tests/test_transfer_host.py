@@ -53,3 +53,7 @@ def test_device_view_covers_the_whole_range(driver):
 def test_small_uploads_are_queued(driver):
     """The caller queues the kernel that reads them and waits once, behind it."""
     _holds(driver, "queued")
+
+
+def test_uploads_take_threads_where_they_are_faster(driver):
+    _holds(driver, "thresholds")
