@@ -133,6 +133,7 @@ constexpr int64_t kGraphLaunches = 8, kGraphSteps = 32;
 struct Launching {
     enum Kind { kSingle, kMarch, kTile } kind;
     int32_t steps;
+    TileShape tile;
 };
 
 Launching launching(const lbm_ctx *c)
@@ -141,12 +142,12 @@ Launching launching(const lbm_ctx *c)
     if (most > 1) {
         const LatticeShape a = shape_of(c);
         const bool asked = c->max_steps > 0;
-        if (const int32_t k = tile_shape(a).halo; k > 0 && (asked || tiles_pay(a)))
-            return {Launching::kTile, std::min(k, most)};
+        const TileShape t = tile_shape(a);
+        if (t.halo > 0 && (asked || tiles_pay(a, t))) return {Launching::kTile, std::min(t.halo, most), t};
         const int32_t k = march_steps(a);
-        if (k > 0 && (asked || march_pays(a))) return {Launching::kMarch, std::min(k, most)};
+        if (k > 0 && (asked || march_pays(a))) return {Launching::kMarch, std::min(k, most), {}};
     }
-    return {Launching::kSingle, 1};
+    return {Launching::kSingle, 1, {}};
 }
 
 // Steps per captured graph.
@@ -162,7 +163,7 @@ void drop_graphs(lbm_ctx *c)
 }
 
 // Launch of k steps from buffer `in`; steady ones unless the kind is kTile.
-hipError_t launch_steps(const lbm_ctx *c, Launching::Kind kind, int in, int32_t k, double *macro = nullptr)
+hipError_t launch_steps(const lbm_ctx *c, const Launching &how, int in, int32_t k, double *macro = nullptr)
 {
     StepArgs a = make_args(c);
     set_input(c, a, in);
@@ -171,8 +172,8 @@ hipError_t launch_steps(const lbm_ctx *c, Launching::Kind kind, int in, int32_t 
         a.bc_cur = c->h_bc_pin + (size_t)c->bc_slot * c->h_bc.size();
         a.bc_new = c->d_bc[c->bc_cur];
     }
-    switch (kind) {
-    case Launching::kTile: return launch_tile(c->storage, k, a, tile_shape(shape_of(c)), c->stream);
+    switch (how.kind) {
+    case Launching::kTile: return launch_tile(c->storage, k, a, how.tile, c->stream);
     case Launching::kMarch: return launch_march(c->storage, k, a, march_plan(shape_of(c), k), c->stream);
     default: return launch_step(c->storage, true, a, c->stream, c->segments);
     }
@@ -180,14 +181,14 @@ hipError_t launch_steps(const lbm_ctx *c, Launching::Kind kind, int in, int32_t 
 
 // Captures a graph's steady steps from the context's current buffer and
 // prescribed values.
-int capture_steps(lbm_ctx *c, Launching how)
+int capture_steps(lbm_ctx *c, const Launching &how)
 {
     hipGraph_t g = nullptr;
     HIP_TRY(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
     hipError_t err = hipSuccess;
     const int64_t launches = graph_steps(how.steps) / how.steps;
     for (int64_t k = 0; k < launches && err == hipSuccess; ++k)
-        err = launch_steps(c, how.kind, c->cur ^ (int)(k & 1), how.steps);
+        err = launch_steps(c, how, c->cur ^ (int)(k & 1), how.steps);
     hipError_t e2 = hipStreamEndCapture(c->stream, &g);
     if (err != hipSuccess) return fail(LBM_ERR_HIP, "step graph capture: %s", hipGetErrorString(err));
     if (e2 != hipSuccess) return fail(LBM_ERR_HIP, "hipStreamEndCapture: %s", hipGetErrorString(e2));
@@ -1120,14 +1121,14 @@ int lbm_step(lbm_ctx *c, int64_t n, uint32_t flags)
                 k = (int32_t)(share ? plain - 2 : std::min<int64_t>(plain, how.steps));
             } else if (how.kind == Launching::kTile && c->state == kFstar) {
                 k = (int32_t)std::min<int64_t>(left, how.steps);
-                if (k < std::min(how.steps, tile_min_steps(shape_of(c), c->bc_pending))) k = 0;
+                if (k < std::min(how.steps, tile_min_steps(shape_of(c), how.tile, c->bc_pending))) k = 0;
                 if (macro && k > 0 && k == left) {
                     int r = claim_macro(c, &fields);
                     if (r) return r;
                 }
             }
             if (k > 0) {
-                HIP_TRY(launch_steps(c, how.kind, c->cur, k, fields));
+                HIP_TRY(launch_steps(c, how, c->cur, k, fields));
                 c->bc_pending = false;
                 c->cur = 1 - c->cur;
                 c->bc_prev = c->bc_cur;
@@ -1291,7 +1292,7 @@ int lbm_autotune(lbm_ctx *c, int32_t steps, int32_t *segments, double *ms_per_st
     if (how.kind != Launching::kSingle) {
         auto launch = [&] {
             return how.kind == Launching::kTile
-                       ? launch_tile(c->storage, how.steps, a, tile_shape(shape_of(c)), c->stream)
+                       ? launch_tile(c->storage, how.steps, a, how.tile, c->stream)
                        : launch_march(c->storage, how.steps, a, march_plan(shape_of(c), how.steps), c->stream);
         };
         if (err == hipSuccess) err = launch();

@@ -267,9 +267,9 @@ TileShape tile_shape(const LatticeShape &a)
 // step a launch / tiles: 3 columns, 40000 rows FP64 9.5 / 12.0, 96666 rows 14.1
 // / 26.8, FP32 10.0 / 14.1, FP16 10.4 / 15.4; 5 columns, 58000 rows FP64 14.4 /
 // 17.7; but 5 columns, 24000 rows FP32 8.4 / 4.9.
-bool tiles_pay(const LatticeShape &a)
+bool tiles_pay(const LatticeShape &a, TileShape t)
 {
-    return a.nc > 5 || tiles_of(a, tile_shape(a)) <= (a.storage == kF64 ? 6 : 10) * (int64_t)a.cus;
+    return a.nc > 5 || tiles_of(a, t) <= (a.storage == kF64 ? 6 : 10) * (int64_t)a.cus;
 }
 
 namespace {
@@ -314,10 +314,10 @@ double tile_us(const LatticeShape &a, int64_t tiles)
 // Where new values wait, a one-step launch takes their copy, of about 10 us, with
 // it: one step with new values FP16 500^2 32.7 / 14.5, 600^2 31.1 / 14.2 (they
 // wait up to nr + nc = 1365).
-int32_t tile_min_steps(const LatticeShape &a, bool waiting)
+int32_t tile_min_steps(const LatticeShape &a, TileShape t, bool waiting)
 {
-    const int64_t nodes = a.nr * a.nc, tiles = tiles_of(a, tile_shape(a)), cus = a.cus;
     if (waiting) return 1;
+    const int64_t nodes = a.nr * a.nc, tiles = tiles_of(a, t), cus = a.cus;
     if (a.psbb) return tiles <= cus ? 2 : 3;
     const int64_t small = a.storage == kF64 ? 32768 : a.storage == kF32 ? 65000 : 110000;
     const double margin = a.storage == kF64 ? 0.78 : 0.9, single = one_step_us(a), tile = tile_us(a, tiles);

@@ -73,7 +73,7 @@ int64_t tiles_of(const LatticeShape &a, TileShape t);
 // Whether launches of many steps in tiles are faster than the one-step
 // kernels, and the fewest steps for which one launch is; waiting: with new
 // prescribed values that the one-step kernels would wait for a copy of.
-bool tiles_pay(const LatticeShape &a);
-int32_t tile_min_steps(const LatticeShape &a, bool waiting);
+bool tiles_pay(const LatticeShape &a, TileShape t);
+int32_t tile_min_steps(const LatticeShape &a, TileShape t, bool waiting);
 
 }  // namespace lbm

@@ -101,7 +101,8 @@ int main()
         } else if (what == "pays") {
             std::cout << march_pays(a);
         } else if (what == "tiles") {
-            std::cout << tiles_pay(a) << " " << tile_min_steps(a, false) << " " << tile_min_steps(a, true);
+            const TileShape t = tile_shape(a);
+            std::cout << tiles_pay(a, t) << " " << tile_min_steps(a, t, false) << " " << tile_min_steps(a, t, true);
         } else if (what == "plan") {
             in >> K;
             const MarchPlan m = march_plan(a, K);
