@@ -255,6 +255,14 @@ int ensure_partials(lbm_ctx *c, int64_t n)
     return LBM_OK;
 }
 
+// Whether nothing is queued on a stream.
+bool stream_idle(hipStream_t s)
+{
+    if (hipStreamQuery(s) == hipSuccess) return true;
+    (void)hipGetLastError();  // "not ready" is no error of the caller's
+    return false;
+}
+
 int ensure_staging(lbm_ctx *c)
 {
     if (c->d_staging) return LBM_OK;
@@ -1064,8 +1072,10 @@ int lbm_download_populations(lbm_ctx *c, double *P)
     if (r) return r;
     StepArgs a = make_args(c);
     a.fin = c->d_F[c->cur];
+    const bool soon = stream_idle(c->stream);
     HIP_TRY(launch_readout(c->storage, c->state == kFstar, a, c->d_staging, nullptr, c->stream));
-    HIP_TRY(copy_to_host(c->desc.device, P, c->d_staging, (size_t)(9 * c->nr * c->nc) * sizeof(double), c->stream));
+    HIP_TRY(copy_to_host(c->desc.device, P, c->d_staging, (size_t)(9 * c->nr * c->nc) * sizeof(double), c->stream,
+                         soon));
     return LBM_OK;
 }
 
@@ -1078,8 +1088,10 @@ int lbm_download_after_collision(lbm_ctx *c, double *P)
     if (r) return r;
     StepArgs a = make_args(c);
     a.fin = c->d_F[c->cur];
+    const bool soon = stream_idle(c->stream);
     HIP_TRY(launch_readout(c->storage, false, a, c->d_staging, nullptr, c->stream));
-    HIP_TRY(copy_to_host(c->desc.device, P, c->d_staging, (size_t)(9 * c->nr * c->nc) * sizeof(double), c->stream));
+    HIP_TRY(copy_to_host(c->desc.device, P, c->d_staging, (size_t)(9 * c->nr * c->nc) * sizeof(double), c->stream,
+                         soon));
     return LBM_OK;
 }
 

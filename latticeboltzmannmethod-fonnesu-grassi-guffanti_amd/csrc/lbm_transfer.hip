@@ -75,7 +75,7 @@ hipError_t run_lane(int device, int lane, char *chunk, char *dst, const char *sr
     return e;
 }
 
-hipError_t copy(int device, void *dst, const void *src, size_t bytes, hipMemcpyKind kind, hipStream_t s)
+hipError_t copy(int device, void *dst, const void *src, size_t bytes, hipMemcpyKind kind, hipStream_t s, bool soon)
 {
     const void *host = kind == hipMemcpyDeviceToHost ? dst : src;
     if (bytes < (kind == hipMemcpyDeviceToHost ? kMinDown : kMinUp) || !pageable(host)) return plain(dst, src, bytes, kind, s);
@@ -91,7 +91,9 @@ hipError_t copy(int device, void *dst, const void *src, size_t bytes, hipMemcpyK
     }
     // The steps queued before the copy are waited for here, by this thread
     // alone: a run of many steps would otherwise hold every lane for its length.
-    if (const hipError_t e = hipStreamSynchronize(s); e != hipSuccess) return e;
+    // Short work is left to the lanes, whose start it hides (10 us).
+    if (!soon)
+        if (const hipError_t e = hipStreamSynchronize(s); e != hipSuccess) return e;
     hipError_t res[kLanes];
     std::thread threads[kLanes];
     auto lane = [&](int k) {
@@ -115,14 +117,14 @@ hipError_t copy(int device, void *dst, const void *src, size_t bytes, hipMemcpyK
 
 }  // namespace
 
-hipError_t copy_to_host(int device, void *dst, const void *src, size_t bytes, hipStream_t s)
+hipError_t copy_to_host(int device, void *dst, const void *src, size_t bytes, hipStream_t s, bool soon)
 {
-    return copy(device, dst, src, bytes, hipMemcpyDeviceToHost, s);
+    return copy(device, dst, src, bytes, hipMemcpyDeviceToHost, s, soon);
 }
 
 hipError_t copy_to_device(int device, void *dst, const void *src, size_t bytes, hipStream_t s)
 {
-    return copy(device, dst, src, bytes, hipMemcpyHostToDevice, s);
+    return copy(device, dst, src, bytes, hipMemcpyHostToDevice, s, false);
 }
 
 namespace {

@@ -136,6 +136,9 @@ int main(int argc, char **argv)
         earlier = true;
         require(lbm::copy_to_host(0, b.data(), a.data(), a.size(), nullptr) == hipSuccess, "down failed");
         require(!lane_waited, "the lanes waited for the stream's earlier work");
+        waits = 0;
+        require(lbm::copy_to_host(0, b.data(), a.data(), a.size(), nullptr, true) == hipSuccess, "down failed");
+        require(waits == 1 && a == b, "short work was waited for before the lanes started");
     } else if (what == "failure") {
         for (const bool up : {false, true}) {
             fail_records = true;
